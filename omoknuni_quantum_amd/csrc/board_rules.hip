@@ -216,93 +216,167 @@ hipError_t launch_gomoku_terminal(const omq_forest& f, const omq_wave& w, const 
 //   0 stones of the player to move, 1 stones of the opponent, 2-15 zero (history, unused by
 //   the reference), 16 ones when player 1 is to move, 17 move count / 100 (the reference's
 //   int16 count divided in double, stored as float), 18 ones (only with 19 planes).
-// Wave 0 rebuilds the leaf's board in LDS; then the whole workgroup writes the slot's planes,
-// one contiguous block of PLANES*cells values, element i by thread i mod 256, two values per
-// store where the block has an even length.
-constexpr int kFeatThreads = 256;
+// NW wavefronts per slot: the first rebuilds the leaf's board in LDS, all write the slot's block
+// of PLANES*cells values, 16 bytes per lane and store where the address allows (an unaligned
+// head and tail of single values; the caller's buffer need not be aligned to more than two values,
+// and a slot of odd length starts anywhere).  The stores are bound by HBM, but a slot's chain of
+// dependent loads (leaf count and first simulation, length, path, actions) takes longer than its
+// share of the stores, so with many slots what counts is how many chains are in flight: one wave
+// per slot keeps 32 of them on a CU, a workgroup of four 8.  With few slots, which one wave each
+// would leave most of the chip idle, four waves share a slot's stores.
+// Measured, 15x15, a call among others, against one 256-thread workgroup per slot with 8-byte
+// stores and the planes found per value: 16384 slots float32 NCHW 99.7 -> 65.5 us (4.3 TB/s; a
+// fill of the same buffers takes 42 us), bfloat16 NHWC 71.0 -> 36.2 us; 8192 slots 53.5 -> 35.2 and
+// 34.6 -> 16.6 us; 2048 slots (four waves) 16.0 -> 10.6 and 12.7 -> 10.4 us, where the launch bounds
+// both.  One wave per slot from 4096 slots (16 per CU): 512 slots took 18 us with it, 11 with four.
+constexpr int kFeatOneWaveSlots = 4096;
 
 template <typename OutT>
 struct PlaneStore;
 template <>
 struct PlaneStore<float> {
-  using Pair = float2;
+  static constexpr int kVec = 4;
   __device__ static float one(float v) { return v; }
-  __device__ static float2 two(float a, float b) { return make_float2(a, b); }
+  __device__ static uint32_t word(const float* v) { return __float_as_uint(v[0]); }
 };
 template <>
 struct PlaneStore<uint16_t> {  // bfloat16, rounded to nearest even
-  using Pair = uint32_t;
+  static constexpr int kVec = 8;
   __device__ static uint16_t one(float v) {
     const uint32_t x = __float_as_uint(v);
     return (uint16_t)((x + 0x7FFFu + ((x >> 16) & 1u)) >> 16);
   }
-  __device__ static uint32_t two(float a, float b) {
-    return (uint32_t)one(a) | ((uint32_t)one(b) << 16);
+  __device__ static uint32_t word(const float* v) {
+    return (uint32_t)one(v[0]) | ((uint32_t)one(v[1]) << 16);
   }
 };
 
-template <typename OutT, int PLANES, bool NHWC>
-__global__ __launch_bounds__(kFeatThreads) void leaf_features_kernel(
+template <typename OutT, int PLANES, bool NHWC, int NW>
+__global__ __launch_bounds__(NW * kWave) void leaf_features_kernel(
     omq_forest f, omq_wave w, const int8_t* root_boards, const int32_t* root_player,
     const int32_t* root_moves, int bs, OutT* out) {
   using S = PlaneStore<OutT>;
-  using Pair = typename S::Pair;
+  constexpr int NT = NW * kWave;
+  constexpr int V = S::kVec;       // values per 16-byte store
+  constexpr int VW = V / 4;        // values per 32-bit word
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ float s_val[4];  // player to move is 1, move count / 100, player to move
+  __shared__ int s_pos[2];  // player to move at the leaf, move count
   const int cells = bs * bs;
   const int t = blockIdx.y;
   const int u = blockIdx.x;
   const int tid = threadIdx.x;
   const int per = PLANES * cells;
   OutT* o = out + ((int64_t)t * w.max_wave + u) * per;
-  const bool pairs = (per & 1) == 0;  // then every slot starts on a pair boundary
+  // the slot's whole 16-byte stores: values [hd, hd + V * nv)
+  const int hd = min(per, (int)((16 - (reinterpret_cast<uintptr_t>(o) & 15)) & 15) /
+                              (int)sizeof(OutT));
+  const int nv = (per - hd) / V;
+  const int ends = per - V * nv;   // single values: the head and the tail
+  uint4* ov = reinterpret_cast<uint4*>(o + hd);
+  const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
   if (u >= w.ucount[t]) {
-    if (pairs) {
-      Pair* o2 = reinterpret_cast<Pair*>(o);
-      for (int i = tid; i < per / 2; i += kFeatThreads) o2[i] = S::two(0.0f, 0.0f);
-    } else {
-      for (int i = tid; i < per; i += kFeatThreads) o[i] = S::one(0.0f);
-    }
+    for (int i = tid; i < nv; i += NT) ov[i] = zero;
+    for (int i = tid; i < ends; i += NT) o[i < hd ? i : V * nv + i] = (OutT)0;
     return;
   }
   int8_t* b = reinterpret_cast<int8_t*>(smem);
-  if (tid < kWave) {
+  int tm, mc;
+  if (NW == 1 || tid < kWave) {
     int rp, stones;
-    const int L = rebuild_leaf_board(f, w, root_boards, root_player, t, u, cells, b, &rp,
-                                     &stones);
-    if (tid == 0) {
-      const int moves = L - 1;
-      const int tm = (moves & 1) == 0 ? rp : 3 - rp;  // player to move at the leaf
-      const int mc = (root_moves != nullptr ? root_moves[t] : stones) + moves;
-      s_val[0] = tm == 1 ? 1.0f : 0.0f;
-      s_val[1] = (float)((double)mc / 100.0);
-      s_val[2] = (float)tm;
+    const int moves =
+        rebuild_leaf_board(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones) - 1;
+    tm = (moves & 1) == 0 ? rp : 3 - rp;
+    mc = (root_moves != nullptr ? root_moves[t] : stones) + moves;
+    if (NW > 1 && tid == 0) {
+      s_pos[0] = tm;
+      s_pos[1] = mc;
     }
   }
-  __syncthreads();
-  const float colour = s_val[0], mcv = s_val[1];
-  const int tm = (int)s_val[2];
-  auto value = [&](int i) -> float {
-    int c, cell;
-    if (NHWC) {
-      cell = i / PLANES;
-      c = i - cell * PLANES;
-    } else {
-      c = i / cells;
-      cell = i - c * cells;
-    }
-    if (c == 0) return b[cell] == tm ? 1.0f : 0.0f;
-    if (c == 1) return b[cell] == 3 - tm ? 1.0f : 0.0f;
-    if (c == 16) return colour;
-    if (c == 17) return mcv;
-    if (c == 18) return 1.0f;
-    return 0.0f;
+  if (NW > 1) {
+    __syncthreads();
+    tm = s_pos[0];
+    mc = s_pos[1];
+  }
+  const float colour = tm == 1 ? 1.0f : 0.0f;
+  const float mcv = (float)((double)mc / 100.0);
+  // the value of plane c at a cell
+  auto value = [&](int c, int cell) -> float {
+    const bool stone = c < 2;
+    const int v = b[stone ? cell : 0];
+    const float rest = c == 16 ? colour : c == 17 ? mcv : c == 18 ? 1.0f : 0.0f;
+    return stone ? (v == (c == 0 ? tm : 3 - tm) ? 1.0f : 0.0f) : rest;
   };
-  if (pairs) {
-    Pair* o2 = reinterpret_cast<Pair*>(o);
-    for (int i = tid; i < per / 2; i += kFeatThreads) o2[i] = S::two(value(2 * i), value(2 * i + 1));
+  auto value_at = [&](int i) -> float {  // the slot's value i
+    const int outer = i / (NHWC ? PLANES : cells);
+    const int inner = i - outer * (NHWC ? PLANES : cells);
+    return NHWC ? value(inner, outer) : value(outer, inner);
+  };
+  if constexpr (NHWC) {
+    // The planes that a store's values fall on repeat every PLANES / gcd(PLANES, V) stores, so
+    // with a stride of a multiple of that a thread's stores all start on the same plane c0: its
+    // words are set up once (base: the planes that no stone decides; mo and mp: where the two
+    // stone planes of its one cell go), and a store is one board read and a few selects (the
+    // planes found anew for each value: 55 us against 36 us for 16384 slots of 15x15 in bfloat16).
+    constexpr int kPeriod = PLANES % 2 != 0 ? PLANES : PLANES / 2;  // (18: gcd 2 with 4 and 8)
+    static_assert(PLANES == 18 || PLANES == 19, "gcd of the planes and 4 or 8");
+    constexpr int kUse = NT / kPeriod * kPeriod;  // threads that store
+    if (tid < kUse) {
+      int cell = (hd + V * tid) / PLANES;
+      const int c0 = hd + V * tid - cell * PLANES;
+      uint32_t base[4], mo[4], mp[4];
+      const int next = c0 >= 2 ? 1 : 0;  // the stones of the next cell, or of this one
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float x[VW];
+        mo[k] = mp[k] = 0u;
+#pragma unroll
+        for (int e = 0; e < VW; ++e) {
+          const int ce = c0 + k * VW + e;
+          const int c = ce >= PLANES ? ce - PLANES : ce;
+          x[e] = c == 16 ? colour : c == 17 ? mcv : c == 18 ? 1.0f : 0.0f;
+          const uint32_t m = VW == 1 ? 0xFFFFFFFFu : 0xFFFFu << (16 * e);
+          mo[k] |= c == 0 ? m : 0u;
+          mp[k] |= c == 1 ? m : 0u;
+        }
+        base[k] = S::word(x);
+      }
+      constexpr uint32_t kOne = VW == 1 ? 0x3F800000u : 0x3F803F80u;  // 1.0 in each value
+      constexpr int kCells = kUse * V / PLANES;  // cells per round
+      static_assert(kUse * V % PLANES == 0, "a round is a whole number of cells");
+      cell += next;
+      for (int i = tid; i < nv; i += kUse, cell += kCells) {
+        const int v = b[min(cell, cells - 1)];  // (past the board where no mask takes it)
+        const uint32_t own = v == tm ? kOne : 0u, opp = v == 3 - tm ? kOne : 0u;
+        ov[i] = make_uint4(base[0] | (own & mo[0]) | (opp & mp[0]),
+                           base[1] | (own & mo[1]) | (opp & mp[1]),
+                           base[2] | (own & mo[2]) | (opp & mp[2]),
+                           base[3] | (own & mo[3]) | (opp & mp[3]));
+      }
+    }
   } else {
-    for (int i = tid; i < per; i += kFeatThreads) o[i] = S::one(value(i));
+    // the stores [z0, z1) lie in planes 2..15 (zeros)
+    const int z0 = min(nv, max(0, 2 * cells - hd + V - 1) / V);
+    const int z1 = max(z0, min(nv, (16 * cells - hd) / V));
+    for (int i = z0 + tid; i < z1; i += NT) ov[i] = zero;
+    const int rest = nv - (z1 - z0);
+    for (int q = tid; q < rest; q += NT) {
+      const int i = q < z0 ? q : q + (z1 - z0);
+      int c = (hd + V * i) / cells;
+      int cell = hd + V * i - c * cells;
+      float x[V];
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        x[e] = value(c, cell);
+        const bool wrap = cell + 1 == cells;
+        cell = wrap ? 0 : cell + 1;
+        c += wrap ? 1 : 0;
+      }
+      ov[i] = make_uint4(S::word(x), S::word(x + VW), S::word(x + 2 * VW), S::word(x + 3 * VW));
+    }
+  }
+  for (int i = tid; i < ends; i += NT) {
+    const int e = i < hd ? i : V * nv + i;
+    o[e] = S::one(value_at(e));
   }
 }
 
@@ -312,15 +386,20 @@ hipError_t launch_leaf_features_t(const omq_forest& f, const omq_wave& w, const 
                                   int planes, bool nhwc, OutT* out, hipStream_t st) {
   const size_t lds = (size_t)(((bs * bs) + 15) & ~15);
   dim3 grid(w.max_wave, f.num_trees);
-#define OMQ_FEAT_LAUNCH(P, NH)                                                                  \
-  hipLaunchKernelGGL((leaf_features_kernel<OutT, P, NH>), grid, dim3(kFeatThreads), lds, st, f, \
-                     w, boards, root_player, root_moves, bs, out)
+  const bool one_wave = (int64_t)w.max_wave * f.num_trees >= kFeatOneWaveSlots;
+#define OMQ_FEAT_LAUNCH(P, NH)                                                               \
+  if (one_wave)                                                                              \
+    hipLaunchKernelGGL((leaf_features_kernel<OutT, P, NH, 1>), grid, dim3(kWave), lds, st, f, \
+                       w, boards, root_player, root_moves, bs, out);                         \
+  else                                                                                       \
+    hipLaunchKernelGGL((leaf_features_kernel<OutT, P, NH, 4>), grid, dim3(4 * kWave), lds,    \
+                       st, f, w, boards, root_player, root_moves, bs, out)
   if (planes == 18) {
-    if (nhwc) OMQ_FEAT_LAUNCH(18, true);
-    else OMQ_FEAT_LAUNCH(18, false);
+    if (nhwc) { OMQ_FEAT_LAUNCH(18, true); }
+    else { OMQ_FEAT_LAUNCH(18, false); }
   } else {
-    if (nhwc) OMQ_FEAT_LAUNCH(19, true);
-    else OMQ_FEAT_LAUNCH(19, false);
+    if (nhwc) { OMQ_FEAT_LAUNCH(19, true); }
+    else { OMQ_FEAT_LAUNCH(19, false); }
   }
 #undef OMQ_FEAT_LAUNCH
   return hipGetLastError();

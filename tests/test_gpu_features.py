@@ -124,3 +124,27 @@ def test_features_board_sizes(device, bs):
     eng.search(3 * W, W, ev)
     torch.cuda.synchronize()
     assert ev.waves == 4
+
+
+@pytest.mark.parametrize("bs,trees,wave", [(5, 9, 480), (15, 9, 480), (15, 3, 40)])
+def test_features_unaligned_buffers(device, bs, trees, wave):
+    # a wave per slot (4320 slots) and four waves per slot (120), into buffers that start 0, 2
+    # and 6 values past a 16-byte boundary: heads and tails of single values around the stores
+    model = games.gomoku(bs)
+    boards = games.random_boards(trees, bs, bs, 3)
+    eng = WaveEngine(model, trees, 1 + 40 * bs * bs, wave, 100, device, SearchParams(c_puct=1.4))
+    eng.set_roots(games.root_keys(3, trees), games.legal_masks(model, boards, trees))
+    eng.search(16, 8, SyntheticEvaluator())
+    eng.select(16)
+    dev_boards = torch.from_numpy(boards.reshape(-1).copy()).to(device)
+    for planes in (18, 19):
+        exp = torch.from_numpy(_expected(eng, boards, planes)[0])
+        for dtype in (torch.float32, torch.bfloat16):
+            for nhwc in (False, True):
+                want = (exp.permute(0, 2, 3, 1) if nhwc else exp).to(dtype).reshape(-1)
+                for off in (0, 2, 6):
+                    buf = torch.full((want.numel() + 6,), 7.0, dtype=dtype, device=device)
+                    out = buf[off:off + want.numel()]
+                    eng.leaf_features(out, dev_boards, planes, nhwc=nhwc)
+                    assert torch.equal(out.cpu(), want), (planes, dtype, nhwc, off)
+                    assert (buf[:off] == 7).all() and (buf[off + want.numel():] == 7).all()
