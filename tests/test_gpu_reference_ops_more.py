@@ -173,6 +173,31 @@ def test_optimized_backup_scatter_equals_vectorized_backup(device):
     assert torch.equal(n1, n3) and torch.equal(w1, w3)
 
 
+@pytest.mark.parametrize("B,D,nn", [(1, 1, 1), (256, 9, 4000), (257, 8, 40), (700, 20, 5000)])
+def test_backup_and_virtual_loss_node_tables(device, B, D, nn):
+    """Paths whose workgroup meets more distinct nodes than its table holds, fewer, and entries
+    past the levels that go through it; the same nodes as a virtual-loss list of several
+    workgroups."""
+    rng = np.random.default_rng(B)
+    paths = rng.integers(-1, nn + 1, (B, D)).astype(np.int32)
+    paths[:, 0] = 0
+    plen = np.full(B, D, np.int32)
+    vals = (rng.integers(-4, 5, B) / 4).astype(F)  # exact sums in any order
+    n_exp, w_exp = np.zeros(nn, np.int64), np.zeros(nn, np.float64)
+    on = (paths >= 0) & (paths < nn)
+    sign = np.where((D - 1 - np.arange(D)) % 2 == 0, 1.0, -1.0)
+    np.add.at(n_exp, paths[on], 1)
+    np.add.at(w_exp, paths[on], (vals[:, None] * sign)[on])
+    n, w = torch.zeros(nn, dtype=torch.int32, device=device), torch.zeros(nn, device=device)
+    torch_ops.vectorized_backup(_t(paths, device), _t(plen, device), _t(vals, device), n, w)
+    assert np.array_equal(_np(n), n_exp) and np.array_equal(_np(w), w_exp.astype(F))
+    vl = torch.zeros(nn, dtype=torch.int32, device=device)
+    torch_ops.batch_apply_virtual_loss(_t(paths.reshape(-1), device), vl)
+    assert np.array_equal(_np(vl), n_exp)
+    torch_ops.batch_remove_virtual_loss(_t(paths.reshape(-1), device), vl)
+    assert not _np(vl).any()
+
+
 # ---- parallel_bfs_subtree / extract_subtree_edges --------------------------------------------
 def _check_subtree(device, rows, root, n, actions=True):
     ptr, col = _csr(rows)
