@@ -400,6 +400,13 @@ int omq_shift_root_noalloc(const omq_forest* f, const int32_t* new_roots, void* 
  * Replaces MCTS._extract_policy (python/mcts/core/mcts.py:1069-1137). */
 int omq_root_policy(const omq_forest* f, double* policy, void* stream);
 
+/* The root's child for one action per tree: out[2t] = the first child (node of tree t) whose
+ * action is actions[t], or -1 without one; out[2t+1] = its visit count (0 without one).  actions
+ * and out are device arrays of num_trees and 2*num_trees int32.  What a caller needs to know of
+ * every tree before omq_shift_root, in one launch and one copy to the host (the reference looks
+ * the child up on the host, python/mcts/core/tree_operations.py:53-133). */
+int omq_root_children(const omq_forest* f, const int32_t* actions, int32_t* out, void* stream);
+
 /* Move selection per tree from policy rows (as omq_root_policy writes them) into actions[t].
  * - temperature 0 takes the first maximum.
  * - Otherwise w_a = p_a^(1/temperature), with w = p at temperature 1 and 0 where p = 0. The

@@ -106,6 +106,7 @@ SIGNATURES = {
     "omq_batched_add_children": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p,
                                                 _p, _p, _p, _p, _p, _i32, _i32, _i32, _p, _p]),
     "omq_root_policy": (ctypes.c_int, [_FP, _p, _p]),
+    "omq_root_children": (ctypes.c_int, [_FP, _p, _p, _p]),
     "omq_sample_actions": (ctypes.c_int, [_FP, _p, ctypes.c_double, ctypes.c_uint64,
                                           ctypes.c_uint64, _p, _p]),
     "omq_root_dirichlet": (ctypes.c_int, [_FP, ctypes.c_double, ctypes.c_uint64,
@@ -150,12 +151,26 @@ _lib = None
 _lock = threading.Lock()
 
 
+def raw_stream(device) -> int:
+    """Handle of torch's current stream on a device (torch.device, or its index), without the
+    Stream object that torch.cuda.current_stream builds: 0.3 us against 2.5 us of every launch
+    from Python."""
+    import torch
+
+    index = device if isinstance(device, int) else device.index
+    if index is None:
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
 def load(path: str | None = None) -> ctypes.CDLL:
     """Load the HIP library once; raise LibraryNotBuilt when it is absent.  torch is imported
     first: the library then binds the HIP runtime torch has loaded, so that both share one
     runtime (loaded first, the library would bring the system's and torch its own, and the
     second runtime finds no device)."""
     global _lib
+    if path is None and _lib is not None:
+        return _lib
     import torch  # noqa: F401  (the HIP runtime the library shares)
 
     with _lock:

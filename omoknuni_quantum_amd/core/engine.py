@@ -108,6 +108,10 @@ class WaveEngine:
         self.root_ko: torch.Tensor | None = None
         self._shift_ws: torch.Tensor | None = None  # subtree-reuse workspace, made on first use
         self._policy: torch.Tensor | None = None    # root policies [T, A] float64
+        self._new_roots: torch.Tensor | None = None  # subtree reuse: the new roots [T]
+        self._child: torch.Tensor | None = None     # root_children: actions [T], results [T, 2]
+        self._pending: dict = {}                    # rule inputs to copy (_copy_pending)
+        self._stage: dict = {}                      # pinned host buffers by name (_host)
 
         f = _lib.OmqForest()
         f.num_trees, f.capacity, f.num_actions, f.game = T, cap, A, model.code
@@ -132,18 +136,48 @@ class WaveEngine:
 
     # ---- plumbing ---------------------------------------------------------------------
     def stream_handle(self) -> int:
-        return torch.cuda.current_stream(self.device).cuda_stream
+        return _lib.raw_stream(self.device)
+
+    def _host(self, name: str, like: torch.Tensor) -> torch.Tensor:
+        """The pinned host buffer for copies to or from tensors of like's size and type (one
+        per name, held by the engine)."""
+        h = self._stage.get(name)
+        if h is None or h.numel() != like.numel() or h.dtype != like.dtype:
+            h = torch.empty(like.numel(), dtype=like.dtype, pin_memory=True)
+            self._stage[name] = h
+        return h
+
+    def _upload(self, **arrays) -> None:
+        """name=(device tensor, host array): the arrays through pinned buffers, their copies in
+        flight together and one wait for all, so that the inputs are on the device for any
+        stream when this returns (a pageable copy waits for each: 20-35 us an array)."""
+        for name, (dst, src) in arrays.items():
+            h = self._host(name, dst)
+            np.copyto(h.numpy(), np.asarray(src).reshape(-1))
+            dst.view(-1).copy_(h, non_blocking=True)
+        torch.cuda.current_stream(self.device).synchronize()
+
+    def _download(self, **tensors) -> list:
+        """name=device tensor: host copies (numpy, the caller's own) after one wait for all."""
+        out = []
+        for name, x in tensors.items():
+            h = self._host(name, x)
+            h.copy_(x.view(-1), non_blocking=True)
+            out.append(h)
+        torch.cuda.current_stream(self.device).synchronize()
+        return [h.numpy().copy() for h in out]
 
     def set_roots(self, keys: np.ndarray, legal: np.ndarray | None = None,
                   noise: np.ndarray | None = None) -> None:
         """Root keys uint64[T], root legal masks uint32[T, legal_words], noise float64[T, A]."""
-        self.root_keys.copy_(torch.from_numpy(_u64_to_i64(keys)))
+        arrays = {"root_keys": (self.root_keys, _u64_to_i64(keys))}
         if legal is not None:
-            lw = np.ascontiguousarray(legal, dtype=np.uint32).reshape(-1).view(np.int32)
-            self.root_legal.copy_(torch.from_numpy(lw.copy()))
+            arrays["root_legal"] = (self.root_legal, np.ascontiguousarray(
+                legal, dtype=np.uint32).reshape(-1).view(np.int32))
         self.has_noise = noise is not None
         if noise is not None:
-            self.noise.copy_(torch.from_numpy(np.ascontiguousarray(noise, dtype=np.float64).reshape(-1)))
+            arrays["noise"] = (self.noise, np.ascontiguousarray(noise, dtype=np.float64))
+        self._upload(**arrays)
 
     def set_gomoku_rules(self, boards, rule: int = _lib.OMQ_RULE_FREESTYLE,
                          root_player=None) -> None:
@@ -155,26 +189,34 @@ class WaveEngine:
             return
         if self.model.kind != "gomoku":
             raise ValueError("the Gomoku terminal rule needs a gomoku game model")
+        self._pending = {}
         b = torch.as_tensor(np.ascontiguousarray(boards, dtype=np.int8)).reshape(-1)
         if b.numel() != self.T * self.A:
             raise ValueError(f"boards hold {b.numel()} cells, expected {self.T} x {self.A}")
-        self.root_boards = self._reuse(self.root_boards, b)
+        self.root_boards = self._reuse("root_boards", b)
         rp = None
         if root_player is not None:
             rp = torch.as_tensor(np.ascontiguousarray(root_player, dtype=np.int32)).reshape(-1)
             if rp.numel() != self.T:
                 raise ValueError("one root player per tree")
-        self.root_player = None if rp is None else self._reuse(self.root_player, rp)
+        self.root_player = None if rp is None else self._reuse("root_player", rp)
+        self._copy_pending()
         self.rule = int(rule)
 
-    def _reuse(self, cur: torch.Tensor | None, x: torch.Tensor) -> torch.Tensor:
-        """x on the device, in cur's storage when cur has its size and type: root inputs keep
-        their addresses from one position to the next, so that a recorded search (whose
+    def _reuse(self, name: str, x: torch.Tensor) -> torch.Tensor:
+        """x as the rule input `name`: on the device, in the present one's storage (copied by _copy_pending)
+        when that has its size and type: root inputs keep their addresses from one position to the next, so that a recorded search (whose
         kernels hold those addresses) stays valid."""
+        cur = getattr(self, name)
         if cur is not None and cur.numel() == x.numel() and cur.dtype == x.dtype:
-            cur.copy_(x)
+            self._pending[name] = (cur, x.numpy())
             return cur
         return x.to(self.device)
+
+    def _copy_pending(self) -> None:
+        """The copies that _reuse left, together."""
+        pending, self._pending = self._pending, {}
+        self._upload(**pending)
 
     def set_go_rules(self, boards, flags: int = _lib.OMQ_GO_KO, root_player=None,
                      root_passes=None, root_ko=None) -> None:
@@ -194,22 +236,24 @@ class WaveEngine:
         if self.model.kind != "go":
             raise ValueError("the Go rules need a go game model")
         cells = self.A - 1
+        self._pending = {}
         b = torch.as_tensor(np.ascontiguousarray(boards, dtype=np.int8)).reshape(-1)
         if b.numel() != self.T * cells:
             raise ValueError(f"boards hold {b.numel()} points, expected {self.T} x {cells}")
 
-        def per_tree(cur, x, name):
+        def per_tree(attr, x, name):
             if x is None:
                 return None
             v = torch.as_tensor(np.ascontiguousarray(x, dtype=np.int32)).reshape(-1)
             if v.numel() != self.T:
                 raise ValueError(f"one {name} per tree")
-            return self._reuse(cur, v)
+            return self._reuse(attr, v)
 
-        self.root_boards = self._reuse(self.root_boards, b)
-        self.root_player = per_tree(self.root_player, root_player, "root player")
-        self.root_passes = per_tree(self.root_passes, root_passes, "root pass count")
-        self.root_ko = per_tree(self.root_ko, root_ko, "ko point")
+        self.root_boards = self._reuse("root_boards", b)
+        self.root_player = per_tree("root_player", root_player, "root player")
+        self.root_passes = per_tree("root_passes", root_passes, "root pass count")
+        self.root_ko = per_tree("root_ko", root_ko, "ko point")
+        self._copy_pending()
         if self.umask is None:
             self.umask = torch.zeros(self.T * self.MW * self.model.legal_words,
                                      dtype=torch.int32, device=self.device)
@@ -267,6 +311,12 @@ class WaveEngine:
                 None if self.root_player is None else self.root_player.data_ptr(), self.rule,
                 self.uterm.data_ptr(), self.stream_handle()), "omq_gomoku_terminal")
 
+    @staticmethod
+    def _feature_input(name, x, n, dty, out) -> None:
+        if x is not None and (x.dtype != dty or x.numel() != n or not x.is_contiguous()
+                              or x.device != out.device):
+            raise ValueError(f"{name} must be contiguous {dty} [{n}] on {out.device}")
+
     def leaf_features(self, out: torch.Tensor, boards: torch.Tensor, planes: int = 18,
                       root_player: torch.Tensor | None = None,
                       root_moves: torch.Tensor | None = None, nhwc: bool = False) -> None:
@@ -281,12 +331,11 @@ class WaveEngine:
             raise ValueError(f"feature planes are float32 or bfloat16, not {out.dtype}")
         if out.numel() != self.T * self.MW * planes * self.A or not out.is_contiguous():
             raise ValueError("out must be a contiguous buffer of T*max_wave*planes*A values")
-        for name, x, n, dty in (("boards", boards, self.T * self.A, torch.int8),
-                                ("root_player", root_player, self.T, torch.int32),
-                                ("root_moves", root_moves, self.T, torch.int32)):
-            if x is not None and (x.dtype != dty or x.numel() != n or not x.is_contiguous()
-                                  or x.device != out.device):
-                raise ValueError(f"{name} must be contiguous {dty} [{n}] on {out.device}")
+        self._feature_input("boards", boards, self.T * self.A, torch.int8, out)
+        if root_player is not None:
+            self._feature_input("root_player", root_player, self.T, torch.int32, out)
+        if root_moves is not None:
+            self._feature_input("root_moves", root_moves, self.T, torch.int32, out)
         self._check(self.lib.omq_leaf_features(
             self.forest_ref, self.wave_ref, boards.data_ptr(),
             None if root_player is None else root_player.data_ptr(),
@@ -327,10 +376,24 @@ class WaveEngine:
         need = _lib.OMQ_SHIFT_WORKSPACE_PER_NODE * self.T * self.cap
         if self._shift_ws is None or self._shift_ws.numel() < need:
             self._shift_ws = torch.empty(need, dtype=torch.int32, device=self.device)
-        d = torch.from_numpy(nr).to(self.device)
+        if self._new_roots is None:
+            self._new_roots = torch.empty(self.T, dtype=torch.int32, device=self.device)
+        d = self._new_roots
+        self._upload(new_roots=(d, nr))
         self._check(self.lib.omq_shift_root(self.forest_ref, d.data_ptr(),
                                             self._shift_ws.data_ptr(), self._shift_ws.numel(),
                                             self.stream_handle()), "omq_shift_root")
+
+    def root_children(self, actions) -> np.ndarray:
+        """[T, 2]: for every tree the root's child for its action (a node of the tree, -1
+        without one) and that child's visit count."""
+        if self._child is None:
+            self._child = torch.empty(3 * self.T, dtype=torch.int32, device=self.device)
+        acts, out = self._child[:self.T], self._child[self.T:]
+        self._upload(child_actions=(acts, np.asarray(actions, np.int32)))
+        self._check(self.lib.omq_root_children(self.forest_ref, acts.data_ptr(), out.data_ptr(),
+                                               self.stream_handle()), "omq_root_children")
+        return self._download(children=out)[0].reshape(self.T, 2)
 
     def _tree_of(self, tree_of, n: int):
         if tree_of is None:
@@ -441,7 +504,10 @@ class WaveEngine:
 
     # ---- results ----------------------------------------------------------------------
     def check_status(self) -> None:
-        st = int(self.status[0].item())
+        self._raise_status(int(self.status[0].item()))
+
+    @staticmethod
+    def _raise_status(st: int) -> None:
         if st & _lib.OMQ_STATUS_STALL:
             raise _lib.OmqError("omq_select: a bounded wait ran out; the selection is incomplete")
         if st & _lib.OMQ_STATUS_ROWLIMIT:
@@ -459,7 +525,16 @@ class WaveEngine:
             self._policy = torch.empty((self.T, self.A), dtype=torch.float64, device=self.device)
         self._check(self.lib.omq_root_policy(self.forest_ref, self._policy.data_ptr(),
                                              self.stream_handle()), "omq_root_policy")
-        return self._policy if device else self._policy.cpu().numpy()
+        if device:
+            return self._policy
+        return self._download(policy=self._policy)[0].reshape(self.T, self.A)
+
+    def checked_root_policies(self) -> np.ndarray:
+        """check_status, then root_policies, with one wait for both."""
+        status, pol = self._download(status=self.status,
+                                     policy=self.root_policies(device=True))
+        self._raise_status(int(status[0]))
+        return pol.reshape(self.T, self.A)
 
     def sample_actions(self, temperature: float, seed: int, counter: int) -> np.ndarray:
         """One move per tree from the root policies (MCTS.select_action): the first maximum at
@@ -470,7 +545,7 @@ class WaveEngine:
                                                 int(seed) & (2**64 - 1), int(counter) & (2**64 - 1),
                                                 out.data_ptr(), self.stream_handle()),
                     "omq_sample_actions")
-        return out.cpu().numpy()
+        return self._download(sampled=out)[0]
 
     def device_root_noise(self, alpha: float, seed: int, counter: int) -> None:
         """Root Dirichlet noise drawn on the device into the noise rows that omq_expand mixes at

@@ -67,8 +67,8 @@ class _BatchEvaluatorAdapter:
             idx = None
             feats = feats[:int(counts[0])]
         else:
-            idx = torch.cat([torch.arange(int(c), dtype=torch.int64) + t * MW
-                             for t, c in enumerate(counts.tolist())]).to(engine.device)
+            used = np.arange(MW) < counts.numpy()[:, None]  # (slot t * MW + u: leaf u of tree t)
+            idx = torch.from_numpy(np.flatnonzero(used)).to(engine.device)
             feats = feats.index_select(0, idx)
         if feats.shape[0] == 0:
             return
@@ -127,7 +127,6 @@ class MCTS:
         self.engine = WaveEngine(self.model, config.num_trees, int(config.max_tree_nodes),
                                  self.wave, int(config.max_depth), self.device, self.params)
         self._roots_key: Optional[bytes] = None
-        self._boards: Optional[torch.Tensor] = None
         self._eval = None
         self._graphs: dict = {}  # recorded searches by launch signature (use_cuda_graphs)
         self._search_count = 0
@@ -266,17 +265,20 @@ class MCTS:
             return b""
         return b"|go" + info[0].tobytes() + info[1].tobytes()
 
-    def _set_roots(self, boards: Optional[np.ndarray], players=None, moves=None) -> None:
+    def _set_roots(self, boards: Optional[np.ndarray], players=None, moves=None) -> bool:
+        """Installs the roots and resets the trees; False when they are the present ones
+        already, whose trees stay."""
         T = self.engine.T
         if boards is not None and boards.shape[0] != T:
             raise ValueError(f"{boards.shape[0]} states given for {T} trees")
         key = self._roots_key_of(boards, players, moves) + self._go_key()
         if key == self._roots_key and self._eval is not None:
-            return
+            return False
         keys = games.root_keys(self.config.seed, T)
         legal = games.legal_masks(self.model, boards, T)
         self._install_roots(keys, legal, boards, players, moves)
         self.engine.reset()
+        return True
 
     def _root_noise(self, keys: np.ndarray, legal: np.ndarray) -> Optional[np.ndarray]:
         if self.config.dirichlet_epsilon <= 0 or self.config.root_noise_source == "device":
@@ -321,8 +323,6 @@ class MCTS:
             self.engine.set_go_rules(boards, go_flags, root_player=players, root_passes=passes,
                                      root_ko=ko)
         self._roots_key = self._roots_key_of(boards, players, moves) + self._go_key()
-        self._boards = None if boards is None else torch.from_numpy(
-            np.ascontiguousarray(boards, np.int8)).to(self.device)
         self._eval = self._make_evaluator()
 
     def _go_root_legal(self, boards: np.ndarray, flags: int) -> np.ndarray:
@@ -330,22 +330,19 @@ class MCTS:
         root's ko point (OMQ_GO_KO) and the points with no empty orthogonal neighbour
         (OMQ_GO_SUICIDE), so that the root's Dirichlet noise has one entry per legal move."""
         T = boards.shape[0]
-        legal = games.legal_masks(self.model, boards, T)
         ko = self._root_go_host[1]
         empty = boards == 0
-        closed = np.zeros_like(empty)
+        taken = ~empty
         if flags & _lib.OMQ_GO_SUICIDE:
             pad = np.zeros((T, boards.shape[1] + 2, boards.shape[2] + 2), bool)
             pad[:, 1:-1, 1:-1] = empty
             open_nb = pad[:, :-2, 1:-1] | pad[:, 2:, 1:-1] | pad[:, 1:-1, :-2] | pad[:, 1:-1, 2:]
-            closed = empty & ~open_nb
-        for t in range(T):
-            drop = np.flatnonzero(closed[t].reshape(-1)).tolist()
-            if flags & _lib.OMQ_GO_KO and 0 <= int(ko[t]) < empty[t].size:
-                drop.append(int(ko[t]))
-            for a in drop:
-                legal[t, a // 32] &= np.uint32(~(1 << (a % 32)) & 0xFFFFFFFF)
-        return legal
+            taken |= ~open_nb
+        if flags & _lib.OMQ_GO_KO:
+            flat = taken.reshape(T, -1)
+            on = np.flatnonzero((ko >= 0) & (ko < flat.shape[1]))
+            flat[on, ko[on]] = True
+        return games.legal_masks(self.model, taken, T)
 
     def _gomoku_rule(self) -> Optional[int]:
         """Terminal rule of Gomoku leaves: the config's, renju when the game interface says
@@ -365,8 +362,9 @@ class MCTS:
             raise NotImplementedError("feature-plane evaluators need a board game model")
         from .features import LeafFeatureBuilder
         planes = _input_planes(self.evaluator)
-        boards = self._boards
-        if boards is None:
+        if self._root_boards_host is not None:
+            boards = torch.from_numpy(self._root_boards_host).to(self.device)
+        else:
             boards = torch.zeros((self.engine.T, self.config.board_size, self.config.board_size),
                                  dtype=torch.int8, device=self.device)
         return _BatchEvaluatorAdapter(self.evaluator, LeafFeatureBuilder(
@@ -395,19 +393,21 @@ class MCTS:
         start = time.perf_counter()
         if not self.config.enable_subtree_reuse:
             self._roots_key = None
-        self._set_roots(boards, players, moves)
-        self.engine.clear_status()
+        fresh = self._set_roots(boards, players, moves)
+        if not fresh:
+            self.engine.clear_status()  # (a reset clears it)
         if num_sims == 0:  # mcts.py:1022-1030 (a configured count of 0)
             return np.full((self.engine.T, self.action_size), 1.0 / self.action_size)
         eng = self.engine
-        fresh = int(eng.nchild[0].item()) == 0 and int(eng.num_nodes[0].item()) == 1
+        if not fresh:  # the trees go on from an earlier search, unless they are lone roots
+            nchild, nodes = eng._download(root_nchild=eng.nchild[:1], root_nodes=eng.num_nodes[:1])
+            fresh = int(nchild[0]) == 0 and int(nodes[0]) == 1
         key = self._graph_key(num_sims, fresh)
         if key is not None:
             self._graph_waves(key, num_sims, fresh)
         else:
             self._waves(num_sims, fresh, check_first=True)
-        eng.check_status()
-        policy = eng.root_policies()
+        policy = eng.checked_root_policies()
         elapsed = time.perf_counter() - start
         self._search_count += 1
         self._update_statistics(num_sims * eng.T, elapsed)
@@ -536,24 +536,12 @@ class MCTS:
         device).  None, with nothing changed, when some tree lacks that child or the child has
         fewer than subtree_reuse_min_visits visits."""
         eng = self.engine
-        T, cap = eng.T, eng.cap
+        T = eng.T
         min_visits = int(self.config.extra.get("subtree_reuse_min_visits", 10))
-        roots = torch.arange(T, device=eng.device, dtype=torch.int64) * cap
-        first = eng.first[roots].cpu().numpy()
-        k = eng.nchild[roots].cpu().numpy()
-        new_roots = np.full(T, -1, np.int32)
-        for t, a in enumerate(actions):
-            if k[t] <= 0:
-                return None
-            lo = t * cap + int(first[t]) + 1
-            acts = eng.action[lo:lo + int(k[t])].cpu().numpy()
-            hit = np.flatnonzero(acts == a)
-            if hit.size == 0:
-                return None
-            node = int(first[t]) + 1 + int(hit[0])
-            if int(eng.N[t * cap + node].item()) < min_visits:
-                return None
-            new_roots[t] = node
+        found = eng.root_children(actions)
+        if (found[:, 0] < 0).any() or (found[:, 1] < min_visits).any():
+            return None
+        new_roots = found[:, 0]
         eng.shift_roots(new_roots)
         keys = np.array([games.child_key(int(key), a)
                          for key, a in zip(self._root_keys_host, actions)], np.uint64)
@@ -589,7 +577,7 @@ class MCTS:
                                   for t, a in enumerate(actions)], np.int32),
                         np.full(T, -1, np.int32))
         self._install_roots(keys, legal, boards, players, moves)
-        return int(eng.num_nodes.sum().item())
+        return int(eng._download(nodes=eng.num_nodes)[0].sum())
 
     def update_with_move(self, move: int) -> None:
         self.update_root(move, None)

@@ -34,6 +34,8 @@ hipError_t launch_shift_root(const omq_forest& f, const int32_t* new_roots, int3
                              hipStream_t st);
 hipError_t shift_scratch(int32_t** out);
 hipError_t launch_root_policy(const omq_forest& f, double* pol, hipStream_t st);
+hipError_t launch_root_children(const omq_forest& f, const int32_t* actions, int32_t* out,
+                                hipStream_t st);
 hipError_t launch_sample_actions(const omq_forest& f, const double* pol, double temperature,
                                  uint64_t seed, uint64_t counter, int32_t* actions,
                                  hipStream_t st);
@@ -362,6 +364,14 @@ int omq_root_policy(const omq_forest* f, double* policy, void* stream) {
   if (rc) return rc;
   if (!policy) return fail(OMQ_E_ARG, "policy is null");
   return hip_status(omq::launch_root_policy(*f, policy, (hipStream_t)stream), "omq_root_policy");
+}
+
+int omq_root_children(const omq_forest* f, const int32_t* actions, int32_t* out, void* stream) {
+  int rc = check_forest(f);
+  if (rc) return rc;
+  if (!actions || !out) return fail(OMQ_E_ARG, "actions and out are required");
+  return hip_status(omq::launch_root_children(*f, actions, out, (hipStream_t)stream),
+                    "omq_root_children");
 }
 
 int omq_sample_actions(const omq_forest* f, const double* policy, double temperature,

@@ -176,6 +176,29 @@ __global__ __launch_bounds__(kRootThreads) void root_policy_kernel(omq_forest f,
   }
 }
 
+// ---- the root's child for an action --------------------------------------------------------
+// One wavefront per tree over the root's row.
+__global__ __launch_bounds__(kWave) void root_children_kernel(omq_forest f,
+                                                              const int32_t* actions,
+                                                              int32_t* out) {
+  const int t = blockIdx.x;
+  const int lane = lane_id();
+  const int64_t tb = (int64_t)t * f.capacity;
+  const int k = f.num_children[tb];
+  const int first = f.first_child[tb];
+  const int want = actions[t];
+  int node = -1;
+  for (int j0 = 0; j0 < k && first >= 0 && node < 0; j0 += kWave) {
+    const int j = j0 + lane;
+    const uint64_t hit = __ballot(j < k && f.actions[tb + first + 1 + j] == want);
+    if (hit != 0) node = first + 1 + j0 + lowest_lane(hit);
+  }
+  if (lane == 0) {
+    out[2 * t] = node;
+    out[2 * t + 1] = node >= 0 ? f.visit_counts[tb + node] : 0;
+  }
+}
+
 // ---- move selection -------------------------------------------------------------------------
 // One wavefront per tree.  Temperature 0 takes the first maximum (a wave reduction on
 // (value, lowest index)).  Otherwise the lanes compute w = p^(1/T) (w = p for T = 1, 0 for
@@ -326,6 +349,12 @@ hipError_t launch_batched_dirichlet(int num_sims, int num_actions, double alpha,
 
 hipError_t launch_root_policy(const omq_forest& f, double* pol, hipStream_t st) {
   hipLaunchKernelGGL(root_policy_kernel, dim3(f.num_trees), dim3(kRootThreads), 0, st, f, pol);
+  return hipGetLastError();
+}
+
+hipError_t launch_root_children(const omq_forest& f, const int32_t* actions, int32_t* out,
+                                hipStream_t st) {
+  hipLaunchKernelGGL(root_children_kernel, dim3(f.num_trees), dim3(kWave), 0, st, f, actions, out);
   return hipGetLastError();
 }
 

@@ -6,6 +6,8 @@
 //   omq::fused_ucb_selection                                 (torch_custom_ops.py:26,71,108)
 //   omq::batch_apply_virtual_loss, omq::batch_remove_virtual_loss
 //                                      (batch_apply/remove_virtual_loss, mcts_kernels.cu:845-953)
+//   omq::fused_select_expand, omq::batched_ucb_selection
+//                                      the accelerator's functions of those names (torch_ops.py)
 //   omq::_alias_mcts(name)            registers the operator `name` under the reference's own
 //                                     namespace as well (mcts::name), for a name no module took;
 //                                     omq::_mcts_aliased(name) says whether it did
@@ -16,12 +18,15 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/full.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <memory>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "omq_tree_ops.h"
@@ -155,6 +160,75 @@ at::Tensor fused_ucb_selection(const at::Tensor& node_indices, const at::Tensor&
   return selected;
 }
 
+// mcts_kernels.cu:2002-2045: one descent per root over the dense children table; paths
+// [W, max_depth], path lengths, the nodes to expand and whether each needs expansion
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> fused_select_expand(
+    const at::Tensor& roots, const at::Tensor& children, const at::Tensor& visit_counts,
+    const at::Tensor& q_values, const at::Tensor& prior_probs, const at::Tensor& is_expanded,
+    int64_t max_depth, double c_puct) {
+  const char* name = "fused_select_expand";
+  const c10::Device dev = check_tensors(
+      name, {&roots, &children, &visit_counts, &q_values, &prior_probs, &is_expanded});
+  check_dtype(name, "roots", roots, at::kInt);
+  check_dtype(name, "children", children, at::kInt);
+  check_dtype(name, "visit_counts", visit_counts, at::kInt);
+  check_dtype(name, "q_values", q_values, at::kFloat);
+  check_dtype(name, "prior_probs", prior_probs, at::kFloat);
+  check_dtype(name, "is_expanded", is_expanded, at::kBool);
+  TORCH_CHECK(children.dim() == 2, "omq::", name, ": children must be [num_nodes, max_children]");
+  TORCH_CHECK(max_depth >= 1, "omq::", name, ": max_depth ", max_depth, " < 1");
+  const int64_t num_nodes =
+      std::min({children.size(0), visit_counts.numel(), q_values.numel(), prior_probs.numel(),
+                is_expanded.numel()});
+  const int64_t W = roots.numel();
+  const auto i32 = roots.options();
+  at::Tensor paths = at::empty({W, max_depth}, i32);
+  at::Tensor lengths = at::empty({W}, i32);
+  at::Tensor expand = at::empty({W}, i32);
+  at::Tensor needs = at::empty({W}, is_expanded.options());
+  const c10::hip::HIPGuard guard(dev.index());
+  check_rc(omq_fused_select_expand(
+               roots.data_ptr<int32_t>(), (int32_t)W, children.data_ptr<int32_t>(),
+               (int32_t)num_nodes, (int32_t)children.size(1), visit_counts.data_ptr<int32_t>(),
+               q_values.data_ptr<float>(), prior_probs.data_ptr<float>(),
+               reinterpret_cast<const uint8_t*>(is_expanded.data_ptr<bool>()),
+               (int32_t)max_depth, (float)c_puct, paths.data_ptr<int32_t>(),
+               lengths.data_ptr<int32_t>(), expand.data_ptr<int32_t>(),
+               reinterpret_cast<uint8_t*>(needs.data_ptr<bool>()), stream_of(dev)),
+           "omq_fused_select_expand");
+  return {paths, lengths, expand, needs};
+}
+
+// mcts_kernels.cu:1412-1464: the row position of each CSR row's UCB maximum; all -1 for an empty
+// batch, no children, or arrays whose sizes disagree (the kernel writes every row otherwise)
+at::Tensor batched_ucb_selection(const at::Tensor& q_values, const at::Tensor& visit_counts,
+                                 const at::Tensor& parent_visits, const at::Tensor& priors,
+                                 const at::Tensor& row_ptr, const at::Tensor& col_indices,
+                                 double c_puct) {
+  const char* name = "batched_ucb_selection";
+  const c10::Device dev = check_tensors(
+      name, {&q_values, &visit_counts, &parent_visits, &priors, &row_ptr, &col_indices});
+  check_dtype(name, "q_values", q_values, at::kFloat);
+  check_dtype(name, "visit_counts", visit_counts, at::kInt);
+  check_dtype(name, "parent_visits", parent_visits, at::kInt);
+  check_dtype(name, "priors", priors, at::kFloat);
+  check_dtype(name, "row_ptr", row_ptr, at::kInt);
+  check_dtype(name, "col_indices", col_indices, at::kInt);
+  const int64_t batch = parent_visits.numel(), nc = q_values.numel();
+  if (batch == 0 || nc == 0 || visit_counts.numel() != nc || priors.numel() != nc ||
+      col_indices.numel() != nc || row_ptr.numel() != batch + 1)
+    return at::full({batch}, -1, parent_visits.options());
+  at::Tensor selected = at::empty({batch}, parent_visits.options());
+  const c10::hip::HIPGuard guard(dev.index());
+  check_rc(omq_batched_ucb_selection(
+               q_values.data_ptr<float>(), visit_counts.data_ptr<int32_t>(), (int32_t)nc,
+               parent_visits.data_ptr<int32_t>(), priors.data_ptr<float>(),
+               row_ptr.data_ptr<int32_t>(), col_indices.data_ptr<int32_t>(), (int32_t)batch,
+               (float)c_puct, selected.data_ptr<int32_t>(), nullptr, stream_of(dev)),
+           "omq_batched_ucb_selection");
+  return selected;
+}
+
 // Meta kernels: shapes only
 void backup_meta(const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
                  const at::Tensor&) {}
@@ -165,6 +239,25 @@ at::Tensor fused_ucb_meta(const at::Tensor& node_indices, const at::Tensor&, con
   return at::empty({node_indices.numel()}, node_indices.options().dtype(at::kInt));
 }
 
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> select_expand_meta(
+    const at::Tensor& roots, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+    const at::Tensor&, const at::Tensor& is_expanded, int64_t max_depth, double) {
+  const int64_t W = roots.numel();
+  const auto i32 = roots.options();
+  return {at::empty({W, max_depth}, i32), at::empty({W}, i32), at::empty({W}, i32),
+          at::empty({W}, is_expanded.options())};
+}
+at::Tensor batched_ucb_meta(const at::Tensor&, const at::Tensor&, const at::Tensor& parent_visits,
+                            const at::Tensor&, const at::Tensor&, const at::Tensor&, double) {
+  return at::empty({parent_visits.numel()}, parent_visits.options());
+}
+
+constexpr const char* kSelectExpandSchema =
+    "(Tensor roots, Tensor children, Tensor visit_counts, Tensor q_values, Tensor prior_probs, "
+    "Tensor is_expanded, int max_depth, float c_puct) -> (Tensor, Tensor, Tensor, Tensor)";
+constexpr const char* kBatchedUcbSchema =
+    "(Tensor q_values, Tensor visit_counts, Tensor parent_visits, Tensor priors, "
+    "Tensor row_ptr, Tensor col_indices, float c_puct) -> Tensor";
 constexpr const char* kBackupSchema =
     "(Tensor paths, Tensor path_lengths, Tensor values, Tensor(a!) visit_counts, "
     "Tensor(b!) value_sums) -> ()";
@@ -235,6 +328,8 @@ TORCH_LIBRARY(omq, m) {
   for (const char* name : {"vectorized_backup", "warp_vectorized_backup", "fused_ucb_selection",
                            "batch_apply_virtual_loss", "batch_remove_virtual_loss"})
     define_op(m, name);
+  define(m, "fused_select_expand", kSelectExpandSchema, fused_select_expand, select_expand_meta);
+  define(m, "batched_ucb_selection", kBatchedUcbSchema, batched_ucb_selection, batched_ucb_meta);
   m.def("_alias_mcts(str name) -> bool", &alias_mcts);
   m.def("_mcts_aliased(str name) -> bool", &mcts_aliased);
 }

@@ -39,7 +39,11 @@ def child_key(key: int, action: int) -> int:
 
 
 def root_keys(seed: int, num_trees: int) -> np.ndarray:
-    return np.array([splitmix64((seed ^ t) & MASK64) for t in range(num_trees)], dtype=np.uint64)
+    z = np.array([(seed ^ t) & MASK64 for t in range(num_trees)], dtype=np.uint64)
+    z = z + np.uint64(GOLDEN)  # (splitmix64 over the array; uint64 arrays wrap)
+    z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    return z ^ (z >> np.uint64(31))
 
 
 @dataclass(frozen=True)
@@ -108,14 +112,12 @@ def legal_masks(model: GameModel, boards: np.ndarray | None, num_trees: int) -> 
     legal[:, :model.cells] = flat == 0
     if model.kind == "go":
         legal[:, model.num_actions - 1] = True
-    bits = legal.reshape(num_trees, model.legal_words, 32).astype(np.uint64)
-    weights = (np.uint64(1) << np.arange(32, dtype=np.uint64))
-    return (bits * weights).sum(axis=2).astype(np.uint32)
+    return np.packbits(legal, axis=1, bitorder="little").view("<u4").astype(np.uint32)
 
 
 def legal_counts(model: GameModel, masks: np.ndarray) -> np.ndarray:
-    return np.array([int(sum(bin(int(w)).count("1") for w in row)) for row in masks],
-                    dtype=np.int64)
+    rows = np.ascontiguousarray(masks, dtype=np.uint32)
+    return np.unpackbits(rows.view(np.uint8), axis=1).sum(axis=1, dtype=np.int64)
 
 
 def dirichlet_noise(model: GameModel, counts: np.ndarray, alpha: float, seed: int) -> np.ndarray:
@@ -127,7 +129,7 @@ def dirichlet_noise(model: GameModel, counts: np.ndarray, alpha: float, seed: in
         L = int(counts[t])
         if L > 0:
             g = np.random.Generator(np.random.PCG64(seed + t))
-            noise[t, :L] = g.dirichlet([alpha] * L)
+            noise[t, :L] = g.dirichlet(np.full(L, alpha, dtype=np.float64))
     return noise
 
 

@@ -17,6 +17,8 @@ reference registers itself are also registered under its own names,
     torch.ops.omq.batch_remove_virtual_loss(node_indices, virtual_loss_counts)
     torch.ops.omq.fused_ucb_selection(node_indices, children_start, children_end, children,
                                       q_values, visit_counts, priors, c_puct) -> int32 [batch]
+    torch.ops.omq.fused_select_expand, torch.ops.omq.batched_ucb_selection
+                                     (the functions of those names below)
 
 ``vectorized_backup`` follows the reference kernel (mcts_kernels.cu:121-158): for every path b
 and d < min(path_lengths[b], max_depth), node x = paths[b, d] in [0, num_nodes) gets
@@ -67,6 +69,10 @@ def _load_torch_ops() -> None:
 
 _load_torch_ops()
 
+# (the overloads themselves: the packets look theirs up at every call)
+_SELECT_EXPAND = torch.ops.omq.fused_select_expand.default
+_BATCHED_UCB = torch.ops.omq.batched_ucb_selection.default
+
 
 def _check_device(name: str, *tensors: torch.Tensor) -> torch.device:
     dev = tensors[0].device
@@ -91,7 +97,7 @@ def _forest(counts: torch.Tensor, sums: torch.Tensor | None) -> _lib.OmqForest:
 
 
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    return _lib.raw_stream(dev)
 
 
 def vectorized_backup(paths: torch.Tensor, path_lengths: torch.Tensor, values: torch.Tensor,
@@ -170,22 +176,8 @@ def batched_ucb_selection(q_values: torch.Tensor, visit_counts: torch.Tensor,
     """The row position of each CSR row's UCB maximum (batched_ucb_selection_cuda,
     mcts_kernels.cu:1412-1464); all -1 for an empty batch, no children, or arrays whose sizes
     disagree, as the reference returns."""
-    dev = _check_device("batched_ucb_selection", q_values, visit_counts, parent_visits, priors,
-                        row_ptr, col_indices)
-    _need("batched_ucb_selection", q_values=(q_values, torch.float32),
-          visit_counts=(visit_counts, torch.int32), parent_visits=(parent_visits, torch.int32),
-          priors=(priors, torch.float32), row_ptr=(row_ptr, torch.int32),
-          col_indices=(col_indices, torch.int32))
-    batch, nc = parent_visits.numel(), q_values.numel()
-    selected = torch.full((batch,), -1, dtype=torch.int32, device=dev)
-    if batch == 0 or nc == 0 or visit_counts.numel() != nc or priors.numel() != nc or \
-            col_indices.numel() != nc or row_ptr.numel() != batch + 1:
-        return selected
-    _lib.check(_lib.load().omq_batched_ucb_selection(
-        q_values.data_ptr(), visit_counts.data_ptr(), nc, parent_visits.data_ptr(),
-        priors.data_ptr(), row_ptr.data_ptr(), col_indices.data_ptr(), batch, float(c_puct),
-        selected.data_ptr(), None, _stream(dev)), "omq_batched_ucb_selection")
-    return selected
+    return _BATCHED_UCB(q_values, visit_counts, parent_visits, priors, row_ptr, col_indices,
+                        float(c_puct))
 
 
 def _table(name: str, children: torch.Tensor) -> tuple[int, int]:
@@ -199,27 +191,8 @@ def fused_select_expand(roots: torch.Tensor, children: torch.Tensor, visit_count
                         is_expanded: torch.Tensor, max_depth: int, c_puct: float):
     """(paths [W, max_depth], path_lengths, expand_nodes, needs_expansion) of one descent per
     root (fused_select_expand_cuda, mcts_kernels.cu:2002-2045)."""
-    name = "fused_select_expand"
-    dev = _check_device(name, roots, children, visit_counts, q_values, prior_probs, is_expanded)
-    _need(name, roots=(roots, torch.int32), children=(children, torch.int32),
-          visit_counts=(visit_counts, torch.int32), q_values=(q_values, torch.float32),
-          prior_probs=(prior_probs, torch.float32), is_expanded=(is_expanded, torch.bool))
-    rows, mc = _table(name, children)
-    num_nodes = min(rows, visit_counts.numel(), q_values.numel(), prior_probs.numel(),
-                    is_expanded.numel())
-    W, D = roots.numel(), int(max_depth)
-    if D < 1:
-        raise RuntimeError(f"omq::{name}: max_depth {D} < 1")
-    paths = torch.empty((W, D), dtype=torch.int32, device=dev)
-    plen = torch.empty(W, dtype=torch.int32, device=dev)
-    expand = torch.empty(W, dtype=torch.int32, device=dev)
-    needs = torch.empty(W, dtype=torch.bool, device=dev)
-    _lib.check(_lib.load().omq_fused_select_expand(
-        roots.data_ptr(), W, children.data_ptr(), num_nodes, mc, visit_counts.data_ptr(),
-        q_values.data_ptr(), prior_probs.data_ptr(), is_expanded.data_ptr(), D, float(c_puct),
-        paths.data_ptr(), plen.data_ptr(), expand.data_ptr(), needs.data_ptr(), _stream(dev)),
-        "omq_fused_select_expand")
-    return paths, plen, expand, needs
+    return _SELECT_EXPAND(roots, children, visit_counts, q_values, prior_probs, is_expanded,
+                          int(max_depth), float(c_puct))
 
 
 def fused_select_expand_optimized(root_nodes: torch.Tensor, children: torch.Tensor,
@@ -525,10 +498,10 @@ def extract_subtree_edges(row_ptr: torch.Tensor, col_indices: torch.Tensor, edge
     max_edges = int(max_edges)
     if max_edges < 0:
         raise RuntimeError(f"omq::{name}: max_edges {max_edges} < 0")
-    parents = torch.zeros(max_edges, dtype=torch.int32, device=dev)
-    children = torch.zeros(max_edges, dtype=torch.int32, device=dev)
-    actions = torch.zeros(max_edges, dtype=torch.int16, device=dev)
-    count = torch.zeros(1, dtype=torch.int32, device=dev)
+    parents = torch.empty(max_edges, dtype=torch.int32, device=dev)  # (the first k are returned)
+    children = torch.empty(max_edges, dtype=torch.int32, device=dev)
+    actions = torch.empty(max_edges, dtype=torch.int16, device=dev)
+    count = torch.empty(1, dtype=torch.int32, device=dev)
     ws = torch.empty(_lib.edges_workspace_ints(n), dtype=torch.int32, device=dev)
     _lib.check(_lib.load().omq_extract_subtree_edges(
         row_ptr.data_ptr(), col_indices.data_ptr(),

@@ -105,3 +105,24 @@ def test_root_ops_wide_boards(device, kind, bs):
     got = eng.noise.view(eng.T, eng.A).cpu().numpy()
     for t in range(eng.T):
         assert np.array_equal(got[t], orc.root_dirichlet(t, 0.03, 31, 4)), t
+
+
+@pytest.mark.parametrize("name", ["C1", "C3", "C4"])
+def test_root_children(device, name):
+    """The root's child for an action and its visits: rows of 20-45, 225 and up to 362 children,
+    the first, last and a middle child, absent actions, a lone root."""
+    wl = get(name).scaled(num_trees=5, num_simulations=64, wave_size=32, capacity=40_000)
+    eng, _, ev = make_pair(wl, device=device)
+    assert eng.root_children([0] * 5).tolist() == [[-1, 0]] * 5  # (not searched yet)
+    eng.search(wl.num_simulations, wl.wave_size, ev)
+    trees = [eng.host_tree(t) for t in range(5)]
+    for pick in (0, -1, 17):
+        first = [int(tr["first"][0]) + 1 for tr in trees]
+        node = [f + range(int(tr["nchild"][0]))[pick] for f, tr in zip(first, trees)]
+        acts = [int(tr["action"][n]) for tr, n in zip(trees, node)]
+        want = [[n, int(tr["N"][n])] for tr, n in zip(trees, node)]
+        assert eng.root_children(acts).tolist() == want
+    rows = [set(tr["action"][f:f + int(tr["nchild"][0])].tolist())
+            for tr, f in zip(trees, first)]
+    free = [next(a for a in range(eng.A + 1) if a not in row) for row in rows]
+    assert (eng.root_children(free)[:, 0] == -1).all()
