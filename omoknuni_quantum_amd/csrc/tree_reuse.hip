@@ -18,6 +18,7 @@
 // kernels follow: one gathers the kept nodes' fields into a workspace, the other writes them
 // over the front of the tree. The workspace holds eight int32 arrays of `capacity` entries
 // per tree.
+#include <algorithm>
 #include <mutex>
 
 #include "omq_common.h"
@@ -353,92 +354,194 @@ __device__ inline void bfs_row(const int32_t* row_ptr, int num_edges, int node, 
   *b = hi;
 }
 
-// candidate k of the level: the level position q with off[q] <= k < off[q + 1] (binary search
-// over off[0..L]), and its child
-__device__ inline int bfs_candidate(const int32_t* row_ptr, const int32_t* col, int num_edges,
-                                    const int32_t* level, const int32_t* off, int L, int k) {
-  int lo = 0, hi = L - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (off[mid] <= k) lo = mid; else hi = mid - 1;
-  }
-  int a, b;
-  bfs_row(row_ptr, num_edges, level[lo], &a, &b);
-  return col[a + (k - off[lo])];
-}
-
-// One workgroup.  Workspace: queue [max_nodes], claim [max_nodes], off [max_nodes + 1].
-__global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
-    const int32_t* row_ptr, const int32_t* col, int num_edges, int root, int max_nodes,
-    uint8_t* in_subtree, int32_t* remap, int32_t* count_out, int32_t* queue, int32_t* claim,
-    int32_t* off) {
-  __shared__ int64_t s_wtot[kBfsWaves];
-  const int tid = threadIdx.x;
-  for (int i = tid; i < max_nodes; i += kBfsThreads) {
-    in_subtree[i] = 0;
-    remap[i] = -1;
+// ---- breadth-first subtree ------------------------------------------------------------------
+// Marks, ids and claims of every node before the search, by the whole chip (one workgroup took
+// about a fifth of the search for it).
+__global__ void bfs_clear_kernel(int root, int max_nodes, uint8_t* in_subtree, int32_t* remap,
+                                 int32_t* claim, int32_t* queue) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < max_nodes;
+       i += gridDim.x * blockDim.x) {
+    in_subtree[i] = i == root ? 1 : 0;
+    remap[i] = i == root ? 0 : -1;
     claim[i] = 0x7FFFFFFF;
   }
-  __syncthreads();
-  if (tid == 0) {
-    in_subtree[root] = 1;
-    remap[root] = 0;
-    queue[0] = root;
-  }
-  __syncthreads();
+  if (blockIdx.x == 0 && threadIdx.x == 0) queue[0] = root;
+}
+
+// Exclusive scans of an int64 and an int per thread over the workgroup, together.
+__device__ inline int64_t bfs_block_scan2(int64_t v, int n, int64_t* s_wtot, int64_t* tot,
+                                          int* n_ex, int* n_tot) {
+  // (n's total stays below 2^16: it rides in the low bits of the scanned value)
+  const int64_t ex = bfs_block_scan((v << 16) | n, s_wtot, tot);
+  *n_ex = (int)(ex & 0xFFFF);
+  *n_tot = (int)(*tot & 0xFFFF);
+  *tot >>= 16;
+  return ex >> 16;
+}
+
+// The search, by one workgroup; its time is its chains of dependent loads, so every round has
+// many of them in flight.  A level's rows are taken kBfsPer nodes per thread at a time: a scan of
+// their lengths gives each row its place in the level's list of candidate edges, the rows with
+// edges are compacted in LDS, and the candidates are dealt in tiles of 64 (their row found by a
+// two-level search of that list, kBfsTiles tiles of a wave in flight).  Every candidate outside
+// the subtree claims its child with its place (the earliest wins), and is kept in the queue past
+// the level, where the winners are then numbered in order and compacted in place, kBfsNumber
+// candidates per thread and scan.  100k of 300k nodes: 208 us with one candidate per thread,
+// its row found by a binary search in memory, twice, and the clearing in this workgroup; 79 us so.  A level of more candidates than the queue has
+// room for (rows that overlap, repeated children) finds its candidates again for the numbering.
+// Workspace: queue [max_nodes], claim [max_nodes].
+constexpr int kBfsPer = 4;
+constexpr int kBfsChunk = kBfsThreads * kBfsPer;
+constexpr int kBfsTiles = 8;
+constexpr int kBfsNumber = 8;
+
+__global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
+    const int32_t* row_ptr, const int32_t* col, int num_edges, int max_nodes,
+    uint8_t* in_subtree, int32_t* remap, int32_t* count_out, int32_t* queue, int32_t* claim) {
+  __shared__ int64_t s_wtot[kBfsWaves];
+  __shared__ int s_cex[kBfsChunk];  // rows with edges: place of the first edge in the chunk
+  __shared__ int s_cof[kBfsChunk];  //   and its index in col
+  const int tid = threadIdx.x;
+  const int lane = lane_id();
+  const int wave = tid / kWave;
   int start = 0, end = 1;  // the current level: queue[start, end)
+  // The rows of level nodes [c0, c0 + kBfsChunk) into s_cex / s_cof; returns their number of
+  // edges, *nz the rows with any.  Ends with a barrier.
+  auto load_chunk = [&](int c0, int* nz) -> int64_t {
+    int of[kBfsPer], len[kBfsPer];
+    int64_t mine = 0;
+    int nzm = 0;
+    const int i0 = start + c0 + tid * kBfsPer;
+    int node[kBfsPer];
+#pragma unroll
+    for (int e = 0; e < kBfsPer; ++e) node[e] = i0 + e < end ? queue[i0 + e] : -1;
+#pragma unroll
+    for (int e = 0; e < kBfsPer; ++e) {
+      of[e] = len[e] = 0;
+      if (node[e] >= 0) {
+        int a, b;
+        bfs_row(row_ptr, num_edges, node[e], &a, &b);
+        of[e] = a;
+        len[e] = b - a;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kBfsPer; ++e) {
+      mine += len[e];
+      nzm += len[e] > 0 ? 1 : 0;
+    }
+    int64_t tot;
+    int zx;
+    int64_t ex = bfs_block_scan2(mine, nzm, s_wtot, &tot, &zx, nz);
+#pragma unroll
+    for (int e = 0; e < kBfsPer; ++e) {
+      if (len[e] > 0) {
+        s_cex[zx] = (int)min(ex, (int64_t)0x7FFFFFFF);
+        s_cof[zx] = of[e];
+        ++zx;
+      }
+      ex += len[e];
+    }
+    __syncthreads();
+    return tot;
+  };
+  // the child of candidate q0 + lane of the chunk (nz rows, tot candidates); called by whole waves
+  auto child_of = [&](int q0, int nz, int tot) -> int {
+    const int si = lane * kWave;
+    const uint64_t b1 = __ballot(si < nz && s_cex[si] <= q0);  // lane 0 always qualifies
+    const int S = kWave - 1 - __clzll(b1);
+    const int sj = S * kWave + lane;
+    const uint64_t b2 = __ballot(sj < nz && s_cex[sj] <= q0);
+    int j = S * kWave + (kWave - 1 - __clzll(b2));
+    const int q = q0 + lane;
+    if (q >= tot) return -1;
+    while (j + 1 < nz && s_cex[j + 1] <= q) ++j;
+    return col[s_cof[j] + (q - s_cex[j])];
+  };
+  auto outside = [&](int c) { return c >= 0 && c < max_nodes && !in_subtree[c]; };
+  auto claimed_by = [&](int c) {  // (past this CU's L1: claims are made by atomics in L2)
+    return __hip_atomic_load(&claim[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   bool overflow = false;
   while (start < end) {
     const int L = end - start;
-    const int32_t* level = queue + start;
-    // offsets of the level's rows in its list of candidates (level order, then row order)
     int64_t run = 0;
-    for (int c0 = 0; c0 < L; c0 += kBfsThreads) {
-      const int q = c0 + tid;
-      int64_t len = 0;
-      if (q < L) {
-        int a, b;
-        bfs_row(row_ptr, num_edges, level[q], &a, &b);
-        len = b - a;
+    bool stash = true;  // the level's candidates so far are in queue[end, end + run)
+    for (int c0 = 0; c0 < L; c0 += kBfsChunk) {
+      int nz;
+      const int64_t tot = load_chunk(c0, &nz);
+      if (run + tot > 0x7FFFFFFF) {  // more candidates than int32 keys (rows that overlap)
+        overflow = true;
+        break;
       }
-      int64_t tot;
-      const int64_t ex = bfs_block_scan(len, s_wtot, &tot);
-      if (q < L) off[q] = (int32_t)min(run + ex, (int64_t)0x7FFFFFFF);
+      stash = stash && end + run + tot <= max_nodes;
+      for (int64_t q0 = wave * kWave; q0 < tot; q0 += kBfsTiles * kBfsThreads) {
+        int c[kBfsTiles];
+        bool ok[kBfsTiles];
+#pragma unroll
+        for (int u = 0; u < kBfsTiles; ++u)
+          c[u] = q0 + u * kBfsThreads < tot
+                     ? child_of((int)q0 + u * kBfsThreads, nz, (int)tot) : -1;
+#pragma unroll
+        for (int u = 0; u < kBfsTiles; ++u) ok[u] = outside(c[u]);
+#pragma unroll
+        for (int u = 0; u < kBfsTiles; ++u) {
+          const int64_t q = q0 + u * kBfsThreads + lane;
+          if (ok[u]) atomicMin(&claim[c[u]], (int)(run + q));
+          if (stash && q < tot) queue[end + run + q] = ok[u] ? c[u] : -1;
+        }
+      }
       run += tot;
+      __syncthreads();  // the next chunk's rows overwrite the list
     }
-    if (run > 0x7FFFFFFF) {  // more candidates than int32 keys (rows that overlap)
-      overflow = true;
-      break;
-    }
-    const int total = (int)run;
-    if (tid == 0) off[L] = total;
-    __syncthreads();
-    // every candidate outside the subtree claims its child with its key (the earliest wins)
-    for (int k = tid; k < total; k += kBfsThreads) {
-      const int c = bfs_candidate(row_ptr, col, num_edges, level, off, L, k);
-      if (c >= 0 && c < max_nodes && !in_subtree[c]) atomicMin(&claim[c], k);
-    }
-    __syncthreads();
-    // the winners, numbered in key order
+    if (overflow) break;
+    // the winners, numbered in the order of the candidates
     int added = 0;
-    for (int k0 = 0; k0 < total; k0 += kBfsThreads) {
-      const int k = k0 + tid;
-      int c = -1;
-      bool win = false;
-      if (k < total) {
-        c = bfs_candidate(row_ptr, col, num_edges, level, off, L, k);
-        win = c >= 0 && c < max_nodes && !in_subtree[c] && claim[c] == k;
+    if (stash) {
+      for (int64_t k0 = 0; k0 < run; k0 += kBfsNumber * kBfsThreads) {
+        const int64_t k = k0 + tid * kBfsNumber;
+        int c[kBfsNumber], by[kBfsNumber];
+        int won = 0;
+#pragma unroll
+        for (int e = 0; e < kBfsNumber; ++e) c[e] = k + e < run ? queue[end + k + e] : -1;
+#pragma unroll
+        for (int e = 0; e < kBfsNumber; ++e) by[e] = c[e] >= 0 ? claimed_by(c[e]) : -1;
+#pragma unroll
+        for (int e = 0; e < kBfsNumber; ++e) won += c[e] >= 0 && by[e] == (int)(k + e) ? 1 : 0;
+        int64_t tot;
+        int at = end + added + (int)bfs_block_scan(won, s_wtot, &tot);
+#pragma unroll
+        for (int e = 0; e < kBfsNumber; ++e) {
+          if (c[e] >= 0 && by[e] == (int)(k + e)) {
+            remap[c[e]] = at;
+            in_subtree[c[e]] = 1;
+            queue[at] = c[e];  // (at or before the candidate's own place, read by now)
+            ++at;
+          }
+        }
+        added += (int)tot;
       }
-      int64_t tot;
-      const int ex = (int)bfs_block_scan(win ? 1 : 0, s_wtot, &tot);
-      if (win) {
-        remap[c] = end + added + ex;
-        queue[end + added + ex] = c;
+    } else {
+      run = 0;
+      for (int c0 = 0; c0 < L; c0 += kBfsChunk) {
+        int nz;
+        const int tot = (int)load_chunk(c0, &nz);
+        for (int64_t k0 = 0; k0 < tot; k0 += kBfsThreads) {
+          const int c = k0 + wave * kWave < tot ? child_of((int)k0 + wave * kWave, nz, tot) : -1;
+          const bool win = outside(c) && claimed_by(c) == (int)(run + k0 + tid);
+          int64_t wins;
+          const int at = end + added + (int)bfs_block_scan(win ? 1 : 0, s_wtot, &wins);
+          if (win) {
+            remap[c] = at;
+            queue[at] = c;
+          }
+          added += (int)wins;
+        }
+        run += tot;
+        __syncthreads();
       }
-      added += (int)tot;
+      for (int i = tid; i < added; i += kBfsThreads) in_subtree[queue[end + i]] = 1;
     }
-    __syncthreads();
-    for (int i = tid; i < added; i += kBfsThreads) in_subtree[queue[end + i]] = 1;
     __syncthreads();
     start = end;
     end += added;
@@ -446,32 +549,79 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
   if (tid == 0) count_out[0] = overflow ? -1 : end;
 }
 
-// Edge extraction: count per node and block scan (pass 1), scan of the block totals (pass 2),
-// writes (pass 3).  Workspace: local [num_nodes], block totals [blocks + 1].
+// Edge extraction: kept edges per wave and block scan (pass 1), scan of the block totals (pass 2),
+// writes (pass 3).  A wave takes kEdgeNodes consecutive nodes and their edges as one list, 64
+// edges at a time, kEdgeTiles such tiles in flight: consecutive lanes read consecutive edges and
+// write consecutive outputs.  100k edges of 300k nodes, of which a contiguous third is kept: one
+// node per thread with its row in a loop 20 us to count and 66 us to write, 64 nodes per wave 20
+// and 31 us (few waves hold all the edges), 16 nodes 12.5 and 14.3 us.  Workspace: the waves'
+// first edges [ceil(num_nodes / kEdgeNodes)], then the block totals.
 constexpr int kEdgeThreads = 1024;
+constexpr int kEdgeTiles = 4;
+constexpr int kEdgeNodes = 16;
+constexpr int kEdgeBlockNodes = kEdgeThreads / kWave * kEdgeNodes;
 
-__device__ inline int edges_kept(const int32_t* row_ptr, const int32_t* col, int num_edges,
-                                 const uint8_t* in_subtree, int num_nodes, int node) {
-  if (!in_subtree[node]) return 0;
-  int a, b;
-  bfs_row(row_ptr, num_edges, node, &a, &b);
-  int n = 0;
-  for (int e = a; e < b; ++e) {
-    const int c = col[e];
-    n += (c >= 0 && c < num_nodes && in_subtree[c]) ? 1 : 0;
+// Calls emit(keep mask, kept by this lane, edge, child, owner lane) for every tile of the kept
+// edges of the wave's nodes [n0, n0 + kEdgeNodes), in order.  Called by whole waves.
+template <class Emit>
+__device__ inline void walk_edges(const int32_t* row_ptr, const int32_t* col, int num_edges,
+                                  const uint8_t* in_subtree, int num_nodes, int64_t n0,
+                                  Emit emit) {
+  const int lane = lane_id();
+  const int64_t node = n0 + lane;
+  int a = 0, len = 0;
+  if (lane < kEdgeNodes && node < num_nodes && in_subtree[node]) {
+    int b;
+    bfs_row(row_ptr, num_edges, (int)node, &a, &b);
+    len = b - a;
   }
-  return n;
+  // places of the rows in the wave's list (int64: rows may overlap)
+  int64_t upto = len;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int64_t y = __shfl_up(upto, off, kWave);
+    if (lane >= off) upto += y;
+  }
+  const int64_t total = __shfl(upto, kWave - 1, kWave);
+  for (int64_t q0 = 0; q0 < total; q0 += kEdgeTiles * kWave) {
+    int edge[kEdgeTiles], own[kEdgeTiles], c[kEdgeTiles];
+    bool keep[kEdgeTiles];
+#pragma unroll
+    for (int u = 0; u < kEdgeTiles; ++u) {
+      const int64_t q = q0 + u * kWave + lane;
+      int lo = 0;  // the first lane whose rows end past q
+#pragma unroll
+      for (int h = kWave / 2; h >= 1; h >>= 1)
+        if (__shfl(upto, lo + h - 1, kWave) <= q) lo += h;
+      lo = min(lo, kWave - 1);
+      const int64_t from = __shfl(upto - len, lo, kWave);
+      const int64_t base = __shfl(a, lo, kWave);
+      own[u] = lo;
+      edge[u] = q < total ? (int)(base + (q - from)) : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < kEdgeTiles; ++u) c[u] = edge[u] >= 0 ? col[edge[u]] : -1;
+#pragma unroll
+    for (int u = 0; u < kEdgeTiles; ++u)
+      keep[u] = c[u] >= 0 && c[u] < num_nodes && in_subtree[c[u]];
+#pragma unroll
+    for (int u = 0; u < kEdgeTiles; ++u)
+      emit(__ballot(keep[u]), keep[u], edge[u], c[u], own[u]);
+  }
 }
 
 __global__ __launch_bounds__(kEdgeThreads) void edges_count_kernel(
     const int32_t* row_ptr, const int32_t* col, int num_edges, const uint8_t* in_subtree,
     int num_nodes, int32_t* local, int32_t* block_tot) {
   __shared__ int64_t s_wtot[kEdgeThreads / kWave];
-  const int i = blockIdx.x * kEdgeThreads + threadIdx.x;
-  const int n = i < num_nodes ? edges_kept(row_ptr, col, num_edges, in_subtree, num_nodes, i) : 0;
+  const int wave = (int)threadIdx.x / kWave;
+  const int64_t n0 = (int64_t)blockIdx.x * kEdgeBlockNodes + wave * kEdgeNodes;
+  int64_t n = 0;
+  walk_edges(row_ptr, col, num_edges, in_subtree, num_nodes, n0,
+             [&](uint64_t kept, bool, int, int, int) { n += __popcll(kept); });
   int64_t tot;
-  const int64_t ex = bfs_block_scan(n, s_wtot, &tot);
-  if (i < num_nodes) local[i] = (int32_t)ex;
+  const int64_t ex = bfs_block_scan(lane_id() == 0 ? n : 0, s_wtot, &tot);
+  if (lane_id() == 0 && n0 < num_nodes) local[n0 / kEdgeNodes] = (int32_t)ex;
   if (threadIdx.x == 0) block_tot[blockIdx.x] = (int32_t)tot;
 }
 
@@ -496,20 +646,25 @@ __global__ __launch_bounds__(kEdgeThreads) void edges_write_kernel(
     const uint8_t* in_subtree, const int32_t* remap, int num_nodes, int max_edges,
     const int32_t* local, const int32_t* block_off, int32_t* out_parent, int32_t* out_child,
     int16_t* out_action) {
-  const int i = blockIdx.x * kEdgeThreads + threadIdx.x;
-  if (i >= num_nodes || !in_subtree[i]) return;
-  int a, b;
-  bfs_row(row_ptr, num_edges, i, &a, &b);
-  int64_t pos = (int64_t)block_off[blockIdx.x] + local[i];
-  const int np = remap[i];
-  for (int e = a; e < b && pos < max_edges; ++e) {
-    const int c = col[e];
-    if (c < 0 || c >= num_nodes || !in_subtree[c]) continue;
-    out_parent[pos] = np;
-    out_child[pos] = remap[c];
-    out_action[pos] = actions != nullptr ? actions[e] : (int16_t)0;
-    ++pos;
-  }
+  const int lane = lane_id();
+  const int64_t n0 =
+      (int64_t)blockIdx.x * kEdgeBlockNodes + (int)threadIdx.x / kWave * kEdgeNodes;
+  if (n0 >= num_nodes) return;  // (whole waves)
+  const int id = n0 + lane < num_nodes ? remap[n0 + lane] : -1;
+  int64_t pos = (int64_t)block_off[blockIdx.x] + local[n0 / kEdgeNodes];
+  walk_edges(row_ptr, col, num_edges, in_subtree, num_nodes, n0,
+             [&](uint64_t kept, bool mine, int edge, int child, int owner) {
+               const int parent = __shfl(id, owner, kWave);
+               const int64_t at = pos + (int)__builtin_amdgcn_mbcnt_hi(
+                                            (uint32_t)(kept >> 32),
+                                            __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0u));
+               if (mine && at < max_edges) {
+                 out_parent[at] = parent;
+                 out_child[at] = remap[child];
+                 out_action[at] = actions != nullptr ? actions[edge] : (int16_t)0;
+               }
+               pos += __popcll(kept);
+             });
 }
 
 hipError_t launch_bfs_subtree(const int32_t* row_ptr, const int32_t* col, int num_edges,
@@ -517,13 +672,19 @@ hipError_t launch_bfs_subtree(const int32_t* row_ptr, const int32_t* col, int nu
                               int32_t* count, int32_t* ws, hipStream_t st) {
   int32_t* queue = ws;
   int32_t* claim = ws + max_nodes;
-  int32_t* off = ws + 2 * (int64_t)max_nodes;
+  const int blocks = std::min(1024, (max_nodes + 255) / 256);
+  hipLaunchKernelGGL(bfs_clear_kernel, dim3(blocks), dim3(256), 0, st, root, max_nodes,
+                     in_subtree, remap, claim, queue);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(bfs_subtree_kernel, dim3(1), dim3(kBfsThreads), 0, st, row_ptr, col,
-                     num_edges, root, max_nodes, in_subtree, remap, count, queue, claim, off);
+                     num_edges, max_nodes, in_subtree, remap, count, queue, claim);
   return hipGetLastError();
 }
 
-int edges_blocks(int num_nodes) { return (num_nodes + kEdgeThreads - 1) / kEdgeThreads; }
+int edges_blocks(int num_nodes) {
+  return (int)(((int64_t)num_nodes + kEdgeBlockNodes - 1) / kEdgeBlockNodes);
+}
 
 hipError_t launch_extract_edges(const int32_t* row_ptr, const int32_t* col, const int16_t* actions,
                                 int num_edges, const uint8_t* in_subtree, const int32_t* remap,
@@ -532,7 +693,8 @@ hipError_t launch_extract_edges(const int32_t* row_ptr, const int32_t* col, cons
                                 int32_t* ws, hipStream_t st) {
   const int blocks = edges_blocks(num_nodes);
   int32_t* local = ws;
-  int32_t* block_tot = ws + num_nodes;
+  // (together at most num_nodes / 16 + num_nodes / 256 + 2 of OMQ_EDGES_WORKSPACE_INTS)
+  int32_t* block_tot = ws + ((int64_t)num_nodes + kEdgeNodes - 1) / kEdgeNodes;
   if (blocks == 0) {
     hipLaunchKernelGGL(edges_scan_kernel, dim3(1), dim3(kEdgeThreads), 0, st, block_tot, 0,
                        edge_count);

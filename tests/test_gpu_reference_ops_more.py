@@ -255,3 +255,22 @@ def test_subtree_random_graphs(device, seed):
     rows = [list(rng.integers(0, n + 3, int(rng.integers(0, 6)))) for _ in range(n)]
     rows = [[int(c) for c in r] for r in rows]
     _check_subtree(device, rows, int(rng.integers(0, n)), n)
+
+
+@pytest.mark.parametrize("repeat", [0, 1])
+def test_subtree_wide_levels(device, repeat):
+    """Levels of 16000 nodes and 48000 edges, several chunks of rows and of candidates; with
+    every row listed again behind itself, a level has more candidates than the queue has room
+    for."""
+    rng = np.random.default_rng(7 + repeat)
+    sizes = [1, 40, 1600, 16000, 48000]
+    base = np.concatenate([[0], np.cumsum(sizes)])
+    n = int(base[-1])
+    rows = [[] for _ in range(n)]
+    for d in range(4):
+        kids = rng.permutation(np.arange(base[d + 1], base[d + 2]))
+        for c, p in zip(kids, rng.integers(base[d], base[d + 1], len(kids))):
+            rows[int(p)].append(int(c))
+    rows = [r + (r[::-1] if repeat else []) for r in rows]
+    _check_subtree(device, rows, 0, n)
+    _check_subtree(device, rows, int(np.argmax([len(r) for r in rows[1:41]])) + 1, n)
