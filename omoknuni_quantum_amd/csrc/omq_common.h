@@ -167,33 +167,67 @@ __device__ inline void xcd_block(int* bx, int* by) {
   *by = logical / X;
 }
 
-__device__ inline float wave_sum_canonical(float partial) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) partial = partial + __shfl_xor(partial, off, 64);
-  return partial;
+// The butterfly's lane exchanges stay in the vector registers: distances 32 and 16 by gfx950's
+// lane swaps, 8, 2 and 1 by DPP, 4 by two DPP moves (the xor by 7 mirrors a half row, the xor by
+// 3 a quad).  __shfl_xor goes through the LDS for each, 60-100 cycles a step against 8-16.
+template <int XOR>
+__device__ inline int lane_xor(int v) {
+  static_assert(XOR == 32 || XOR == 16 || XOR == 8 || XOR == 4 || XOR == 2 || XOR == 1, "");
+  if constexpr (XOR == 32 || XOR == 16) {
+    // the swap of v with itself leaves, in lane i, the values of lanes i and i ^ XOR in the two
+    // results (which is which depends on the half); their xor with v is the other one
+    const auto r = XOR == 32 ? __builtin_amdgcn_permlane32_swap(v, v, false, false)
+                             : __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (int)(r[0] ^ r[1]) ^ v;
+  } else if constexpr (XOR == 8) {
+    return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);  // row_ror:8
+  } else if constexpr (XOR == 4) {
+    const int m = __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true);  // row_half_mirror
+    return __builtin_amdgcn_mov_dpp(m, 0x1B, 0xF, 0xF, true);          // quad_perm [3,2,1,0]
+  } else {
+    return __builtin_amdgcn_mov_dpp(v, XOR == 2 ? 0x4E : 0xB1, 0xF, 0xF, true);
+  }
 }
+template <int XOR>
+__device__ inline float add_xor(float x) {
+  return x + __int_as_float(lane_xor<XOR>(__float_as_int(x)));
+}
+template <int XOR>
+__device__ inline double add_xor(double x) {
+  return x + __hiloint2double(lane_xor<XOR>(__double2hiint(x)), lane_xor<XOR>(__double2loint(x)));
+}
+template <class F>
+__device__ inline F wave_sum_butterfly(F x) {
+  x = add_xor<32>(x);
+  x = add_xor<16>(x);
+  x = add_xor<8>(x);
+  x = add_xor<4>(x);
+  x = add_xor<2>(x);
+  return add_xor<1>(x);
+}
+__device__ inline float wave_sum_canonical(float partial) { return wave_sum_butterfly(partial); }
 __device__ inline double wave_sum_canonical_d(double partial) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) partial = partial + __shfl_xor(partial, off, 64);
-  return partial;
+  return wave_sum_butterfly(partial);
 }
 
-__device__ inline int wave_sum_i(int v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+// Inclusive prefix sum over lanes, in the vector registers (DPP row shifts, then the row
+// broadcasts of lanes 15 and 31); a lane whose source lies outside its row reads 0.
+__device__ inline int wave_incl_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, true);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, true);  // row_bcast:31
+  return x;
 }
+
+__device__ inline int wave_sum_i(int v) { return readlane_i(wave_incl_scan(v), kWave - 1); }
 
 // exclusive prefix sum over lanes (lane 0 gets 0); total returned through *total
 __device__ inline int wave_excl_scan(int v, int* total) {
-  const int lane = lane_id();
-  int x = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    int y = __shfl_up(x, off, 64);
-    if (lane >= off) x += y;
-  }
-  *total = __shfl(x, 63, 64);
+  const int x = wave_incl_scan(v);
+  *total = readlane_i(x, kWave - 1);
   return x - v;
 }
 
