@@ -30,12 +30,31 @@ namespace omq {
 // the path length L (the leaf has L-1 moves on it).  *rp_out receives the root's player to
 // move: root_player[t], or 1 when the root board holds an even number of stones, else 2
 // (python/mcts/core/mcts.py:1503-1508); *stones_out the root board's stone count.
+// AHEAD: the path's first entries (most paths; one line of the row) are loaded with its length
+// instead of after it, and the board under the path's loads.  That is one of three dependent
+// rounds less for a kernel that waits for them (the feature planes: 512 slots 9.0 -> 6.0 us in the
+// kernel trace, 16384 slots 52.3 -> 48.9 us); the rule kernels, which spend their time on the
+// scan, gain nothing (Gomoku 13.3 -> 13.8 us, Go 11.7 -> 12.0 us with it).
+template <bool AHEAD>
 __device__ inline int rebuild_leaf_board(const omq_forest& f, const omq_wave& w,
                                          const int8_t* root_boards, const int32_t* root_player,
                                          int t, int u, int cells, int8_t* b, int* rp_out,
                                          int* stones_out) {
   const int lane = lane_id();
   const int8_t* rb = root_boards + (int64_t)t * cells;
+  int L = 0, a_lo = -1, a_hi = -1;
+  if constexpr (AHEAD) {
+    constexpr int kAhead = 16;
+    const int64_t s0 = (int64_t)t * w.max_wave + w.ufirst[(int64_t)t * w.max_wave + u];
+    const int64_t tb = (int64_t)t * f.capacity;
+    const int32_t* path = w.paths + s0 * w.max_depth;
+    const bool ahead = lane + 1 < min(kAhead, w.max_depth);
+    L = w.path_len[s0];
+    int node = ahead ? path[lane + 1] : 0;  // (past the path: unused)
+    if (!ahead && lane + 1 < L) node = path[lane + 1];
+    if (lane + 1 < L) a_lo = f.actions[tb + node];
+    if (lane + 65 < L) a_hi = f.actions[tb + path[lane + 65]];
+  }
   int stones = 0;
   for (int i = lane; i < cells; i += kWave) {
     const int8_t v = rb[i];
@@ -43,9 +62,10 @@ __device__ inline int rebuild_leaf_board(const omq_forest& f, const omq_wave& w,
     stones += v != 0;
   }
   stones = wave_sum_i(stones);
-  const int s0 = w.ufirst[(int64_t)t * w.max_wave + u];
-  int a_lo, a_hi;
-  const int L = load_path_actions(f, w, t, s0, &a_lo, &a_hi);
+  if constexpr (!AHEAD) {
+    const int s0 = w.ufirst[(int64_t)t * w.max_wave + u];
+    L = load_path_actions(f, w, t, s0, &a_lo, &a_hi);
+  }
   const int rp = root_player != nullptr ? root_player[t] : ((stones & 1) == 0 ? 1 : 2);
   wave_sync();
   // move j (0-based, depth j+1) is played by rp when j is even; lane l holds moves l and l+64
@@ -72,7 +92,7 @@ __global__ void gomoku_terminal_kernel(omq_forest f, omq_wave w, const int8_t* r
   if (u >= w.ucount[t]) return;
   int8_t* b = reinterpret_cast<int8_t*>(smem + (size_t)wave * stride);
   int rp, stones;
-  const int L = rebuild_leaf_board(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones);
+  const int L = rebuild_leaf_board<false>(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones);
   if (L <= 1) {  // the root position itself is not checked (the reference never flags it)
     if (uterm != nullptr && lane == 0) uterm[wb + u] = OMQ_TERM_NONE;
     return;
@@ -139,7 +159,7 @@ __global__ void go_rules_kernel(omq_forest f, omq_wave w, const int8_t* root_boa
   if (u >= w.ucount[t]) return;
   int8_t* b = reinterpret_cast<int8_t*>(smem + (size_t)wave * stride);
   int rp, stones;
-  const int L = rebuild_leaf_board(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones);
+  const int L = rebuild_leaf_board<false>(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones);
   // trailing passes of the path (moves 0..L-2; lane j holds move j, lane j holds move j+64 in
   // the high word)
   const int s0 = w.ufirst[wb + u];
@@ -284,7 +304,7 @@ __global__ __launch_bounds__(NW * kWave) void leaf_features_kernel(
   if (NW == 1 || tid < kWave) {
     int rp, stones;
     const int moves =
-        rebuild_leaf_board(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones) - 1;
+        rebuild_leaf_board<true>(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones) - 1;
     tm = (moves & 1) == 0 ? rp : 3 - rp;
     mc = (root_moves != nullptr ? root_moves[t] : stones) + moves;
     if (NW > 1 && tid == 0) {
