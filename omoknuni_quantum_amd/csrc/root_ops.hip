@@ -281,12 +281,17 @@ __global__ __launch_bounds__(kWave) void sample_actions_kernel(omq_forest f, con
 // ---- root Dirichlet noise -------------------------------------------------------------------
 // Entry i of row t is the noise of the i-th legal root action (the layout omq_expand reads).
 // The row's legal count L is the root's legal mask popcount (board models) or its sparse-model
-// count.  One workgroup per tree: lane-parallel gamma variates, then the canonical wave sum
-// and the division.
-__global__ __launch_bounds__(kWave) void root_dirichlet_kernel(omq_forest f, double alpha,
-                                                               uint64_t seed, uint64_t counter,
-                                                               double* noise) {
+// count (at most OMQ_MAX_ROW either way).  One workgroup per tree, one gamma variate per thread
+// (about 4 us each, a serial rejection loop in doubles: one wave per tree took them six in a row
+// on 362 actions, 24 us against 10 so), then the canonical wave sum by every wave and the division.
+constexpr int kNoiseThreads = OMQ_MAX_ROW;
+__global__ __launch_bounds__(kNoiseThreads) void root_dirichlet_kernel(omq_forest f, double alpha,
+                                                                       uint64_t seed,
+                                                                       uint64_t counter,
+                                                                       double* noise) {
+  __shared__ double s_g[OMQ_MAX_ROW];
   const int t = blockIdx.x;
+  const int tid = threadIdx.x;
   const int lane = lane_id();
   const int A = f.num_actions;
   double* row = noise + (int64_t)t * A;
@@ -299,16 +304,16 @@ __global__ __launch_bounds__(kWave) void root_dirichlet_kernel(omq_forest f, dou
       c += __popc(f.root_legal[(int64_t)t * f.legal_words + i]);
     L = wave_sum_i(c);
   }
-  double part = 0.0;
-  for (int i = lane; i < L; i += kWave) {
+  for (int i = tid; i < L && i < OMQ_MAX_ROW; i += kNoiseThreads) {
     Stream st = make_stream(seed, counter, t, i);
-    const double g = gamma_mt(alpha, st);
-    row[i] = g;
-    part = part + g;
+    s_g[i] = gamma_mt(alpha, st);
   }
+  __syncthreads();
+  double part = 0.0;
+  for (int i = lane; i < L && i < OMQ_MAX_ROW; i += kWave) part = part + s_g[i];
   const double S = wave_sum_canonical_d(part);
-  for (int i = lane; i < A; i += kWave) {
-    if (i < L) row[i] = S > 0.0 ? row[i] / S : 1.0 / (double)L;
+  for (int i = tid; i < A; i += kNoiseThreads) {
+    if (i < L) row[i] = S > 0.0 ? s_g[i] / S : 1.0 / (double)L;
     else row[i] = 0.0;
   }
 }
@@ -369,8 +374,8 @@ hipError_t launch_sample_actions(const omq_forest& f, const double* pol, double 
 
 hipError_t launch_root_dirichlet(const omq_forest& f, double alpha, uint64_t seed,
                                  uint64_t counter, double* noise, hipStream_t st) {
-  hipLaunchKernelGGL(root_dirichlet_kernel, dim3(f.num_trees), dim3(kWave), 0, st, f, alpha, seed,
-                     counter, noise);
+  hipLaunchKernelGGL(root_dirichlet_kernel, dim3(f.num_trees), dim3(kNoiseThreads), 0, st, f,
+                     alpha, seed, counter, noise);
   return hipGetLastError();
 }
 
