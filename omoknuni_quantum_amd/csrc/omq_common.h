@@ -52,14 +52,15 @@ __device__ inline float key_normal(uint64_t k, int a) {
   uint64_t h0 = splitmix64(k ^ ((uint64_t)(a + 1) * kSaltLogit));
   uint64_t h1 = splitmix64(h0);
   uint64_t h2 = splitmix64(h1);
-  int32_t s = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    s += (int32_t)((h0 >> (16 * i)) & 0xFFFF);
-    s += (int32_t)((h1 >> (16 * i)) & 0xFFFF);
-    s += (int32_t)((h2 >> (16 * i)) & 0xFFFF);
-  }
-  return (float)(s + 6 - 393216) * (1.0f / 65536.0f);
+  // the twelve 16-bit fields, two per instruction (|x - 0| summed over both halves)
+  uint32_t s = 0;
+  s = __builtin_amdgcn_sad_u16((uint32_t)h0, 0u, s);
+  s = __builtin_amdgcn_sad_u16((uint32_t)(h0 >> 32), 0u, s);
+  s = __builtin_amdgcn_sad_u16((uint32_t)h1, 0u, s);
+  s = __builtin_amdgcn_sad_u16((uint32_t)(h1 >> 32), 0u, s);
+  s = __builtin_amdgcn_sad_u16((uint32_t)h2, 0u, s);
+  s = __builtin_amdgcn_sad_u16((uint32_t)(h2 >> 32), 0u, s);
+  return (float)((int32_t)s + 6 - 393216) * (1.0f / 65536.0f);
 }
 
 // e^x from basic operations: Cody-Waite reduction x = k ln2 + r (ln2 split into a 15-bit

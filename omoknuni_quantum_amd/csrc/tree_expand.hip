@@ -107,6 +107,9 @@ __global__ __launch_bounds__(kLeafInfoThreads) void leaf_info_kernel(omq_forest 
 }
 
 // ---------------------------------------------------------------------------------------
+// Bound by the logits' hashes, six 64-bit products per action at a quarter of the vector rate
+// (32 x 1024 leaves of about 300 actions: 41 us; 45 us with the hash's twelve fields taken out one
+// by one and the logits kept as doubles).
 __global__ void synth_eval_kernel(omq_forest f, omq_wave w, float scale) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int t = blockIdx.y;
@@ -119,22 +122,23 @@ __global__ void synth_eval_kernel(omq_forest f, omq_wave w, float scale) {
   const uint64_t key = w.ukey[wb + u];
   const int n = leaf_legal_list(f, w, t, u, l.mask, l.list);
   float* row = w.policy + (wb + u) * (int64_t)f.num_actions;
-  // the scaled logits are kept in the wave's LDS (exactly, as doubles) for the second pass
+  // the scaled logits, then their exponentials, are kept in the wave's LDS
+  float* val = reinterpret_cast<float*>(l.val);
   float mx = -__builtin_inff();
   for (int i = lane; i < n; i += kWave) {
     const float z = scale * key_normal(key, l.list[i]);
-    l.val[i] = (double)z;
+    val[i] = z;
     mx = fmaxf(mx, z);
   }
   mx = wave_max_f32(mx);
   float part = 0.0f;
   for (int i = lane; i < n; i += kWave) {
-    const float e = exp_cw((float)l.val[i] - mx);
-    l.val[i] = (double)e;
+    const float e = exp_cw(val[i] - mx);
+    val[i] = e;
     part = part + e;
   }
   const float S = wave_sum_canonical(part);
-  for (int i = lane; i < n; i += kWave) row[l.list[i]] = (float)l.val[i] / S;
+  for (int i = lane; i < n; i += kWave) row[l.list[i]] = val[i] / S;
   if (lane == 0) w.values[wb + u] = key_value(key);
 }
 
