@@ -710,10 +710,15 @@ struct ChainCfg {
   int vli;
 };
 
-template <int R, bool PERSIST, bool PARTIAL>
+// OWN_PREFIX (one child per lane): the chain finds its first-unvisited prefix itself, from the
+// counts it loads anyway, and starts after it; *all_prefix is set when that takes every rank.  (A
+// separate pass over the counts first costs each group a round of loads and a call: 16 trees,
+// waves of 2048 on rows of 20-45 children, select 431 -> 419 us per launch.)
+template <int R, bool PERSIST, bool PARTIAL, bool OWN_PREFIX = false>
 __device__ int run_chain(ChainRows f, int64_t tb, int first, int k, int Np0, int m, int npre,
                          ChainCfg c, uint32_t* ch, uint16_t* cnt_s, float4* cscr,
-                         int* progress, const int* stop) {
+                         int* progress, const int* stop, bool* all_prefix = nullptr) {
+  static_assert(!OWN_PREFIX || (R == 1 && !PARTIAL), "");
   const int lane = lane_id();
   const float vlf = c.vlf;
   const float fvl = (float)c.vli;
@@ -723,6 +728,7 @@ __device__ int run_chain(ChainRows f, int64_t tb, int first, int k, int Np0, int
   float qbl = 0.0f;
   bool negcp = false;
   int pre0 = 0;  // (R == 1) the lane's child was taken by the prefix
+  bool unv = false;  // (OWN_PREFIX) the lane's child is unvisited
 #pragma unroll
   for (int j = 0; j < R; ++j) {
     const int i = j * kWave + lane;
@@ -739,6 +745,7 @@ __device__ int run_chain(ChainRows f, int64_t tb, int first, int k, int Np0, int
         d = d + fvl * (float)pre;  // (exact: integers below 2^24)
         if (j == 0) pre0 = pre;
       }
+      if (OWN_PREFIX) unv = n == 0;
       negcp = negcp || !(cpv >= 0.0f);
       if (child_state(d, w, cpv, i, vlf, &qv, &av)) qbl = fmaxf(qbl, __builtin_fabsf(qv));
     }
@@ -747,6 +754,31 @@ __device__ int run_chain(ChainRows f, int64_t tb, int first, int k, int Np0, int
     x.cp[j] = cpv;
     x.q[j] = qv;
     x.ar[j] = av;
+  }
+  if (OWN_PREFIX && c.vli > 0) {
+    const uint64_t um = __ballot(unv);
+    const int pos = (int)__builtin_amdgcn_mbcnt_hi(
+        (uint32_t)(um >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)um, 0u));
+    npre = min(__popcll(um), m);
+    const bool taken = unv && pos < m;
+    if (taken) ch[pos] = (uint32_t)lane << 16;
+    if (npre >= m) {
+      if (lane < k) cnt_s[lane] = taken ? 1 : 0;
+      wave_sync();
+      *all_prefix = true;
+      if (progress != nullptr) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0)
+          __hip_atomic_store(progress, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      return -1;
+    }
+    if (taken) {  // (the prefix took every unvisited child: one pick each)
+      pre0 = 1;
+      x.den[0] = 1.0f + fvl;
+      if (child_state(x.den[0], x.wv[0], x.cp[0], lane, vlf, &x.q[0], &x.ar[0]))
+        qbl = fmaxf(qbl, __builtin_fabsf(x.q[0]));
+    }
   }
   const uint32_t QBb = wave_max_rows(__float_as_uint(qbl));  // bits of QB (non-negative)
   const float qbt = __uint_as_float(QBb) * (-1.0f / 524288.0f);
@@ -830,13 +862,14 @@ __device__ int run_chain(ChainRows f, int64_t tb, int first, int k, int Np0, int
     conbits = 0u;
     wopen = false;
   };
-  for (int r0 = PARTIAL ? (npre / kWave) * kWave : 0; r0 < m; r0 += kWave) {
+  constexpr bool kAfter = PARTIAL || OWN_PREFIX;  // ranks [0, npre) are taken already
+  for (int r0 = kAfter ? (npre / kWave) * kWave : 0; r0 < m; r0 += kWave) {
     const int Npl = Np0 + c.vli * (r0 + lane + 1);
     const float svec = sqrtf((float)Npl);
     const int rend = __builtin_amdgcn_readfirstlane(min(kWave, m - r0));
     // the block's ranks taken by the prefix (npre is uniform: a call's result is not known
     // to be, so it is made so here)
-    const int rs = PARTIAL ? __builtin_amdgcn_readfirstlane(max(0, npre - r0)) : 0;
+    const int rs = kAfter ? __builtin_amdgcn_readfirstlane(max(0, npre - r0)) : 0;
     // lane rr of rec / rnk: the child picked at rank r0+rr and the chain's picks of that child
     // up to and including it (the picked lane's count after the pick: its rank plus one)
     uint32_t rec = kNoChild;
@@ -1050,6 +1083,11 @@ __device__ inline int group_chain(ChainRows rows, int64_t tb, int first, int k, 
     *all_prefix = false;
     return dispatch_chain<RMAX, WIDE>(rows, tb, first, k, Np0, m, taken, cc, ch, cnt_s, cscr,
                                       progress, stop);
+  }
+  if constexpr (RMAX == 1 && !WIDE) {
+    *all_prefix = false;
+    return run_chain<1, true, false, true>(rows, tb, first, k, Np0, m, 0, cc, ch, cnt_s, cscr,
+                                           progress, stop, all_prefix);
   }
   const int npre = unvisited_prefix<RMAX>(rows.N, tb, first, k, m, cc.vli > 0, ch, cnt_s);
   *all_prefix = npre >= m;
