@@ -33,8 +33,7 @@ namespace omq {
 // AHEAD: the path's first entries (most paths; one line of the row) are loaded with its length
 // instead of after it, and the board under the path's loads.  That is one of three dependent
 // rounds less for a kernel that waits for them (the feature planes: 512 slots 9.0 -> 6.0 us in the
-// kernel trace, 16384 slots 52.3 -> 48.9 us); the rule kernels, which spend their time on the
-// scan, gain nothing (Gomoku 13.3 -> 13.8 us, Go 11.7 -> 12.0 us with it).
+// kernel trace, 16384 slots 52.3 -> 48.9 us); the rule kernels gain nothing.
 template <bool AHEAD>
 __device__ inline int rebuild_leaf_board(const omq_forest& f, const omq_wave& w,
                                          const int8_t* root_boards, const int32_t* root_player,
@@ -78,26 +77,90 @@ __device__ inline int rebuild_leaf_board(const omq_forest& f, const omq_wave& w,
   return L;
 }
 
-__global__ void gomoku_terminal_kernel(omq_forest f, omq_wave w, const int8_t* root_boards,
-                                       const int32_t* root_player, int rule, int bs,
-                                       int32_t* uterm) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int cells = bs * bs;
-  const int stride = (cells + 15) & ~15;
-  const int t = blockIdx.y;
-  const int wave = threadIdx.x / kWave;
-  const int u = blockIdx.x * (blockDim.x / kWave) + wave;
-  const int lane = lane_id();
-  const int64_t wb = (int64_t)t * w.max_wave;
-  if (u >= w.ucount[t]) return;
-  int8_t* b = reinterpret_cast<int8_t*>(smem + (size_t)wave * stride);
-  int rp, stones;
-  const int L = rebuild_leaf_board<false>(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones);
-  if (L <= 1) {  // the root position itself is not checked (the reference never flags it)
-    if (uterm != nullptr && lane == 0) uterm[wb + u] = OMQ_TERM_NONE;
-    return;
-  }
+// LDS of a wave of the rule kernels: a board in bytes, or row words for two players.
+__host__ __device__ inline int rule_lds_per_wave(int cells) {
+  const int words = 2 * (2 * ((OMQ_MAX_ROW + kWave - 1) / kWave) + 2) * 4;
+  const int board = (cells + 15) & ~15;
+  return board > words ? board : (words + 15) & ~15;
+}
 
+// ---- boards as row masks ----------------------------------------------------------------------
+// Lane r holds row r of a board as bits (bit c: column c), at most 22 rows and columns.  The rules
+// are then shifts of whole rows: a few dozen instructions a leaf, where the scan of the cells
+// from LDS bytes takes up to 20 dependent reads per cell and direction.
+constexpr int kRowWords = 2 * ((OMQ_MAX_ROW + kWave - 1) / kWave) + 2;  // and a pad
+
+// The set of cells as rows, from one ballot per 64 cells in the wave's LDS words.
+struct RowBits {
+  uint32_t* words;  // [kRowWords] of the wave's LDS
+  __device__ void clear() const {
+    if (lane_id() < kRowWords) words[lane_id()] = 0u;
+  }
+  __device__ void put(int c0, uint64_t cells64) const {  // cells c0 .. c0 + 63
+    if (lane_id() < 2)
+      words[(c0 >> 5) + lane_id()] = lane_id() == 0 ? (uint32_t)cells64
+                                                    : (uint32_t)(cells64 >> 32);
+  }
+  __device__ uint32_t row(int bs) const {  // (after wave_sync)
+    const int r = lane_id();
+    if (r >= bs) return 0u;
+    const int o = r * bs;
+    const uint64_t x = (uint64_t)words[(o >> 5) + 1] << 32 | words[o >> 5];
+    return (uint32_t)(x >> (o & 31)) & ((1u << bs) - 1u);
+  }
+};
+
+// Calls stone(move, bit) for the path's moves on the board in order: bit is the move's column in
+// the lane of its row, 0 in the others.
+template <class Stone>
+__device__ inline void each_move(int L, int a_lo, int a_hi, int cells, int bs, Stone stone) {
+  const int lane = lane_id();
+  const int r_lo = a_lo / bs, r_hi = a_hi / bs;
+  const int c_lo = a_lo - r_lo * bs, c_hi = a_hi - r_hi * bs;
+  for (int j = 0; j + 1 < L; ++j) {
+    const bool lo = j < kWave;
+    const int jj = j & (kWave - 1);
+    const int a = lo ? readlane_i(a_lo, jj) : readlane_i(a_hi, jj);
+    if (a < 0 || a >= cells) continue;
+    const int r = lo ? readlane_i(r_lo, jj) : readlane_i(r_hi, jj);
+    const int c = lo ? readlane_i(c_lo, jj) : readlane_i(c_hi, jj);
+    stone(j, lane == r ? 1u << c : 0u);
+  }
+}
+
+// Row l + k of the rows in m (0 past the board: lanes past it hold 0).
+__device__ inline uint32_t row_at(uint32_t m, int k) {
+  const int l = lane_id() + k;
+  const uint32_t x = (uint32_t)__shfl((int)m, l & (kWave - 1), kWave);
+  return l >= 0 ? x : 0u;
+}
+
+// The cells of the player's rows m where a counting five starts (the file comment's rule; over:
+// renju's player 1, whose overlines end the scan of their cell).
+__device__ inline uint32_t five_starts(uint32_t m, bool over) {
+  const uint32_t d1 = row_at(m, 1), d2 = row_at(m, 2), d3 = row_at(m, 3), d4 = row_at(m, 4);
+  const uint32_t h = m & m >> 1 & m >> 2 & m >> 3 & m >> 4;
+  const uint32_t v = m & d1 & d2 & d3 & d4;
+  const uint32_t dr = m & d1 >> 1 & d2 >> 2 & d3 >> 3 & d4 >> 4;
+  const uint32_t dl = m & d1 << 1 & d2 << 2 & d3 << 3 & d4 << 4;
+  if (!over) return h | v | dr | dl;
+  const uint32_t d5 = row_at(m, 5), u1 = row_at(m, -1);
+  uint32_t win = 0u, ended = 0u;  // (the directions in the scan's order)
+  auto dir = [&](uint32_t five, uint32_t longer) {
+    const uint32_t f = five & ~win & ~ended;
+    ended |= f & longer;
+    win |= f & ~longer;
+  };
+  dir(h, m >> 5 | m << 1);
+  dir(v, d5 | u1);
+  dir(dr, d5 >> 5 | u1 << 1);
+  dir(dl, d5 << 5 | u1 >> 1);
+  return win;
+}
+
+// The terminal code of the position in the wave's LDS board b by a scan of its cells.
+__device__ inline int scan_terminal(const int8_t* b, int cells, int bs, int rule) {
+  const int lane = lane_id();
   constexpr int dr[4] = {0, 1, 1, 1};
   constexpr int dc[4] = {1, 0, 1, -1};
   int win = 0x7FFFFFFF;
@@ -133,38 +196,108 @@ __global__ void gomoku_terminal_kernel(omq_forest f, omq_wave w, const int8_t* r
   int code = OMQ_TERM_NONE;
   if (win != 0x7FFFFFFF) code = b[win];
   else if (empty == 0) code = OMQ_TERM_DRAW;
-  if (lane == 0) {
-    if (code != OMQ_TERM_NONE) w.ulegal[wb + u] = 0;
-    if (uterm != nullptr) uterm[wb + u] = code;
-  }
+  return code;
 }
 
-// Go rules of unique leaf u of tree t (one wavefront per leaf): the leaf's position is rebuilt
-// as for Gomoku (a pass, action cells, places no stone), then lane l takes the points l, l+64,
-// ... of the board.  A point is legal when it is empty, is not the root's ko point (OMQ_GO_KO:
-// the reference's clones inherit a state's ko point, so it holds at every depth), and, with
-// OMQ_GO_SUICIDE, has an empty orthogonal neighbour; the pass is always legal.  The 64 points of each chunk become two mask words by one ballot.  Trailing passes are
-// counted from the path's end (the root's own when every path move is a pass).
-__global__ void go_rules_kernel(omq_forest f, omq_wave w, const int8_t* root_boards,
-                                const int32_t* root_player, const int32_t* root_passes,
-                                const int32_t* root_ko, int flags, int bs, int32_t* uterm) {
+// One wavefront per unique leaf, on the row masks of the two players; a board with other stones
+// than 1 and 2, or another root player, is scanned cell by cell as the reference scans it.  64
+// trees of 256 leaves, 15x15: 13.0 us with the scan for every board, 10.3 us so; 16 trees of 32
+// leaves 5.8 and 4.2 us.
+__global__ void gomoku_terminal_kernel(omq_forest f, omq_wave w, const int8_t* root_boards,
+                                       const int32_t* root_player, int rule, int bs,
+                                       int32_t* uterm) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int cells = bs * bs;
-  const int stride = (cells + 15) & ~15;
+  const int stride = rule_lds_per_wave(cells);
   const int t = blockIdx.y;
   const int wave = threadIdx.x / kWave;
   const int u = blockIdx.x * (blockDim.x / kWave) + wave;
   const int lane = lane_id();
   const int64_t wb = (int64_t)t * w.max_wave;
   if (u >= w.ucount[t]) return;
-  int8_t* b = reinterpret_cast<int8_t*>(smem + (size_t)wave * stride);
-  int rp, stones;
-  const int L = rebuild_leaf_board<false>(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones);
-  // trailing passes of the path (moves 0..L-2; lane j holds move j, lane j holds move j+64 in
-  // the high word)
   const int s0 = w.ufirst[wb + u];
   int a_lo, a_hi;
-  load_path_actions(f, w, t, s0, &a_lo, &a_hi);
+  const int L = load_path_actions(f, w, t, s0, &a_lo, &a_hi);
+  if (L <= 1) {  // the root position itself is not checked (the reference never flags it)
+    if (uterm != nullptr && lane == 0) uterm[wb + u] = OMQ_TERM_NONE;
+    return;
+  }
+  const RowBits one{reinterpret_cast<uint32_t*>(smem + (size_t)wave * stride)};
+  const RowBits two{one.words + kRowWords};
+  one.clear();
+  two.clear();
+  wave_sync();
+  const int8_t* rb = root_boards + (int64_t)t * cells;
+  int stones = 0;
+  uint64_t other = 0;
+  for (int c0 = 0; c0 < cells; c0 += kWave) {
+    const int v = c0 + lane < cells ? rb[c0 + lane] : 0;
+    const uint64_t b1 = __ballot(v == 1), b2 = __ballot(v == 2), bx = __ballot(v != 0);
+    one.put(c0, b1);
+    two.put(c0, b2);
+    stones += __popcll(bx);
+    other |= bx & ~(b1 | b2);
+  }
+  const int rp = root_player != nullptr ? root_player[t] : ((stones & 1) == 0 ? 1 : 2);
+  wave_sync();
+  int code = OMQ_TERM_NONE;
+  if (other == 0 && (rp == 1 || rp == 2)) {
+    uint32_t m1 = one.row(bs), m2 = two.row(bs);
+    each_move(L, a_lo, a_hi, cells, bs, [&](int j, uint32_t bit) {
+      const bool first = ((j & 1) == 0) == (rp == 1);  // played by player 1
+      m1 = first ? m1 | bit : m1 & ~bit;
+      m2 = first ? m2 & ~bit : m2 | bit;
+    });
+    const uint32_t f1 = five_starts(m1, rule == OMQ_RULE_RENJU), f2 = five_starts(m2, false);
+    const uint64_t rows = __ballot((f1 | f2) != 0u);
+    if (rows != 0) {  // the first cell in row-major order names the winner
+      const int c = __ffs(f1 | f2) - 1;
+      code = readlane_i((f1 >> (c & 31)) & 1u ? 1 : 2, lowest_lane(rows));
+    } else if (wave_sum_i(__popc(m1 | m2)) == cells) {
+      code = OMQ_TERM_DRAW;
+    }
+  } else {
+    int8_t* b = reinterpret_cast<int8_t*>(smem + (size_t)wave * stride);
+    wave_sync();
+    int rp2, stones2;
+    rebuild_leaf_board<false>(f, w, root_boards, root_player, t, u, cells, b, &rp2, &stones2);
+    code = scan_terminal(b, cells, bs, rule);
+  }
+  if (lane == 0) {
+    if (code != OMQ_TERM_NONE) w.ulegal[wb + u] = 0;
+    if (uterm != nullptr) uterm[wb + u] = code;
+  }
+}
+
+// Go rules of unique leaf u of tree t (one wavefront per leaf), on the row masks of the empty
+// points (a pass, action cells, places no stone).  A point is legal when it is empty, is not the
+// root's ko point (OMQ_GO_KO: the reference's clones inherit a state's ko point, so it holds at
+// every depth), and, with OMQ_GO_SUICIDE, has an empty orthogonal neighbour; the pass is always
+// legal.  The rows are put together to the leaf's mask words in LDS.  Trailing passes are counted
+// from the path's end (the root's own when every path move is a pass).  16 trees of 512 leaves,
+// 19x19: 11.5 us with the points read one by one from an LDS board, 7.0 us so.
+__global__ void go_rules_kernel(omq_forest f, omq_wave w, const int8_t* root_boards,
+                                const int32_t* root_player, const int32_t* root_passes,
+                                const int32_t* root_ko, int flags, int bs, int32_t* uterm) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int cells = bs * bs;
+  const int stride = rule_lds_per_wave(cells);
+  const int t = blockIdx.y;
+  const int wave = threadIdx.x / kWave;
+  const int u = blockIdx.x * (blockDim.x / kWave) + wave;
+  const int lane = lane_id();
+  const int64_t wb = (int64_t)t * w.max_wave;
+  if (u >= w.ucount[t]) return;
+  const int s0 = w.ufirst[wb + u];
+  int a_lo, a_hi;
+  const int L = load_path_actions(f, w, t, s0, &a_lo, &a_hi);
+  const RowBits bits{reinterpret_cast<uint32_t*>(smem + (size_t)wave * stride)};
+  bits.clear();
+  wave_sync();
+  const int8_t* rb = root_boards + (int64_t)t * cells;
+  for (int c0 = 0; c0 < cells; c0 += kWave)
+    bits.put(c0, __ballot(c0 + lane < cells && rb[c0 + lane] == 0));
+  // trailing passes of the path (moves 0..L-2; lane j holds moves j and j+64)
   int trail = 0;
   for (int j = L - 2; j >= 0; --j) {
     const int a = j < kWave ? readlane_i(a_lo, j) : readlane_i(a_hi, j - kWave);
@@ -173,33 +306,35 @@ __global__ void go_rules_kernel(omq_forest f, omq_wave w, const int8_t* root_boa
   }
   if (trail == L - 1 && root_passes != nullptr) trail += root_passes[t];
   const int ko = ((flags & OMQ_GO_KO) && root_ko != nullptr) ? root_ko[t] : -1;
-  const bool suicide = (flags & OMQ_GO_SUICIDE) != 0;
-  uint32_t* mask = w.umask + (wb + u) * (int64_t)f.legal_words;
-  int legal = 0, empty = 0;
-  // points 0..cells-1, then the pass (action cells, always legal)
-  for (int c0 = 0; c0 <= cells; c0 += kWave) {
-    const int c = c0 + lane;
-    bool ok = c == cells;
-    if (c < cells && b[c] == 0) {
-      ++empty;
-      ok = c != ko;
-      if (ok && suicide) {
-        const int r = c / bs, col = c - r * bs;
-        const bool lib = (r > 0 && b[c - bs] == 0) || (r + 1 < bs && b[c + bs] == 0) ||
-                         (col > 0 && b[c - 1] == 0) || (col + 1 < bs && b[c + 1] == 0);
-        ok = lib;
-      }
-    }
-    const uint64_t m = __ballot(ok);
-    legal += ok ? 1 : 0;
-    // words c0/32 and c0/32 + 1 (legal_words = ceil((cells + 1) / 32) covers the pass)
-    if (lane == 0) mask[c0 >> 5] = (uint32_t)m;
-    if (lane == 1 && (c0 >> 5) + 1 < f.legal_words) mask[(c0 >> 5) + 1] = (uint32_t)(m >> 32);
+  wave_sync();
+  uint32_t empty = bits.row(bs);
+  const int rp = root_player != nullptr ? root_player[t] : 1;  // (whose stone does not matter)
+  each_move(L, a_lo, a_hi, cells, bs, [&](int j, uint32_t bit) {
+    const bool stone = (int8_t)((j & 1) == 0 ? rp : 3 - rp) != 0;
+    empty = stone ? empty & ~bit : empty | bit;
+  });
+  uint32_t ok = empty;
+  if (flags & OMQ_GO_SUICIDE)
+    ok &= empty << 1 | empty >> 1 | row_at(empty, 1) | row_at(empty, -1);
+  if (ko >= 0 && ko < cells && lane == ko / bs) ok &= ~(1u << (ko - ko / bs * bs));
+  // rows to words: row r starts at bit r * bs; then the pass
+  wave_sync();
+  bits.clear();
+  wave_sync();
+  if (lane < bs) {
+    const int o = lane * bs;
+    const uint64_t x = (uint64_t)ok << (o & 31);
+    atomicOr(&bits.words[o >> 5], (uint32_t)x);
+    if ((uint32_t)(x >> 32) != 0u) atomicOr(&bits.words[(o >> 5) + 1], (uint32_t)(x >> 32));
   }
-  legal = wave_sum_i(legal);
-  empty = wave_sum_i(empty);
+  if (lane == bs) atomicOr(&bits.words[cells >> 5], 1u << (cells & 31));
+  wave_sync();
+  uint32_t* mask = w.umask + (wb + u) * (int64_t)f.legal_words;
+  if (lane < f.legal_words) mask[lane] = bits.words[lane];
+  const int legal = wave_sum_i(__popc(ok)) + 1;
+  const int free_points = wave_sum_i(__popc(empty));
   if (lane == 0) {
-    const bool term = L > 1 && (trail >= 2 || empty == 0);
+    const bool term = L > 1 && (trail >= 2 || free_points == 0);
     w.ulegal[wb + u] = term ? 0 : legal;
     if (uterm != nullptr) uterm[wb + u] = term ? OMQ_TERM_END : OMQ_TERM_NONE;
   }
@@ -210,10 +345,10 @@ hipError_t launch_go_rules(const omq_forest& f, const omq_wave& w, const int8_t*
                            const int32_t* root_ko, int flags, int bs, int32_t* uterm,
                            hipStream_t st) {
   constexpr int wpb = 4;
-  const size_t lds = (size_t)(((bs * bs) + 15) & ~15) * wpb;
+  const size_t lds = (size_t)rule_lds_per_wave(bs * bs) * wpb;
   dim3 grid((w.max_wave + wpb - 1) / wpb, f.num_trees);
-  hipLaunchKernelGGL(go_rules_kernel, grid, dim3(wpb * kWave), lds, st, f, w, boards,
-                     root_player, root_passes, root_ko, flags, bs, uterm);
+  hipLaunchKernelGGL(go_rules_kernel, grid, dim3(wpb * kWave), lds, st, f, w, boards, root_player,
+                     root_passes, root_ko, flags, bs, uterm);
   return hipGetLastError();
 }
 
@@ -221,7 +356,7 @@ hipError_t launch_gomoku_terminal(const omq_forest& f, const omq_wave& w, const 
                                   const int32_t* root_player, int rule, int bs, int32_t* uterm,
                                   hipStream_t st) {
   constexpr int wpb = 4;
-  const size_t lds = (size_t)(((bs * bs) + 15) & ~15) * wpb;
+  const size_t lds = (size_t)rule_lds_per_wave(bs * bs) * wpb;
   dim3 grid((w.max_wave + wpb - 1) / wpb, f.num_trees);
   hipLaunchKernelGGL(gomoku_terminal_kernel, grid, dim3(wpb * kWave), lds, st, f, w, boards,
                      root_player, rule, bs, uterm);

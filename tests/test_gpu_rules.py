@@ -11,6 +11,7 @@ from omoknuni_quantum_amd.synthetic.evaluator import SyntheticEvaluator
 from omoknuni_quantum_amd.synthetic.workloads import get
 from oracle.oracle import Oracle
 from oracle.parity import compare_wave, run_parity
+from oracle.ref_np import gomoku_terminal, leaf_position
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +88,45 @@ def test_planted_overlines_parity(device, rule):
         torch.cuda.synchronize()
         compare_wave(eng, orc, w, f"planted rule {rule} wave {i}")
     assert codes[1] + codes[2] > 0
+
+
+@pytest.mark.parametrize("rule", [_lib.OMQ_RULE_FREESTYLE, _lib.OMQ_RULE_RENJU])
+@pytest.mark.parametrize("bs", [4, 5, 6, 8, 13, 19, 22])
+def test_leaf_codes_of_dense_boards(device, bs, rule):
+    """Every leaf's code against the numpy scan of its position, on boards nearly full of both
+    colours (fives and overlines in all directions, draws), with given root players, and with
+    stones of a third value (scanned cell by cell)."""
+    T, W = 16, 16
+    model = games.gomoku(bs)
+    rng = np.random.default_rng(100 * bs + rule)
+    boards = (1 + (rng.random((T, bs, bs)) < 0.35)).astype(np.int8)  # long lines of 1s
+    for t in range(T):
+        free = rng.permutation(bs * bs)[:2 + t % 3 * bs]
+        boards[t].reshape(-1)[free] = 0
+    boards[T - 2:][boards[T - 2:] == 2] = 3
+    eng = WaveEngine(model, T, 20_000, W, 100, device, SearchParams(c_puct=1.4))
+    eng.set_roots(games.root_keys(5, T), games.legal_masks(model, boards, T))
+    for players in (None, rng.integers(1, 3, T).astype(np.int32)):
+        eng.set_gomoku_rules(boards, rule, root_player=players)
+        eng.reset()
+        ev = SyntheticEvaluator(1.0)
+        codes = set()
+        for w in (1, W, W):
+            eng.run_wave(w, ev)
+            uterm = eng.uterm.view(T, W).cpu().numpy()
+            ulegal = eng.ulegal.view(T, W).cpu().numpy()
+            ufirst = eng.ufirst.view(T, W).cpu().numpy()
+            plen = eng.path_len.view(T, W).cpu().numpy()
+            paths = eng.paths.view(T, W, eng.MD).cpu().numpy()
+            action = eng.action.view(T, eng.cap).cpu().numpy()
+            for t in range(T):
+                for u in range(int(eng.ucount[t])):
+                    s = ufirst[t, u]
+                    moves = [int(action[t, n]) for n in paths[t, s, 1:plen[t, s]]]
+                    b, _, _ = leaf_position(boards[t], moves,
+                                            None if players is None else players[t])
+                    want = gomoku_terminal(b, rule == _lib.OMQ_RULE_RENJU) if moves else 0
+                    assert uterm[t, u] == want, (t, u, moves)
+                    assert want == 0 or ulegal[t, u] == 0
+                    codes.add(want)
+        assert len(codes) >= 2
