@@ -68,7 +68,6 @@ struct SelArgs {
   int max_depth_buf;
   int num_trees;
   // selection scratch (omq_wave::sel_scratch)
-  int32_t* lflag;  // [T*max_wave] 1 for the first simulation of a leaf group
   int32_t* lfs;    // [T*max_wave] first simulation of a simulation's leaf group
 };
 
@@ -1110,38 +1109,6 @@ __device__ inline int group_chain(ChainRows rows, int64_t tb, int first, int k, 
                                     cscr, progress, stop);
 }
 
-// Block-wide exclusive scan of a[0..n) in place (n <= 4 * NT); returns the total.  a may be
-// LDS or global memory (each thread touches its own chunk only).
-template <int NT>
-__device__ int block_excl_scan(int32_t* a, int n, int* s_wtot) {
-  constexpr int NW = NT / kWave;
-  const int tid = threadIdx.x;
-  const int per = (n + NT - 1) / NT;
-  const int lo = tid * per;
-  const int hi = min(lo + per, n);
-  int sum = 0;
-  for (int i = lo; i < hi; ++i) sum += a[i];
-  int wtotal;
-  const int wex = wave_excl_scan(sum, &wtotal);
-  const int wave = tid / kWave;
-  if (lane_id() == 0) s_wtot[wave] = wtotal;
-  __syncthreads();
-  int wbase = 0, total = 0;
-  for (int i = 0; i < NW; ++i) {
-    const int v = s_wtot[i];
-    if (i < wave) wbase += v;
-    total += v;
-  }
-  int run = wbase + wex;
-  for (int i = lo; i < hi; ++i) {
-    const int v = a[i];
-    a[i] = run;
-    run += v;
-  }
-  __syncthreads();
-  return total;
-}
-
 // ---- State of the level loop -----------------------------------------------------------
 // Dynamic LDS (sized for W, the simulations of the wave; a group's members occupy a segment
 // [seg, seg + m) of [0, W) at every level, so the arrays are indexed by absolute positions):
@@ -1272,7 +1239,7 @@ struct SelTraits {
 template <int RMAX, int NT>
 __device__ inline void small_groups_body(const SelArgs& f, const SelCfg& c, int t, int d, int W,
                                          int64_t tb, int64_t gmax, const LevelLds& L,
-                                         LevelShared<NT>& sh, int32_t* lfs, int32_t* lflag,
+                                         LevelShared<NT>& sh, int32_t* lfs,
                                          bool vl_done) {
   constexpr int kSmallGroup = SelTraits<RMAX>::kSmall;
   constexpr int kLaneRound = SelTraits<RMAX>::kLaneRound;
@@ -1463,7 +1430,6 @@ __device__ inline void small_groups_body(const SelArgs& f, const SelCfg& c, int 
       gsl[nxt * W + g] = (uint32_t)pos | ((uint32_t)cntc << 16);
       pos += cntc;
     }
-    if (s_end >= 0) lflag[s_end] = 1;
   }
 }
 
@@ -1472,16 +1438,16 @@ __device__ inline void small_groups_body(const SelArgs& f, const SelCfg& c, int 
 template <int RMAX, int NT>
 __device__ inline void small_groups(const SelArgs& f, const SelCfg& c, int t, int d, int W,
                                     int64_t tb, int64_t gmax, const LevelLds& L,
-                                    LevelShared<NT>& sh, int32_t* lfs, int32_t* lflag,
+                                    LevelShared<NT>& sh, int32_t* lfs,
                                     bool vl_done) {
-  small_groups_body<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, lflag, vl_done);
+  small_groups_body<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, vl_done);
 }
 template <int RMAX, int NT>
 __device__ inline void small_groups_call(const SelArgs& f, const SelCfg& c, int t, int d,
                                                int W, int64_t tb, int64_t gmax,
                                                const LevelLds& L, LevelShared<NT>& sh,
-                                               int32_t* lfs, int32_t* lflag, bool vl_done) {
-  small_groups_body<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, lflag, vl_done);
+                                               int32_t* lfs, bool vl_done) {
+  small_groups_body<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, vl_done);
 }
 
 // Single-member groups of level d in the kernels without a lane pass.  Such a group's node is
@@ -1495,7 +1461,7 @@ __device__ inline void small_groups_call(const SelArgs& f, const SelCfg& c, int 
 template <int RMAX, int NT>
 __device__ inline void leaf_pass(const SelArgs& f, const SelCfg& c, int t, int d, int W,
                                  int64_t tb, int64_t gmax, const LevelLds& L,
-                                 LevelShared<NT>& sh, int32_t* lfs, int32_t* lflag, int ns,
+                                 LevelShared<NT>& sh, int32_t* lfs, int ns,
                                  bool vl_done) {
   const SelArgs& w = f;
   const int tid = threadIdx.x;
@@ -1552,7 +1518,6 @@ __device__ inline void leaf_pass(const SelArgs& f, const SelCfg& c, int t, int d
         w.path_len[(int64_t)t * MW + s] = d + 1;
         w.leaves[(int64_t)t * MW + s] = p;
         lfs[s] = s;
-        lflag[s] = 1;
       }
     }
     const uint64_t km = __ballot(keep);
@@ -1601,7 +1566,7 @@ constexpr int kPrefixWindow = 8;
 template <int RMAX, int NT>
 __device__ inline void prefix_pass(const SelArgs& f, const SelCfg& c, int t, int d, int W,
                                    int64_t tb, int64_t gmax, const LevelLds& L,
-                                   LevelShared<NT>& sh, int32_t* lfs, int32_t* lflag, int nb,
+                                   LevelShared<NT>& sh, int32_t* lfs, int nb,
                                    bool vl_done, bool sg) {
   const SelArgs& w = f;
   const int tid = threadIdx.x;
@@ -1692,7 +1657,6 @@ __device__ inline void prefix_pass(const SelArgs& f, const SelCfg& c, int t, int
         }
         const uint16_t* mem = L.buf + cur * W + seg;
         const int s0 = mem[0];
-        if (leaf) lflag[s0] = 1;
         uint32_t rest = upos;
         for (int r = 0; r < m; ++r) {
           const int s = mem[r];
@@ -2004,11 +1968,11 @@ __device__ inline int replay_spec(const uint32_t* spec, int n, int k, uint32_t* 
 //               chain (run_ahead_chain); level 1 replays them where they cover a group
 //   root_first, root_k: the root's row (the overlap and the run-ahead)
 //   glog_ctr:   counter of the tree's group-log entries (LDS or global)
-//   lfs, lflag: the tree's per-simulation leaf records (global)
+//   lfs: the first simulation of every simulation's leaf (global)
 template <int RMAX, int NT, bool WIDE>
 __device__ int level_loop(const SelArgs& f, const SelCfg& c, int t, int d0, int dend, int W,
                           const LevelLds& L, LevelShared<NT>& sh, int* glog_ctr, int32_t* lfs,
-                          int32_t* lflag, bool pipe, int root_first, int vl_done_to,
+                          bool pipe, int root_first, int vl_done_to,
                           bool run_ahead, int root_k) {
   constexpr int NW = NT / kWave;
   using Tr = SelTraits<RMAX>;
@@ -2044,7 +2008,7 @@ __device__ int level_loop(const SelArgs& f, const SelCfg& c, int t, int d0, int 
       // single-member groups: leaves finished by all threads at once, the rest become chains
       const int ns = sh.nsmall[cur];
       if (ns > 0) {
-        leaf_pass<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, lflag, ns,
+        leaf_pass<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, ns,
                             vl_done && d == vl_done_to);
         if (!Tr::kWideLanePass && tid == 0) sh.nsmall[cur] = 0;
         __syncthreads();
@@ -2054,7 +2018,7 @@ __device__ int level_loop(const SelArgs& f, const SelCfg& c, int t, int d0, int 
     // replays the followers' picks; not for a level of at most one chain group per wave,
     // whose chains take their prefixes themselves without the pass's barriers)
     if (Tr::kPrefixPass && !replay && sh.nbig[cur] > NW)
-      prefix_pass<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, lflag, sh.nbig[cur], vl_done,
+      prefix_pass<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, sh.nbig[cur], vl_done,
                             sg);
     const int nb = sh.nbig[cur];
     // more chain groups than waves: the longest first.  The scratch is the next level's group
@@ -2144,7 +2108,6 @@ __device__ int level_loop(const SelArgs& f, const SelCfg& c, int t, int d0, int 
           lfs[s] = s0;
         }
         if (lane == 0) {
-          lflag[s0] = 1;
           atomicAdd(&sh.st[OMQ_ST_PATHENTRIES], (unsigned long long)m * (d + 1));
         }
         continue;
@@ -2295,17 +2258,14 @@ __device__ int level_loop(const SelArgs& f, const SelCfg& c, int t, int d0, int 
           }
         }
       }
-      if (fe >= 0 && lane == 0) {
-        lflag[s_end] = 1;
-        atomicOr(&w.status[0], OMQ_STATUS_NOCHILD);
-      }
+      if (fe >= 0 && lane == 0) atomicOr(&w.status[0], OMQ_STATUS_NOCHILD);
       wave_sync();
     }
     if (Tr::kLanePass)
-      small_groups<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, lflag,
+      small_groups<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs,
                              vl_done && d == vl_done_to);
     if (Tr::kWideLanePass && sh.nsmall[cur] > 0)
-      small_groups_call<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs, lflag,
+      small_groups_call<RMAX, NT>(f, c, t, d, W, tb, gmax, L, sh, lfs,
                                   vl_done && d == vl_done_to);
     __syncthreads();
     if (tid == 0) {
@@ -2349,21 +2309,40 @@ __device__ inline void start_group(const LevelLds& L, LevelShared<NT>& sh, int W
   __syncthreads();
 }
 
-// Unique leaves of tree t in order of first occurrence, from the per-simulation leaf records
-// lflag / lfs (global; lflag is scanned in place), and, with kRecords, each unique leaf's key
-// and legal count (leaf_key_count, as omq_leaf_info forms them).  Called by every thread of
-// the workgroup.
+// Unique leaves of tree t in order of first occurrence, from lfs (a simulation is its leaf's
+// first when lfs names itself), and, with kRecords, each unique leaf's key and legal count
+// (leaf_key_count, as omq_leaf_info forms them; at most one simulation per thread).  The loads
+// that need no unique id are made first, all in flight together, and the records are formed before
+// the ids: one tree, waves of 32, select 22.8 -> 22.3 us per
+// launch; 64 trees, waves of 256, 61.8 -> 60.4; 32 trees, waves of 1024, 206.0 -> 203.7.  s_uid: W ints and s_slot: 64 ints
+// of LDS.  Called by every thread of the workgroup.
 template <int NT, bool kRecords>
 __device__ inline void finish_tree(const SelArgs& w, const RecordArgs& ra, int t, int W,
-                                   int32_t* lfs, int32_t* lflag, int* s_wtot,
+                                   const int32_t* lfs, int* s_uid, int* s_slot,
                                    unsigned long long* s_uleafpath) {
+  constexpr int NW = NT / kWave;
+  // simulations per thread, a workgroup's width apart: slot c * NW + wave holds 64 of them in order
+  constexpr int kPer = kRecords ? 1 : OMQ_MAX_WAVE / NT;
+  static_assert(kPer * NW <= kWave, "one wave scans the slots");
+  static_assert(!kRecords || OMQ_SELECT_RECORDS_MAX_WAVE <= NT, "one simulation per thread");
   const int tid = threadIdx.x;
+  const int lane = lane_id();
+  const int wave = tid / kWave;
   const int MW = w.max_wave;
-  const int nu = block_excl_scan<NT>(lflag, W, s_wtot);
-  int rc = 0;
-  omq_forest fo{};
-  omq_wave wo{};
+  const int64_t wb = (int64_t)t * MW;
+  if (tid < kWave) s_slot[tid] = 0;
+  int s0[kPer], leaf[kPer];
+#pragma unroll
+  for (int c = 0; c < kPer; ++c) {
+    const int s = c * NT + tid;
+    s0[c] = s < W ? lfs[s] : -1;
+    leaf[c] = s < W ? w.leaves[wb + s] : 0;
+  }
+  uint64_t key = 0;
+  int count = 0, plen = 0;
   if constexpr (kRecords) {
+    omq_forest fo{};
+    omq_wave wo{};
     fo.capacity = w.capacity;
     fo.num_actions = ra.num_actions;
     fo.game = ra.game;
@@ -2377,28 +2356,47 @@ __device__ inline void finish_tree(const SelArgs& w, const RecordArgs& ra, int t
     wo.max_depth = w.max_depth_buf;
     wo.paths = w.paths;
     wo.path_len = w.path_len;
-    rc = fo.game != OMQ_GAME_SPARSE ? root_legal_count(fo, t) : 0;
+    const int rc = fo.game != OMQ_GAME_SPARSE ? root_legal_count(fo, t) : 0;
+    if (tid < W) plen = leaf_key_count(fo, wo, t, tid, rc, &key, &count);
   }
-  int plen_sum = 0;
-  for (int s = tid; s < W; s += NT) {
-    const int s0 = lfs[s];
-    const int uid = lflag[s0];
-    w.sim_uid[(int64_t)t * MW + s] = uid;
-    if (s0 == s) {
-      w.uleaf[(int64_t)t * MW + uid] = w.leaves[(int64_t)t * MW + s];
-      w.ufirst[(int64_t)t * MW + uid] = s;
+  __syncthreads();  // (s_slot is cleared)
+  uint64_t firsts[kPer];
+#pragma unroll
+  for (int c = 0; c < kPer; ++c) {
+    firsts[c] = __ballot(s0[c] >= 0 && s0[c] == c * NT + tid);
+    if (lane == 0) s_slot[c * NW + wave] = __popcll(firsts[c]);
+  }
+  __syncthreads();
+  int nu;
+  const int slot_ex = wave_excl_scan(s_slot[lane], &nu);
+  int mine = 0;  // path lengths of this thread's unique leaves
+#pragma unroll
+  for (int c = 0; c < kPer; ++c) {
+    const int s = c * NT + tid;
+    const int uid = readlane_i(slot_ex, c * NW + wave) +
+                    (int)__builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(firsts[c] >> 32),
+                        __builtin_amdgcn_mbcnt_lo((uint32_t)firsts[c], 0u));
+    if (s0[c] >= 0 && s0[c] == s) {
+      s_uid[s] = uid;
+      w.uleaf[wb + uid] = leaf[c];
+      w.ufirst[wb + uid] = s;
       if constexpr (kRecords) {
-        uint64_t key;
-        int count;
-        plen_sum += leaf_key_count(fo, wo, t, s, rc, &key, &count);
-        ra.ukey[(int64_t)t * MW + uid] = key;
-        ra.ulegal[(int64_t)t * MW + uid] = count;
+        ra.ukey[wb + uid] = key;
+        ra.ulegal[wb + uid] = count;
+        mine = plen;
       }
     }
   }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < kPer; ++c) {
+    const int s = c * NT + tid;
+    if (s < W) w.sim_uid[wb + s] = s_uid[min(max(s0[c], 0), W - 1)];
+  }
   if constexpr (kRecords) {
-    const int ws = wave_sum_i(plen_sum);
-    if (lane_id() == 0 && ws > 0) atomicAdd(s_uleafpath, (unsigned long long)ws);
+    const int ws = wave_sum_i(mine);
+    if (lane == 0 && ws > 0) atomicAdd(s_uleafpath, (unsigned long long)ws);
   }
   if (tid == 0) {
     w.ucount[t] = nu;
@@ -2442,17 +2440,14 @@ __global__ __launch_bounds__(NT, 1) void select_root_kernel(SelArgs f, SelCfg c,
   const int tid = threadIdx.x;
   const int64_t tb = (int64_t)t * f.capacity;
   const int MW = f.max_wave;
-  int32_t* lflag = f.lflag + (int64_t)t * MW;
   int32_t* lfs = f.lfs + (int64_t)t * MW;
   // the level overlap needs an internal root, an integer virtual loss and the ordered mode
   const int root_k = f.nchild[tb], root_first = f.first[tb];
   const bool pipe = kPipe && L.pick2 != nullptr && W > kWave && !c.vl_atomic && c.vli > 0 &&
                     c.max_depth >= 2 && root_k > 0 && root_first >= 0 &&
                     root_k <= RMAX * kWave;
-  for (int s = tid; s < W; s += NT) {
-    lflag[s] = 0;
-    if (L.pick2 != nullptr) L.pick2[s] = kPickNone;
-  }
+  if (L.pick2 != nullptr)
+    for (int s = tid; s < W; s += NT) L.pick2[s] = kPickNone;
   if (tid == 0) {
     s_glog = 0;
     // the chains keep a row's counts as floats (1 + N) advanced by the virtual loss, exact
@@ -2465,10 +2460,11 @@ __global__ __launch_bounds__(NT, 1) void select_root_kernel(SelArgs f, SelCfg c,
   // and levels below 1 (a level-1 group at the last level is a leaf)
   const bool run_ahead = NT <= 512 && L.spec != nullptr && c.vli > 0 && c.max_depth >= 3 &&
                          root_k > 0 && root_first >= 0 && root_k <= RMAX * kWave;
-  level_loop<RMAX, NT, NT <= 512>(f, c, t, 0, c.max_depth, W, L, sh, &s_glog, lfs, lflag, pipe,
+  level_loop<RMAX, NT, NT <= 512>(f, c, t, 0, c.max_depth, W, L, sh, &s_glog, lfs, pipe,
                                   root_first, pipe ? 2 : -1, run_ahead, root_k);
   __syncthreads();
-  finish_tree<NT, kRecords>(f, ra, t, W, lfs, lflag, sh.wtot, &sh.st[OMQ_ST_ULEAFPATH]);
+  finish_tree<NT, kRecords>(f, ra, t, W, lfs, reinterpret_cast<int*>(L.choice),
+                            reinterpret_cast<int*>(L.cscr_all), &sh.st[OMQ_ST_ULEAFPATH]);
   __syncthreads();
   if (tid == 0) f.gcount[t] = s_glog;
   flush_stats<NT>(f, t, sh);
@@ -2603,8 +2599,7 @@ hipError_t launch_select(const omq_forest& f, const omq_wave& w, int W, float c_
   a.max_depth_buf = w.max_depth;
   a.num_trees = f.num_trees;
   const int64_t TM = (int64_t)f.num_trees * w.max_wave;
-  a.lflag = w.sel_scratch;
-  a.lfs = w.sel_scratch + TM;
+  a.lfs = w.sel_scratch;
   RecordArgs ra;
   ra.actions = f.actions;
   ra.root_keys = f.root_keys;
