@@ -182,6 +182,8 @@ typedef struct omq_wave {
 #define OMQ_ST_ROOTCHAIN 11   /* omq_select: duration of the root's chain (the serial part of a
                                  wave's selection), in ticks of the device's constant wall clock
                                  (omq_wall_clock_khz) */
+#define OMQ_ST_TICKET 12       /* not a counter: omq_expand_backup counts a tree's finished blocks
+                               * here; 0 between calls (omq_select clears it) */
 #define OMQ_NSTATS 16
 
 /* device status bits */

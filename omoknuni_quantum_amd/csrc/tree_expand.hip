@@ -163,6 +163,32 @@ struct ExpCfg {
 
 constexpr int kPlanThreads = 1024;
 
+// First-fit of 64 leaves in lane order, k children each (0: none wanted): the node id of the
+// leaf's first child, or -1 when its children do not fit; *cur, the next free node, advances.
+// Leaf i fits when cur_i + k_i <= capacity, cur_i = cur + the children of the leaves before it
+// that fit.  Each round first drops the leaves that cannot fit even now (cur only grows, so they
+// never will), then lets every remaining leaf fit up to the first one whose running sum
+// overflows; that one is dropped by the next round.  Each round settles at least one leaf.
+__device__ inline int first_fit(int k, int64_t cap, int64_t* cur) {
+  const int lane = lane_id();
+  bool pend = k > 0;
+  int64_t at = -1;
+  for (int round = 0; round <= kWave && __ballot(pend) != 0; ++round) {
+    pend = pend && !(*cur + k > cap);
+    int tot;
+    const int ex = wave_excl_scan(pend ? k : 0, &tot);
+    const uint64_t over = __ballot(pend && *cur + ex + k > cap);
+    const int f0 = over != 0 ? lowest_lane(over) : kWave;
+    if (pend && lane < f0) {
+      at = *cur + ex;
+      pend = false;
+    }
+    // the children of the leaves that fit this round: those before f0 (all when f0 = 64)
+    *cur += f0 < kWave ? readlane_i(ex, f0) : tot;
+  }
+  return (int)at;
+}
+
 // The plan of tree t, by a workgroup of kPlanThreads threads; want is its LDS array of
 // max_wave ints.
 __device__ inline void expand_plan_block(const omq_forest& f, const omq_wave& w, const ExpCfg& c,
@@ -263,11 +289,6 @@ __device__ inline void expand_plan_block(const omq_forest& f, const omq_wave& w,
   } else if (tid < kWave) {
     // Capacity boundary: first-fit in leaf order (expand_node refuses a leaf whose children do
     // not fit; later, smaller leaves may still fit), decided by one wave, 64 leaves at a time.
-    // Leaf i fits when cur_i + k_i <= capacity, cur_i = base + the children of the leaves
-    // before it that fit.  Within a chunk each round first drops the leaves that cannot fit
-    // even now (cur only grows, so they never will), then lets every remaining leaf fit up to
-    // the first one whose running sum overflows; that one is dropped by the next round.  Each
-    // round settles at least one leaf.
     const int lane = tid;
     const int64_t cap = f.capacity;
     int64_t cur = base;
@@ -275,29 +296,14 @@ __device__ inline void expand_plan_block(const omq_forest& f, const omq_wave& w,
     for (int c0 = 0; c0 < U; c0 += kWave) {
       const int i = c0 + lane;
       const int k = i < U ? want[i] : 0;
-      bool pend = k > 0;
-      bool fits = false;
-      int64_t at = -1;  // node id of the first child, when the leaf fits
-      for (int round = 0; round <= kWave && __ballot(pend) != 0; ++round) {
-        pend = pend && !(cur + k > cap);
-        int tot;
-        const int ex = wave_excl_scan(pend ? k : 0, &tot);
-        const uint64_t over = __ballot(pend && cur + ex + k > cap);
-        const int f0 = over != 0 ? lowest_lane(over) : kWave;
-        if (pend && lane < f0) {
-          fits = true;
-          at = cur + ex;
-          pend = false;
-        }
-        // the children of the leaves that fit this round: those before f0 (all when f0 = 64)
-        cur += f0 < kWave ? readlane_i(ex, f0) : tot;
-      }
+      const int at = first_fit(k, cap, &cur);  // node id of the first child
+      const bool fits = at >= 0;
       if (i < U) {
         if (fits) {
-          w.uedge[wb + i] = (int)at - 1;
+          w.uedge[wb + i] = at - 1;
           w.unew[wb + i] = k;
           const int leaf = w.uleaf[wb + i];
-          f.first_child[tb + leaf] = (int)at - 1;
+          f.first_child[tb + leaf] = at - 1;
           f.num_children[tb + leaf] = k;
         } else {
           w.uedge[wb + i] = -1;
@@ -336,9 +342,12 @@ __global__ __launch_bounds__(kPlanThreads) void expand_plan_kernel(omq_forest f,
 
 // ---------------------------------------------------------------------------------------
 // Block bx of tree t's expansion writes (one wave per expanded leaf), with the block's
-// dynamic LDS smem.
+// dynamic LDS smem.  plan(u, &k, &first): the leaf's children and the node id of the first, from
+// the plan (called by every wave of the block with a slot u < W, after its loads are issued).
+template <class Plan>
 __device__ inline void expand_write_block(const omq_forest& f, const omq_wave& w,
-                                          const ExpCfg& c, int bx, int t, unsigned char* smem) {
+                                          const ExpCfg& c, int bx, int t, unsigned char* smem,
+                                          Plan plan) {
   const int wave = threadIdx.x / kWave;
   const int u = bx * (blockDim.x / kWave) + wave;
   const int lane = lane_id();
@@ -349,9 +358,7 @@ __device__ inline void expand_write_block(const omq_forest& f, const omq_wave& w
   // checks below, so that their latencies overlap.  (For a slot past the wave's unique leaves
   // they are stale and unused.)
   const int ucnt = w.ucount[t];
-  const int k = w.unew[wb + u];
   const int leaf = w.uleaf[wb + u];
-  const int cbase = w.uedge[wb + u] + 1;  // node id of the first child
   const int s0 = w.ufirst[wb + u];
   const uint64_t ukey = f.game == OMQ_GAME_SPARSE ? w.ukey[wb + u] : 0ull;
   const float* pol = w.policy + (wb + u) * (int64_t)f.num_actions;
@@ -362,6 +369,8 @@ __device__ inline void expand_write_block(const omq_forest& f, const omq_wave& w
     const int a = j * kWave + lane;
     prow[j] = (staged && a < f.num_actions) ? pol[a] : 0.0f;
   }
+  int k, cbase;  // children, node id of the first
+  plan(u, &k, &cbase);
   if (u >= ucnt || k <= 0) return;
   LeafLds l = carve(f, smem, wave, expand_lds_per_wave(f));
   float* spol = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(l.mask) +
@@ -526,11 +535,16 @@ __global__ void expand_write_kernel(omq_forest f, omq_wave w, ExpCfg c) {
   extern __shared__ __align__(16) unsigned char smem[];
   int bx = blockIdx.x, by = blockIdx.y;
   xcd_block(&bx, &by);  // one contiguous run of blocks (leaves of few trees) per XCD
-  expand_write_block(f, w, c, bx, by, smem);
+  const int64_t wb = (int64_t)by * w.max_wave;
+  expand_write_block(f, w, c, bx, by, smem, [&](int u, int* k, int* first) {
+    *k = w.unew[wb + u];
+    *first = w.uedge[wb + u] + 1;
+  });
 }
 
 // ---------------------------------------------------------------------------------------
-// A wave's expansion and group backup in two launches instead of four.  The expansion writes
+// A wave's expansion and group backup in two launches instead of four (in one for waves of at most
+// kFuseMaxWave simulations, below).  The expansion writes
 // the expanded leaves' row headers and their new children, the backup N and W of the path
 // nodes: no address is written by both, and neither reads what the other writes (the new
 // children lie past every path node, and the backup reads no row header).  Under the
@@ -552,10 +566,157 @@ __global__ __launch_bounds__(kPlanThreads) void plan_values_kernel(omq_forest f,
   if (s < c.W) sim_value_at(f, w, t, s, sign_mode);
 }
 
+// The plan of tree t inside each of the tree's expansion blocks (waves of at most kFuseMaxWave
+// simulations, OMQ_EXPAND_FULL): every block forms the whole plan for itself, two leaves per
+// thread, and keeps it in registers; the last of the tree's blocks to get there writes it out
+// (commit).  The plan reads what the commit changes (the row lengths of the leaves, the tree's
+// node count), so no block may commit before all have read: each takes a ticket once its reads
+// are done, and the one with the last ticket commits after its own writes.  That saves the plan's
+// launch: plan and writes, kernel trace, 4.1 + 9.0 -> 8.6 us (1 tree x 32), 4.7 + 18.3 -> 19.9 us
+// (16 x 512, Go), 4.9 + 23.7 -> 26.6 us (64 x 256).  With more leaves the plan outgrows a block's
+// two leaves per thread, and the signed leaf values run beside it anyway (plan_values_kernel).
+constexpr int kPlanPer = kFuseMaxWave / kBackupThreads;
+constexpr int kPlanBlockWaves = kBackupThreads / kWave;
+
+struct BlockPlan {
+  int leaf[kPlanPer], k[kPlanPer], at[kPlanPer];  // children wanted; first child's node, or -1
+  int U, base, total;                             // unique leaves, nodes before, children created
+  bool over;                                      // a row past OMQ_MAX_ROW was refused
+  int ticket;                                     // (thread 0)
+};
+struct PlanShared {
+  int tot[kPlanPer * kPlanBlockWaves];
+  int own_k[kPlanBlockWaves], own_at[kPlanBlockWaves];
+  int64_t cur;
+  int last;
+};
+
+// OMQ_ST_TICKET of tree t: 0 between calls (omq_select clears it, and so does the commit).
+__device__ inline unsigned long long* plan_ticket(const omq_wave& w, int t) {
+  return reinterpret_cast<unsigned long long*>(&w.stats[(int64_t)t * OMQ_NSTATS + OMQ_ST_TICKET]);
+}
+
+// Called by every thread of expansion block eb; ends with a barrier.
+__device__ inline BlockPlan plan_block(const omq_forest& f, const omq_wave& w, int eb, int t,
+                                       PlanShared& sh) {
+  const int tid = threadIdx.x;
+  const int lane = lane_id();
+  const int wave = tid / kWave;
+  const int64_t tb = (int64_t)t * f.capacity;
+  const int64_t wb = (int64_t)t * w.max_wave;
+  BlockPlan p;
+  p.U = w.ucount[t];
+  p.base = f.num_nodes[t];
+  p.over = false;
+  int legal[kPlanPer], upto[kPlanPer];
+#pragma unroll
+  for (int j = 0; j < kPlanPer; ++j) {
+    const int u = j * kBackupThreads + tid;
+    p.leaf[j] = u < w.max_wave ? w.uleaf[wb + u] : 0;
+    legal[j] = u < w.max_wave ? w.ulegal[wb + u] : 0;
+  }
+#pragma unroll
+  for (int j = 0; j < kPlanPer; ++j) {
+    const int u = j * kBackupThreads + tid;
+    int k = 0;
+    if (u < p.U && u < w.max_wave && f.num_children[tb + p.leaf[j]] == 0) k = max(legal[j], 0);
+    if (k > OMQ_MAX_ROW) {  // a selection row must fit the register tile
+      p.over = true;
+      k = 0;
+    }
+    p.k[j] = k;
+    upto[j] = wave_incl_scan(k);
+    if (lane == kWave - 1) sh.tot[j * kPlanBlockWaves + wave] = upto[j];
+  }
+  __syncthreads();
+  int total;
+  const int before =
+      wave_excl_scan(lane < kPlanPer * kPlanBlockWaves ? sh.tot[lane] : 0, &total);
+  if ((int64_t)p.base + total <= (int64_t)f.capacity) {
+    p.total = total;
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j) {
+      const int at = p.base + readlane_i(before, j * kPlanBlockWaves + wave) + upto[j] - p.k[j];
+      p.at[j] = p.k[j] > 0 ? at : -1;
+    }
+  } else {
+    // the capacity boundary: first-fit, 64 leaves at a time in order, a wave's turn each
+    if (tid == 0) sh.cur = p.base;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j) {
+      for (int q = 0; q < kPlanBlockWaves; ++q) {
+        if (q == wave) {
+          int64_t cur = sh.cur;
+          p.at[j] = first_fit(p.k[j], f.capacity, &cur);
+          if (lane == 0) sh.cur = cur;
+        }
+        __syncthreads();
+      }
+    }
+    p.total = (int)(sh.cur - p.base);
+  }
+  const int u0 = eb * kPlanBlockWaves;
+#pragma unroll
+  for (int j = 0; j < kPlanPer; ++j) {
+    const int q = j * kBackupThreads + tid - u0;
+    if (q >= 0 && q < kPlanBlockWaves) {
+      sh.own_k[q] = p.at[j] >= 0 ? p.k[j] : 0;
+      sh.own_at[q] = p.at[j];
+    }
+  }
+  __syncthreads();
+  p.ticket = 0;
+  if (tid == 0) p.ticket = (int)atomicAdd(plan_ticket(w, t), 1ull);
+  return p;
+}
+
+// Writes the plan out if this block has the last of the tree's `blocks` tickets: the leaves' row
+// headers, the plan's records, the node count and the counters.  Called by every thread.
+__device__ inline void commit_plan(const omq_forest& f, const omq_wave& w, int t, int blocks,
+                                   const BlockPlan& p, PlanShared& sh) {
+  const int tid = threadIdx.x;
+  const int64_t tb = (int64_t)t * f.capacity;
+  const int64_t wb = (int64_t)t * w.max_wave;
+  if (tid == 0) sh.last = p.ticket == blocks - 1;
+  __syncthreads();
+  if (!sh.last) return;
+  int n_exp = 0, n_fail = 0;
+#pragma unroll
+  for (int j = 0; j < kPlanPer; ++j) {
+    const int u = j * kBackupThreads + tid;
+    if (u >= p.U || u >= w.max_wave) break;
+    const bool fits = p.at[j] >= 0;
+    w.uedge[wb + u] = fits ? p.at[j] - 1 : -1;
+    w.unew[wb + u] = fits ? p.k[j] : 0;
+    if (fits) {
+      f.first_child[tb + p.leaf[j]] = p.at[j] - 1;
+      f.num_children[tb + p.leaf[j]] = p.k[j];
+    }
+    n_exp += fits ? 1 : 0;
+    n_fail += p.k[j] > 0 && !fits ? 1 : 0;
+  }
+  if (p.over) atomicOr(&w.status[0], OMQ_STATUS_ROWLIMIT);
+  n_exp = wave_sum_i(n_exp);
+  n_fail = wave_sum_i(n_fail);
+  unsigned long long* st =
+      reinterpret_cast<unsigned long long*>(&w.stats[(int64_t)t * OMQ_NSTATS]);
+  if (lane_id() == 0) {
+    if (n_exp > 0) atomicAdd(&st[OMQ_ST_EXPANDED], (unsigned long long)n_exp);
+    if (n_fail > 0) atomicAdd(&st[OMQ_ST_CAPFAIL], (unsigned long long)n_fail);
+  }
+  if (tid == 0) {
+    atomicAdd(&st[OMQ_ST_NEWCHILD], (unsigned long long)p.total);
+    f.num_nodes[t] = p.base + p.total;
+    *plan_ticket(w, t) = 0;
+  }
+}
+
 // Blocks [0, nbb) of a tree: backup_groups_block; the rest: expand_write_block (kBackupThreads
 // / 64 leaves each), nbe of them.  The backup's blocks come first, so that their dependent
 // loads start with the first writes instead of after the last (C3's expansion-and-backup phase
 // 68.2 -> 63.1 us, C4's 68.0 -> 61.5 us, C2's 33.6 -> 31.6 us against the writes first).
+// FUSED: the signed leaf values are formed by the backup, and the plan by the expansion's blocks.
 template <bool FUSED>
 __global__ __launch_bounds__(kBackupThreads) void write_backup_kernel(omq_forest f, omq_wave w,
                                                                       ExpCfg c, int sign_mode,
@@ -563,10 +724,24 @@ __global__ __launch_bounds__(kBackupThreads) void write_backup_kernel(omq_forest
   extern __shared__ __align__(16) unsigned char smem[];
   int bx = blockIdx.x, by = blockIdx.y;
   xcd_block(&bx, &by);  // one contiguous run of blocks (leaves of few trees) per XCD
-  if (bx < nbb)
+  if (bx < nbb) {
     backup_groups_block<FUSED>(f, w, c.vli, sign_mode, bx, by, nbb);
-  else
-    expand_write_block(f, w, c, bx - nbb, by, smem);
+  } else if constexpr (FUSED) {
+    __shared__ PlanShared sh;
+    const BlockPlan p = plan_block(f, w, bx - nbb, by, sh);
+    const int wave = threadIdx.x / kWave;
+    expand_write_block(f, w, c, bx - nbb, by, smem, [&](int, int* k, int* first) {
+      *k = sh.own_k[wave];
+      *first = sh.own_at[wave];
+    });
+    commit_plan(f, w, by, nbe, p, sh);
+  } else {
+    const int64_t wb = (int64_t)by * w.max_wave;
+    expand_write_block(f, w, c, bx - nbb, by, smem, [&](int u, int* k, int* first) {
+      *k = w.unew[wb + u];
+      *first = w.uedge[wb + u] + 1;
+    });
+  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -628,13 +803,16 @@ hipError_t launch_expand_backup(const omq_forest& f, const omq_wave& w, int W,
   c.policy = OMQ_EXPAND_FULL;
   c.noise = noise;
   c.eps = eps;
-  // the signed leaf values: formed by the group backup itself for the waves it fuses them in
+  // waves of at most kFuseMaxWave: one launch, the signed leaf values formed by the group backup
+  // and the plan by the expansion's blocks; larger ones: the plan and the values first
   const bool fused_values = W <= kFuseMaxWave;
-  const int nvb = fused_values ? 0 : (W + kPlanThreads - 1) / kPlanThreads;
-  hipLaunchKernelGGL(plan_values_kernel, dim3(1 + nvb, f.num_trees), dim3(kPlanThreads),
-                     (size_t)w.max_wave * sizeof(int), st, f, w, c, sign_mode);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (!fused_values) {
+    const int nvb = (W + kPlanThreads - 1) / kPlanThreads;
+    hipLaunchKernelGGL(plan_values_kernel, dim3(1 + nvb, f.num_trees), dim3(kPlanThreads),
+                       (size_t)w.max_wave * sizeof(int), st, f, w, c, sign_mode);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   constexpr int wpb = kBackupThreads / kWave;
   const size_t lds = expand_lds_per_wave(f) * wpb;
   const int nbe = (W + wpb - 1) / wpb;

@@ -310,3 +310,42 @@ def test_expand_backup_equals_expand_then_backup(device, name, kw):
         x, y = getattr(a, name_), getattr(b, name_)
         assert torch.equal(x.view(torch.int32) if x.dtype == torch.float32 else x,
                            y.view(torch.int32) if y.dtype == torch.float32 else y), name_
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,W,capacity", [
+    ("C2", 1, 100_000), ("C2", 5, 3_000), ("C2", 64, 9_000), ("C2", 257, 100_000),
+    ("C2", 512, 30_000), ("C4", 512, 2_500), ("C4", 300, 20_000)])
+def test_plan_of_one_launch_waves(device, name, W, capacity):
+    """Waves of at most 512 simulations, whose expansion blocks form the plan themselves, against
+    omq_expand's plan: the plan's records, node counts and counters after every wave, with trees
+    that fill up (leaves refused, later ones taken), and the blocks' counter back at 0."""
+    wl = get(name).scaled(name=f"{name}-plan", num_trees=3, wave_size=W, capacity=capacity)
+    params = SearchParams(c_puct=wl.c_puct, virtual_loss=wl.virtual_loss, max_depth=4)
+    engs = [WaveEngine(wl.model, 3, capacity, W, 100, device, params) for _ in range(2)]
+    ev = SyntheticEvaluator(wl.logit_scale)
+    for e in engs:
+        e.set_roots(*wl.root_inputs())
+        e.reset()
+    a, b = engs
+    a.stats.fill_(7)  # (omq_select clears the blocks' counter itself)
+    b.stats.fill_(7)
+    for i, w in enumerate([1] + [W] * 12):
+        a.run_wave(w, ev)
+        b.select(w)
+        ev.evaluate_wave(b)
+        b.expand(w)
+        b.backup(w)
+        torch.cuda.synchronize()
+        assert torch.equal(a.num_nodes, b.num_nodes), i
+        for t in range(3):
+            u = t * W + torch.arange(int(a.ucount[t]), device=device)
+            assert torch.equal(a.uedge[u], b.uedge[u]) and torch.equal(a.unew[u], b.unew[u]), i
+        sa, sb = a.stats.view(3, -1), b.stats.view(3, -1)
+        for col in (5, 6, 9):  # leaves expanded, children created, expansions refused
+            assert torch.equal(sa[:, col], sb[:, col]), (i, col)
+        assert not sa[:, 12].any()
+        assert torch.equal(a.nchild, b.nchild) and torch.equal(a.first, b.first)
+        assert torch.equal(a.P.view(torch.int32), b.P.view(torch.int32)), i
+    if capacity < 25_000 and W > 1:
+        assert (sa[:, 9] > 7).all()  # the trees did fill up
