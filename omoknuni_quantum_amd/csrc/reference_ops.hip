@@ -203,6 +203,12 @@ expansion_compact_kernel(int32_t* nodes, int wave_size, int32_t* count) {
 }
 
 // ---- batched_ucb_selection ---------------------------------------------------------------
+// A row to a wave.  A row's time is its three dependent loads (bounds, edge, child's values), so
+// each lane has kUcbAhead positions in flight at a time: with 4, a row of up to 256 children is
+// one trip.  8192 rows of 112-225 children: the call 7.7 -> 6.7 us (the kernel 5.9; two ahead
+// 6.1, six 5.9).
+constexpr int kUcbAhead = 4;
+
 __global__ void batched_ucb_kernel(const float* q_values, const int32_t* visit_counts,
                                    int num_children, const int32_t* parent_visits,
                                    const float* priors, const int32_t* row_ptr,
@@ -224,16 +230,32 @@ __global__ void batched_ucb_kernel(const float* q_values, const int32_t* visit_c
   float best = -1e10f;
   int best_pos = 0x7FFFFFFF;
   const int hi = min(end, num_children);
-  for (int i = start + lane; i < hi; i += kWave) {
-    const int c = col_indices[i];
-    if (c < 0 || c >= num_children) continue;
-    const float n = (float)visit_counts[c];
-    const float q = n > 0.0f ? q_values[c] : 0.0f;
-    const float exploration = c_puct * priors[i] * sqrt_parent / (1.0f + n);
-    const float ucb = q + exploration;
-    if (ucb > best) {
-      best = ucb;
-      best_pos = i - start;
+  for (int64_t i0 = start + lane; i0 < hi; i0 += kUcbAhead * kWave) {
+    int c[kUcbAhead];
+    float pr[kUcbAhead], q[kUcbAhead];
+    int nv[kUcbAhead];
+#pragma unroll
+    for (int j = 0; j < kUcbAhead; ++j) {
+      const int64_t i = i0 + j * kWave;
+      c[j] = i < hi ? col_indices[i] : -1;
+      pr[j] = i < hi ? priors[i] : 0.0f;
+      if (c[j] >= num_children) c[j] = -1;
+    }
+#pragma unroll
+    for (int j = 0; j < kUcbAhead; ++j) {
+      nv[j] = c[j] >= 0 ? visit_counts[c[j]] : 0;
+      q[j] = c[j] >= 0 ? q_values[c[j]] : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < kUcbAhead; ++j) {
+      if (c[j] < 0) continue;
+      const float n = (float)nv[j];
+      const float exploration = c_puct * pr[j] * sqrt_parent / (1.0f + n);
+      const float ucb = (n > 0.0f ? q[j] : 0.0f) + exploration;
+      if (ucb > best) {
+        best = ucb;
+        best_pos = (int)(i0 + j * kWave - start);
+      }
     }
   }
   const uint32_t key = best_pos != 0x7FFFFFFF ? fkey(best + 0.0f) : 0u;

@@ -103,6 +103,25 @@ def test_batched_ucb_selection(device, seed):
     assert (bad.cpu() == -1).all()
 
 
+@pytest.mark.parametrize("width", [255, 256, 257, 512, 513, 1100])
+def test_batched_ucb_wide_rows(device, width):
+    """Rows around the positions a wave has in flight at a time, with ties and skipped edges."""
+    rng = np.random.default_rng(width)
+    B = 9
+    nc = B * width - 3                            # the last row runs past the children
+    row_ptr = (np.arange(B + 1) * width).astype(np.int32)
+    col = rng.integers(-1, nc + 2, nc).astype(np.int32)
+    visits = rng.integers(0, 3, nc).astype(np.int32)
+    q = (np.round(rng.random(nc) * 4) / 4).astype(F)
+    priors = (np.round(rng.random(nc) * 4) / 4).astype(F)
+    pv = rng.integers(0, 50, B).astype(np.int32)
+    args = (q, visits, pv, priors, row_ptr, col)
+    sel_np, _ = ref_np.batched_ucb_selection(*args, 1.4)
+    print(f"batched_ucb_wide_rows width={width}", flush=True)
+    got = torch_ops.batched_ucb_selection(*(_t(a, device) for a in args), 1.4)
+    assert np.array_equal(got.cpu().numpy(), sel_np)
+
+
 @pytest.mark.parametrize("mc", [4, 64, 150, 700])
 def test_fused_select_expand(device, mc):
     rng = np.random.default_rng(7 + mc)
