@@ -383,7 +383,8 @@ hipError_t launch_gomoku_terminal(const omq_forest& f, const omq_wave& w, const 
 // stores and the planes found per value: 16384 slots float32 NCHW 99.7 -> 65.5 us (4.3 TB/s; a
 // fill of the same buffers takes 42 us), bfloat16 NHWC 71.0 -> 36.2 us; 8192 slots 53.5 -> 35.2 and
 // 34.6 -> 16.6 us; 2048 slots (four waves) 16.0 -> 10.6 and 12.7 -> 10.4 us, where the launch bounds
-// both.  One wave per slot from 4096 slots (16 per CU): 512 slots took 18 us with it, 11 with four.
+// both.  With one wave per slot each XCD writes one run of slots (the first of these 65.0 -> 63.3
+// us; all slots zero, without the chains, 51).  One wave per slot from 4096 slots (16 per CU): 512 slots took 18 us with it, 11 with four.
 constexpr int kFeatOneWaveSlots = 4096;
 
 template <typename OutT>
@@ -417,8 +418,8 @@ __global__ __launch_bounds__(NW * kWave) void leaf_features_kernel(
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_pos[2];  // player to move at the leaf, move count
   const int cells = bs * bs;
-  const int t = blockIdx.y;
-  const int u = blockIdx.x;
+  int t = blockIdx.y, u = blockIdx.x;
+  if (NW == 1) xcd_block(&u, &t);
   const int tid = threadIdx.x;
   const int per = PLANES * cells;
   OutT* o = out + ((int64_t)t * w.max_wave + u) * per;
