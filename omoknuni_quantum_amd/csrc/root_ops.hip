@@ -280,16 +280,18 @@ __global__ __launch_bounds__(kWave) void sample_actions_kernel(omq_forest f, con
 
 // ---- root Dirichlet noise -------------------------------------------------------------------
 // Entry i of row t is the noise of the i-th legal root action (the layout omq_expand reads).
-// The row's legal count L is the root's legal mask popcount (board models) or its sparse-model
-// count (at most OMQ_MAX_ROW either way).  One workgroup per tree, one gamma variate per thread
-// (about 4 us each, a serial rejection loop in doubles: one wave per tree took them six in a row
-// on 362 actions, 24 us against 10 so), then the canonical wave sum by every wave and the division.
+// The row's legal count L is the root's legal mask popcount (board models; at most OMQ_MAX_ROW
+// cells, and the pass of a Go root) or its sparse-model count.  One workgroup per tree, one gamma
+// variate per thread (about 4 us each, a serial rejection loop in doubles: one wave per tree took
+// them six in a row on 362 actions, 24 us against 10 so), then the canonical wave sum by every wave
+// and the division.
 constexpr int kNoiseThreads = OMQ_MAX_ROW;
+constexpr int kNoiseMax = OMQ_MAX_ROW + 1;
 __global__ __launch_bounds__(kNoiseThreads) void root_dirichlet_kernel(omq_forest f, double alpha,
                                                                        uint64_t seed,
                                                                        uint64_t counter,
                                                                        double* noise) {
-  __shared__ double s_g[OMQ_MAX_ROW];
+  __shared__ double s_g[kNoiseMax];
   const int t = blockIdx.x;
   const int tid = threadIdx.x;
   const int lane = lane_id();
@@ -304,13 +306,13 @@ __global__ __launch_bounds__(kNoiseThreads) void root_dirichlet_kernel(omq_fores
       c += __popc(f.root_legal[(int64_t)t * f.legal_words + i]);
     L = wave_sum_i(c);
   }
-  for (int i = tid; i < L && i < OMQ_MAX_ROW; i += kNoiseThreads) {
+  for (int i = tid; i < L && i < kNoiseMax; i += kNoiseThreads) {
     Stream st = make_stream(seed, counter, t, i);
     s_g[i] = gamma_mt(alpha, st);
   }
   __syncthreads();
   double part = 0.0;
-  for (int i = lane; i < L && i < OMQ_MAX_ROW; i += kWave) part = part + s_g[i];
+  for (int i = lane; i < L && i < kNoiseMax; i += kWave) part = part + s_g[i];
   const double S = wave_sum_canonical_d(part);
   for (int i = tid; i < A; i += kNoiseThreads) {
     if (i < L) row[i] = S > 0.0 ? s_g[i] / S : 1.0 / (double)L;

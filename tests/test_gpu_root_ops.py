@@ -107,6 +107,21 @@ def test_root_ops_wide_boards(device, kind, bs):
         assert np.array_equal(got[t], orc.root_dirichlet(t, 0.03, 31, 4)), t
 
 
+def test_device_dirichlet_of_the_widest_root(device):
+    """513 legal actions, one more than a row holds children: a Go root's pass."""
+    wl = get("C3").scaled(model=games.GameModel("go", 513, 22), num_trees=2, capacity=1000)
+    eng, orc, _ = make_pair(wl, device=device)
+    legal = np.zeros((2, eng.model.legal_words), np.uint32)
+    legal[:, :16], legal[:, 16] = 0xFFFFFFFF, 1
+    keys = wl.root_inputs()[0]
+    eng.set_roots(keys, legal)
+    orc.set_roots(keys, legal, None)
+    eng.device_root_noise(0.3, 9, 1)
+    got = eng.noise.view(2, 513).cpu().numpy()
+    for t in range(2):
+        assert np.array_equal(got[t], orc.root_dirichlet(t, 0.3, 9, 1)), t
+
+
 @pytest.mark.parametrize("name", ["C1", "C3", "C4"])
 def test_root_children(device, name):
     """The root's child for an action and its visits: rows of 20-45, 225 and up to 362 children,
