@@ -345,7 +345,7 @@ __device__ inline void bfs_row(const int32_t* row_ptr, int num_edges, int node, 
 // about a fifth of the search for it).
 __global__ void bfs_clear_kernel(int root, int max_nodes, uint8_t* in_subtree, int32_t* remap,
                                  int32_t* claim, int32_t* queue) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < max_nodes;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < max_nodes;
        i += gridDim.x * blockDim.x) {
     in_subtree[i] = i == root ? 1 : 0;
     remap[i] = i == root ? 0 : -1;
@@ -373,8 +373,9 @@ __device__ inline int64_t bfs_block_scan2(int64_t v, int n, int64_t* s_wtot, int
 // the subtree claims its child with its place (the earliest wins), and is kept in the queue past
 // the level, where the winners are then numbered in order and compacted in place, kBfsNumber
 // candidates per thread and scan.  100k of 300k nodes: 208 us with one candidate per thread,
-// its row found by a binary search in memory, twice, and the clearing in this workgroup; 79 us so.  A level of more candidates than the queue has
-// room for (rows that overlap, repeated children) finds its candidates again for the numbering.
+// its row found by a binary search in memory, twice, and the clearing in this workgroup; 79 us
+// so.  A level of more candidates than the queue has room for (rows that overlap, repeated
+// children) finds its candidates again for the numbering.
 // Workspace: queue [max_nodes], claim [max_nodes].
 constexpr int kBfsPer = 4;
 constexpr int kBfsChunk = kBfsThreads * kBfsPer;
