@@ -204,9 +204,10 @@ class WaveEngine:
         self.rule = int(rule)
 
     def _reuse(self, name: str, x: torch.Tensor) -> torch.Tensor:
-        """x as the rule input `name`: on the device, in the present one's storage (copied by _copy_pending)
-        when that has its size and type: root inputs keep their addresses from one position to the next, so that a recorded search (whose
-        kernels hold those addresses) stays valid."""
+        """x as the rule input `name`: on the device, in the present one's storage (copied by
+        _copy_pending) when that has its size and type: root inputs keep their addresses from
+        one position to the next, so that a recorded search (whose kernels hold those addresses)
+        stays valid."""
         cur = getattr(self, name)
         if cur is not None and cur.numel() == x.numel() and cur.dtype == x.dtype:
             self._pending[name] = (cur, x.numpy())

@@ -384,7 +384,8 @@ hipError_t launch_gomoku_terminal(const omq_forest& f, const omq_wave& w, const 
 // fill of the same buffers takes 42 us), bfloat16 NHWC 71.0 -> 36.2 us; 8192 slots 53.5 -> 35.2 and
 // 34.6 -> 16.6 us; 2048 slots (four waves) 16.0 -> 10.6 and 12.7 -> 10.4 us, where the launch bounds
 // both.  With one wave per slot each XCD writes one run of slots (the first of these 65.0 -> 63.3
-// us; all slots zero, without the chains, 51).  One wave per slot from 4096 slots (16 per CU): 512 slots took 18 us with it, 11 with four.
+// us; all slots zero, without the chains, 51).  One wave per slot from 4096 slots (16 per CU): 512
+// slots took 18 us with it, 11 with four.
 constexpr int kFeatOneWaveSlots = 4096;
 
 template <typename OutT>

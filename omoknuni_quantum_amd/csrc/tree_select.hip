@@ -2313,9 +2313,9 @@ __device__ inline void start_group(const LevelLds& L, LevelShared<NT>& sh, int W
 // first when lfs names itself), and, with kRecords, each unique leaf's key and legal count
 // (leaf_key_count, as omq_leaf_info forms them; at most one simulation per thread).  The loads
 // that need no unique id are made first, all in flight together, and the records are formed before
-// the ids: one tree, waves of 32, select 22.8 -> 22.3 us per
-// launch; 64 trees, waves of 256, 61.8 -> 60.4; 32 trees, waves of 1024, 206.0 -> 203.7.  s_uid: W ints and s_slot: 64 ints
-// of LDS.  Called by every thread of the workgroup.
+// the ids: one tree, waves of 32, select 22.8 -> 22.3 us per launch; 64 trees, waves of 256,
+// 61.8 -> 60.4; 32 trees, waves of 1024, 206.0 -> 203.7.  s_uid: W ints and s_slot: 64 ints of LDS.
+// Called by every thread of the workgroup.
 template <int NT, bool kRecords>
 __device__ inline void finish_tree(const SelArgs& w, const RecordArgs& ra, int t, int W,
                                    const int32_t* lfs, int* s_uid, int* s_slot,
