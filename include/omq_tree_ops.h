@@ -146,8 +146,10 @@ typedef struct omq_wave {
   int32_t* unew;            /* [T*max_wave] number of children created */
   float* policy;            /* [T*max_wave*num_actions] evaluator policy rows of the unique leaves */
   float* values;            /* [T*max_wave] evaluator values of the unique leaves */
-  float* sim_value;         /* [T*max_wave] backup scratch: signed leaf value of every simulation
-                               (written in atomic mode and for waves of more than 512) */
+  float* sim_value;         /* [T*max_wave] backup scratch (no contents to keep between calls):
+                               signed leaf value of every simulation, written in atomic mode and
+                               for waves of more than 512; in smaller waves omq_expand_backup
+                               counts a tree's finished blocks in the first word of its row */
   int64_t* stats;           /* [T*OMQ_NSTATS] accumulated operation counters */
   int32_t* status;          /* [4] device-side error flags (bit set, never cleared by the library) */
   int32_t* sel_scratch;     /* [OMQ_SEL_SCRATCH_INTS(T, max_wave)] omq_select's scratch: per-
@@ -182,8 +184,7 @@ typedef struct omq_wave {
 #define OMQ_ST_ROOTCHAIN 11   /* omq_select: duration of the root's chain (the serial part of a
                                  wave's selection), in ticks of the device's constant wall clock
                                  (omq_wall_clock_khz) */
-#define OMQ_ST_TICKET 12       /* not a counter: omq_expand_backup counts a tree's finished blocks
-                               * here; 0 between calls (omq_select clears it) */
+#define OMQ_ST_RESERVED 12     /* not a counter: omq_select sets it to 0 */
 #define OMQ_NSTATS 16
 
 /* device status bits */
@@ -275,10 +276,14 @@ int omq_backup(const omq_forest* f, const omq_wave* w, int32_t wave_size, float 
 
 /* omq_expand followed by omq_backup, with the same arguments, and the same results: the two
  * write no common address and neither reads what the other writes, so their kernels run side
- * by side, in two launches instead of four (the expansion plan beside the signed leaf values,
- * then the child records beside the group backup).  Under OMQ_EXPAND_REFERENCE_PW (whose rule
- * reads the root's count, which the backup changes), with OMQ_WACC_ATOMIC, or where the
- * expansion's LDS per leaf exceeds 16 KiB, it runs the two one after the other.
+ * by side: waves of more than 512 simulations in two launches instead of four (the expansion plan
+ * beside the signed leaf values, then the child records beside the group backup), smaller ones in
+ * one (each of a tree's expansion blocks forms the plan, and the last to have read what it needs
+ * writes it out).  wave_size is the size of the omq_select before (no tree has more unique leaves
+ * than that).  Nothing need be set up for it: stats and sim_value may hold anything.  Under
+ * OMQ_EXPAND_REFERENCE_PW (whose rule reads the root's count, which the backup changes), with
+ * OMQ_WACC_ATOMIC, or where the expansion's LDS per leaf exceeds 16 KiB, it runs the two one after
+ * the other.
  * Replaces the expansion and the backup of OptimizedCPUWaveSearch._batch_expand_and_backup
  * (python/mcts/cpu/optimized_wave_search.py:367-483), run back to back. */
 int omq_expand_backup(const omq_forest* f, const omq_wave* w, int32_t wave_size,

@@ -591,9 +591,33 @@ struct PlanShared {
   int last;
 };
 
-// OMQ_ST_TICKET of tree t: 0 between calls (omq_select clears it, and so does the commit).
-__device__ inline unsigned long long* plan_ticket(const omq_wave& w, int t) {
-  return reinterpret_cast<unsigned long long*>(&w.stats[(int64_t)t * OMQ_NSTATS + OMQ_ST_TICKET]);
+// The tickets of tree t are counted in the first word of its sim_value row, which the one-launch
+// waves use for nothing else, as kTicketTag | tickets taken.  The row is scratch, so a call may find
+// anything there (a larger wave's values, say): a block that finds no tag has taken no ticket, sees
+// to it that the word is kTicketTag, by its own exchange or another block's, and takes one then.
+// Every block so adds to a tagged word exactly once, whichever comes first, and waits for none (a
+// failed exchange means that another block has changed the word, at most twice each).  The commit
+// leaves kTicketTag, so that the usual call takes one atomic.  As a float the tagged word is a
+// signalling NaN, and so are the words about it: no leaf value, which is finite or a quiet NaN, is
+// taken for one.
+constexpr uint32_t kTicketTag = 0xFFA5C300u;
+constexpr uint32_t kTicketCount = 0xFFu;
+static_assert(kFuseMaxWave / kPlanBlockWaves <= (int)kTicketCount, "a tree's blocks are counted");
+
+__device__ inline uint32_t* plan_ticket(const omq_wave& w, int t) {
+  return reinterpret_cast<uint32_t*>(&w.sim_value[(int64_t)t * w.max_wave]);
+}
+__device__ inline int take_ticket(uint32_t* word) {
+  auto tagged = [](uint32_t x) { return (x & ~kTicketCount) == kTicketTag; };
+  const uint32_t got = atomicAdd(word, 1u);
+  if (tagged(got)) return (int)(got & kTicketCount);
+  uint32_t at = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  while (!tagged(at)) {
+    const uint32_t was = atomicCAS(word, at, kTicketTag);
+    if (was == at) break;
+    at = was;
+  }
+  return (int)(atomicAdd(word, 1u) & kTicketCount);
 }
 
 // Called by every thread of expansion block eb; ends with a barrier.
@@ -667,7 +691,7 @@ __device__ inline BlockPlan plan_block(const omq_forest& f, const omq_wave& w, i
   }
   __syncthreads();
   p.ticket = 0;
-  if (tid == 0) p.ticket = (int)atomicAdd(plan_ticket(w, t), 1ull);
+  if (tid == 0) p.ticket = take_ticket(plan_ticket(w, t));
   return p;
 }
 
@@ -708,7 +732,7 @@ __device__ inline void commit_plan(const omq_forest& f, const omq_wave& w, int t
   if (tid == 0) {
     atomicAdd(&st[OMQ_ST_NEWCHILD], (unsigned long long)p.total);
     f.num_nodes[t] = p.base + p.total;
-    *plan_ticket(w, t) = 0;
+    *plan_ticket(w, t) = kTicketTag;
   }
 }
 

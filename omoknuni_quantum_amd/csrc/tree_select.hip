@@ -2450,7 +2450,7 @@ __global__ __launch_bounds__(NT, 1) void select_root_kernel(SelArgs f, SelCfg c,
     for (int s = tid; s < W; s += NT) L.pick2[s] = kPickNone;
   if (tid == 0) {
     s_glog = 0;
-    f.stats[(int64_t)t * OMQ_NSTATS + OMQ_ST_TICKET] = 0;  // (for this wave's expansion)
+    f.stats[(int64_t)t * OMQ_NSTATS + OMQ_ST_RESERVED] = 0;
     // the chains keep a row's counts as floats (1 + N) advanced by the virtual loss, exact
     // while below 2^24; every node's count is at most its root's
     if ((int64_t)f.N[tb] + 1 + (int64_t)c.vli * W >= (int64_t)(1 << 24))

@@ -349,3 +349,37 @@ def test_plan_of_one_launch_waves(device, name, W, capacity):
         assert torch.equal(a.P.view(torch.int32), b.P.view(torch.int32)), i
     if capacity < 25_000 and W > 1:
         assert (sa[:, 9] > 7).all()  # the trees did fill up
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W", [1, 8, 512])
+@pytest.mark.parametrize("word", [0, 1, 3, 0x7F, -1, 0x3F800000, 0x7FC00000, "values"])
+def test_one_launch_plan_from_any_scratch(device, W, word):
+    """omq_expand_backup of small waves with arbitrary words in stats and sim_value when it is
+    called (small counts, floats, a quiet NaN, the values of an earlier atomic backup) against
+    omq_expand and omq_backup."""
+    wl = get("C2").scaled(name="C2-scratch", num_trees=3, wave_size=W, capacity=60_000)
+    params = SearchParams(c_puct=wl.c_puct, virtual_loss=wl.virtual_loss, max_depth=4)
+    a, b = [WaveEngine(wl.model, 3, wl.capacity, W, 100, device, params) for _ in range(2)]
+    ev = SyntheticEvaluator(wl.logit_scale)
+    for e in (a, b):
+        e.set_roots(*wl.root_inputs())
+        e.reset()
+    for i, w in enumerate([1] + [W] * 4):
+        for e in (a, b):
+            e.select(w)
+            ev.evaluate_wave(e)
+        if word == "values":
+            a.sim_value.copy_(a.values)
+        else:
+            a.sim_value.view(torch.int32).fill_(word)
+        a.stats.fill_(5 if word == "values" else word)
+        a.expand_backup(w)
+        b.expand(w)
+        b.backup(w)
+        torch.cuda.synchronize()
+        for name in ("num_nodes", "N", "nchild", "first", "action", "parent"):
+            assert torch.equal(getattr(a, name), getattr(b, name)), (i, name)
+        for name in ("W", "P"):
+            x, y = getattr(a, name), getattr(b, name)
+            assert torch.equal(x.view(torch.int32), y.view(torch.int32)), (i, name)
