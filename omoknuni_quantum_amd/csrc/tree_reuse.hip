@@ -394,11 +394,11 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
   int start = 0, end = 1;  // the current level: queue[start, end)
   // The rows of level nodes [c0, c0 + kBfsChunk) into s_cex / s_cof; returns their number of
   // edges, *nz the rows with any.  Ends with a barrier.
-  auto load_chunk = [&](int c0, int* nz) -> int64_t {
+  auto load_chunk = [&](int64_t c0, int* nz) -> int64_t {
     int of[kBfsPer], len[kBfsPer];
     int64_t mine = 0;
     int nzm = 0;
-    const int i0 = start + c0 + tid * kBfsPer;
+    const int64_t i0 = start + c0 + tid * kBfsPer;  // (64 bits: up to a chunk past max_nodes)
     int node[kBfsPer];
 #pragma unroll
     for (int e = 0; e < kBfsPer; ++e) node[e] = i0 + e < end ? queue[i0 + e] : -1;
@@ -454,7 +454,7 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
     const int L = end - start;
     int64_t run = 0;
     bool stash = true;  // the level's candidates so far are in queue[end, end + run)
-    for (int c0 = 0; c0 < L; c0 += kBfsChunk) {
+    for (int64_t c0 = 0; c0 < L; c0 += kBfsChunk) {
       int nz;
       const int64_t tot = load_chunk(c0, &nz);
       if (run + tot > 0x7FFFFFFF) {  // more candidates than int32 keys (rows that overlap)
@@ -510,7 +510,7 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
       }
     } else {
       run = 0;
-      for (int c0 = 0; c0 < L; c0 += kBfsChunk) {
+      for (int64_t c0 = 0; c0 < L; c0 += kBfsChunk) {
         int nz;
         const int tot = (int)load_chunk(c0, &nz);
         for (int64_t k0 = 0; k0 < tot; k0 += kBfsThreads) {
@@ -659,7 +659,7 @@ hipError_t launch_bfs_subtree(const int32_t* row_ptr, const int32_t* col, int nu
                               int32_t* count, int32_t* ws, hipStream_t st) {
   int32_t* queue = ws;
   int32_t* claim = ws + max_nodes;
-  const int blocks = std::min(1024, (max_nodes + 255) / 256);
+  const int blocks = (int)std::min<int64_t>(1024, ((int64_t)max_nodes + 255) / 256);
   hipLaunchKernelGGL(bfs_clear_kernel, dim3(blocks), dim3(256), 0, st, root, max_nodes,
                      in_subtree, remap, claim, queue);
   hipError_t e = hipGetLastError();

@@ -274,3 +274,21 @@ def test_subtree_wide_levels(device, repeat):
     rows = [r + (r[::-1] if repeat else []) for r in rows]
     _check_subtree(device, rows, 0, n)
     _check_subtree(device, rows, int(np.argmax([len(r) for r in rows[1:41]])) + 1, n)
+
+
+def test_subtree_of_the_largest_node_count(device):
+    """max_nodes = 2^31 - 1 (the most an int32 holds): the subtree of the last node, with children
+    at both ends."""
+    n = 2**31 - 1
+    if torch.cuda.mem_get_info()[0] < 80 * 2**30:
+        pytest.skip("needs 42 GiB of device memory for the graph and the workspace")
+    ptr = torch.zeros(n + 1, dtype=torch.int32, device=device)
+    ptr[n] = 3
+    col = _t(np.array([5, n - 2, 5], np.int32), device)
+    ins, remap, cnt = torch_ops.parallel_bfs_subtree(ptr, col, n - 1, n)
+    assert int(_np(cnt)[0]) == 3
+    assert [int(remap[i]) for i in (n - 1, 5, n - 2)] == [0, 1, 2]
+    assert int(ins.sum()) == 3 and int((remap != -1).sum()) == 3
+    assert bool(ins[n - 1]) and bool(ins[5]) and bool(ins[n - 2])
+    del ptr, ins, remap
+    torch.cuda.empty_cache()
