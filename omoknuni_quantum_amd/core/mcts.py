@@ -331,8 +331,8 @@ class MCTS:
         (OMQ_GO_SUICIDE), so that the root's Dirichlet noise has one entry per legal move."""
         T = boards.shape[0]
         ko = self._root_go_host[1]
-        empty = boards == 0
-        taken = ~empty
+        taken = np.ascontiguousarray(boards != 0)  # (a C-ordered copy: `flat` below is its view)
+        empty = ~taken
         if flags & _lib.OMQ_GO_SUICIDE:
             pad = np.zeros((T, boards.shape[1] + 2, boards.shape[2] + 2), bool)
             pad[:, 1:-1, 1:-1] = empty

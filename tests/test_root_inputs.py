@@ -46,3 +46,24 @@ def test_go_root_legal(flags):
                 legal.append(a)
         bits = [a for a in range(32) if masks[t, 0] >> a & 1]
         assert bits == legal + [bs * bs]
+
+
+@pytest.mark.parametrize("layout", ["F", "transposed", "strided"])
+@pytest.mark.parametrize("flags", [_lib.OMQ_GO_KO, _lib.OMQ_GO_KO | _lib.OMQ_GO_SUICIDE])
+def test_go_root_legal_of_any_board_layout(flags, layout):
+    """The masks of boards in other memory orders are those of the same boards in C order, the ko
+    points excluded."""
+    bs, T = 5, 12
+    boards = games.random_boards(T, bs, bs * bs, 3, min_stones=8)
+    ko = np.array([int(np.flatnonzero(b.reshape(-1) == 0)[0]) for b in boards], np.int32)
+    me = SimpleNamespace(model=games.go(bs), _root_go_host=(np.zeros(T, np.int32), ko))
+    want = MCTS._go_root_legal(me, boards, flags)
+    assert not any(want[t, 0] >> int(ko[t]) & 1 for t in range(T))
+    if layout == "F":
+        other = np.asfortranarray(boards)
+    elif layout == "transposed":
+        other = np.ascontiguousarray(boards.transpose(0, 2, 1)).transpose(0, 2, 1)
+    else:
+        other = np.repeat(boards, 2, axis=2)[:, :, ::2]
+    assert np.array_equal(other, boards) and not other.flags.c_contiguous
+    assert np.array_equal(MCTS._go_root_legal(me, other, flags), want)
