@@ -10,6 +10,7 @@ expand -> backup.
 from __future__ import annotations
 
 import ctypes
+import threading
 from dataclasses import dataclass
 
 import numpy as np
@@ -111,7 +112,7 @@ class WaveEngine:
         self._new_roots: torch.Tensor | None = None  # subtree reuse: the new roots [T]
         self._child: torch.Tensor | None = None     # root_children: actions [T], results [T, 2]
         self._pending: dict = {}                    # rule inputs to copy (_copy_pending)
-        self._stage: dict = {}                      # pinned host buffers by name (_host)
+        self._init_staging()
 
         f = _lib.OmqForest()
         f.num_trees, f.capacity, f.num_actions, f.game = T, cap, A, model.code
@@ -135,6 +136,11 @@ class WaveEngine:
         self.wave_ref = ctypes.byref(self.wave)
 
     # ---- plumbing ---------------------------------------------------------------------
+    def _init_staging(self) -> None:
+        self._stage: dict = {}  # pinned host buffers by name (_host)
+        # held from a buffer's first use to its last: the waits let other threads run
+        self._stage_lock = threading.RLock()
+
     def stream_handle(self) -> int:
         return _lib.raw_stream(self.device)
 
@@ -151,21 +157,23 @@ class WaveEngine:
         """name=(device tensor, host array): the arrays through pinned buffers, their copies in
         flight together and one wait for all, so that the inputs are on the device for any
         stream when this returns (a pageable copy waits for each: 20-35 us an array)."""
-        for name, (dst, src) in arrays.items():
-            h = self._host(name, dst)
-            np.copyto(h.numpy(), np.asarray(src).reshape(-1))
-            dst.view(-1).copy_(h, non_blocking=True)
-        torch.cuda.current_stream(self.device).synchronize()
+        with self._stage_lock:
+            for name, (dst, src) in arrays.items():
+                h = self._host(name, dst)
+                np.copyto(h.numpy(), np.asarray(src).reshape(-1))
+                dst.view(-1).copy_(h, non_blocking=True)
+            torch.cuda.current_stream(self.device).synchronize()
 
     def _download(self, **tensors) -> list:
         """name=device tensor: host copies (numpy, the caller's own) after one wait for all."""
         out = []
-        for name, x in tensors.items():
-            h = self._host(name, x)
-            h.copy_(x.view(-1), non_blocking=True)
-            out.append(h)
-        torch.cuda.current_stream(self.device).synchronize()
-        return [h.numpy().copy() for h in out]
+        with self._stage_lock:
+            for name, x in tensors.items():
+                h = self._host(name, x)
+                h.copy_(x.view(-1), non_blocking=True)
+                out.append(h)
+            torch.cuda.current_stream(self.device).synchronize()
+            return [h.numpy().copy() for h in out]
 
     def set_roots(self, keys: np.ndarray, legal: np.ndarray | None = None,
                   noise: np.ndarray | None = None) -> None:
@@ -388,13 +396,15 @@ class WaveEngine:
     def root_children(self, actions) -> np.ndarray:
         """[T, 2]: for every tree the root's child for its action (a node of the tree, -1
         without one) and that child's visit count."""
-        if self._child is None:
-            self._child = torch.empty(3 * self.T, dtype=torch.int32, device=self.device)
-        acts, out = self._child[:self.T], self._child[self.T:]
-        self._upload(child_actions=(acts, np.asarray(actions, np.int32)))
-        self._check(self.lib.omq_root_children(self.forest_ref, acts.data_ptr(), out.data_ptr(),
-                                               self.stream_handle()), "omq_root_children")
-        return self._download(children=out)[0].reshape(self.T, 2)
+        with self._stage_lock:
+            if self._child is None:
+                self._child = torch.empty(3 * self.T, dtype=torch.int32, device=self.device)
+            acts, out = self._child[:self.T], self._child[self.T:]
+            self._upload(child_actions=(acts, np.asarray(actions, np.int32)))
+            self._check(self.lib.omq_root_children(self.forest_ref, acts.data_ptr(),
+                                                   out.data_ptr(), self.stream_handle()),
+                        "omq_root_children")
+            return self._download(children=out)[0].reshape(self.T, 2)
 
     def _tree_of(self, tree_of, n: int):
         if tree_of is None:
