@@ -243,13 +243,13 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> select_expand_meta(
     const at::Tensor& roots, const at::Tensor&, const at::Tensor&, const at::Tensor&,
     const at::Tensor&, const at::Tensor& is_expanded, int64_t max_depth, double) {
   const int64_t W = roots.numel();
-  const auto i32 = roots.options();
+  const auto i32 = roots.options().device(at::kMeta);  // (also where another argument is the meta)
   return {at::empty({W, max_depth}, i32), at::empty({W}, i32), at::empty({W}, i32),
-          at::empty({W}, is_expanded.options())};
+          at::empty({W}, is_expanded.options().device(at::kMeta))};
 }
 at::Tensor batched_ucb_meta(const at::Tensor&, const at::Tensor&, const at::Tensor& parent_visits,
                             const at::Tensor&, const at::Tensor&, const at::Tensor&, double) {
-  return at::empty({parent_visits.numel()}, parent_visits.options());
+  return at::empty({parent_visits.numel()}, parent_visits.options().device(at::kMeta));
 }
 
 constexpr const char* kSelectExpandSchema =

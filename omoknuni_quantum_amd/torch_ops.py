@@ -129,6 +129,12 @@ def fused_ucb_selection(node_indices: torch.Tensor, children_start: torch.Tensor
                                              float(c_puct))
 
 
+def _refuse_meta(name: str) -> None:
+    """For the functions whose operators have Meta kernels (shapes for a tracer): any meta tensor
+    given makes the result one."""
+    raise RuntimeError(f"omq::{name}: tensors must be on a HIP device (got meta)")
+
+
 def _need(name: str, **tensors) -> None:
     """dtype checks: name=(tensor, dtype)."""
     for arg, (t, dt) in tensors.items():
@@ -176,8 +182,11 @@ def batched_ucb_selection(q_values: torch.Tensor, visit_counts: torch.Tensor,
     """The row position of each CSR row's UCB maximum (batched_ucb_selection_cuda,
     mcts_kernels.cu:1412-1464); all -1 for an empty batch, no children, or arrays whose sizes
     disagree, as the reference returns."""
-    return _BATCHED_UCB(q_values, visit_counts, parent_visits, priors, row_ptr, col_indices,
-                        float(c_puct))
+    selected = _BATCHED_UCB(q_values, visit_counts, parent_visits, priors, row_ptr, col_indices,
+                            float(c_puct))
+    if selected.is_meta:
+        _refuse_meta("batched_ucb_selection")
+    return selected
 
 
 def _table(name: str, children: torch.Tensor) -> tuple[int, int]:
@@ -191,8 +200,11 @@ def fused_select_expand(roots: torch.Tensor, children: torch.Tensor, visit_count
                         is_expanded: torch.Tensor, max_depth: int, c_puct: float):
     """(paths [W, max_depth], path_lengths, expand_nodes, needs_expansion) of one descent per
     root (fused_select_expand_cuda, mcts_kernels.cu:2002-2045)."""
-    return _SELECT_EXPAND(roots, children, visit_counts, q_values, prior_probs, is_expanded,
-                          int(max_depth), float(c_puct))
+    out = _SELECT_EXPAND(roots, children, visit_counts, q_values, prior_probs, is_expanded,
+                         int(max_depth), float(c_puct))
+    if out[0].is_meta:
+        _refuse_meta("fused_select_expand")
+    return out
 
 
 def fused_select_expand_optimized(root_nodes: torch.Tensor, children: torch.Tensor,

@@ -234,3 +234,28 @@ def test_mcts_name_taken_first_is_left_to_its_owner():
     r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True,
                        timeout=300)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("device", ["cpu", "meta"])
+def test_accelerator_functions_refuse_tensors_off_the_device(device):
+    """batched_ucb_selection and fused_select_expand take tensors on a HIP device only, also when
+    one of several is not."""
+    import torch
+
+    from omoknuni_quantum_amd import torch_ops
+
+    def t(dt, *shape, dev=device):
+        return torch.zeros(shape, dtype=dt, device=dev)
+
+    i32, f32 = torch.int32, torch.float32
+    for odd in (None, 0, 2):
+        ucb = [(f32, 4), (i32, 4), (i32, 2), (f32, 4), (i32, 3), (i32, 4)]
+        args = [t(dt, n, dev=device if odd in (None, i) else "cpu")
+                for i, (dt, n) in enumerate(ucb)]
+        with pytest.raises(RuntimeError, match="HIP device"):
+            torch_ops.batched_ucb_selection(*args, 1.4)
+        desc = [(i32, 2), (i32, 4, 3), (i32, 4), (f32, 4), (f32, 4), (torch.bool, 4)]
+        args = [t(dt, *n, dev=device if odd in (None, i) else "cpu")
+                for i, (dt, *n) in enumerate(desc)]
+        with pytest.raises(RuntimeError, match="HIP device"):
+            torch_ops.fused_select_expand(*args, 3, 1.4)
