@@ -538,7 +538,8 @@ def _register() -> None:
     already taken in the ``mcts`` namespace (the reference's own module imported first) is left
     to its owner."""
     for name in ("vectorized_backup", "warp_vectorized_backup", "fused_ucb_selection",
-                 "batch_apply_virtual_loss", "batch_remove_virtual_loss"):
+                 "batch_apply_virtual_loss", "batch_remove_virtual_loss",
+                 "fused_select_expand", "batched_ucb_selection"):
         REGISTERED[f"omq::{name}"] = getattr(torch.ops.omq, name)
     for name in MCTS_ALIASES:
         if not torch.ops.omq._mcts_aliased(name):

@@ -259,3 +259,14 @@ def test_accelerator_functions_refuse_tensors_off_the_device(device):
                 for i, (dt, *n) in enumerate(desc)]
         with pytest.raises(RuntimeError, match="HIP device"):
             torch_ops.fused_select_expand(*args, 3, 1.4)
+
+
+def test_registered_operators_are_recorded():
+    """REGISTERED holds every omq:: operator of the C++ library (its own helpers aside)."""
+    import torch
+
+    from omoknuni_quantum_amd import torch_ops
+
+    names = {n.split(".")[0] for n in torch._C._dispatch_get_all_op_names()
+             if n.startswith("omq::") and not n.startswith("omq::_")}
+    assert names == {n for n in torch_ops.REGISTERED if n.startswith("omq::")}
