@@ -47,130 +47,164 @@ __global__ void backup_atomic_kernel(omq_forest f, omq_wave w, int W, int vli) {
   }
 }
 
-// Counts (and value sums) per node gathered in a workgroup's LDS before they go to memory: a
-// hash table of the nodes its paths share.  An atomic on one address of device memory costs
-// about 24 ns after the one before it (each is carried out past the XCD's own L2), and every path
-// adds to its root, so the nodes of the first levels set the time; a workgroup adds to each of
-// them once.  A node that finds no slot within kProbes is added to memory directly.
-template <bool SUMS>
+// Counts (and value sums) per node gathered in a workgroup's LDS before they go to memory.  An
+// atomic on one address of device memory costs about 24 ns after the one before it (each is carried
+// out past the XCD's own L2), and every path adds to its root, so the nodes of the first levels set
+// the time; a workgroup adds to each of them once.
+// The workgroup's entries (kEntries nodes) meet in a table of slots without probing or compare-and-
+// swap: every entry writes its number to its node's slot, and after a barrier the entries whose
+// node is that of the number left there add up in the slot.  The entry left (the slot's owner) adds
+// the result to memory; an entry that finds another node's number adds to memory directly.  A node
+// that no other entry shares so costs a few LDS accesses more than a direct add and keeps its place
+// in the list's order (a table probed by compare-and-swap and written out in its own order took
+// up to 4.7 us more than direct adds on such lists, and 159 against 11.2 us on 4M nodes in order).
+template <bool SUMS, int kEntries>
 struct NodeTable {
-  static constexpr int kSlots = 1024;
-  static constexpr int kProbes = 8;
-  static constexpr unsigned long long kFree = ~0ull;
-  unsigned long long key[kSlots];  // the node's index in the forest's arrays
+  static constexpr int kBits = 11;
+  static constexpr int kSlots = 1 << kBits;
+  static_assert(kEntries <= 65536, "entries are numbered in 16 bits");
+  int64_t node[kEntries];  // an entry's node, as an index into the forest's arrays
+  uint16_t left[kSlots];   // the number of one of the slot's entries
   int count[kSlots];
   float sum[SUMS ? kSlots : 1];
 
-  __device__ void clear(int tid, int threads) {
-    for (int i = tid; i < kSlots; i += threads) {
-      key[i] = kFree;
-      count[i] = 0;
-      if (SUMS) sum[i] = 0.0f;
-    }
+  __device__ static int slot(int64_t nd) {
+    return (int)(((uint32_t)nd * 0x9E3779B1u) >> (32 - kBits));
   }
-  __device__ bool add(int64_t node, int c, float v) {
-    const unsigned long long k = (unsigned long long)node;
-    uint32_t h = ((uint32_t)k * 0x9E3779B1u) >> 22;  // (10 bits: kSlots)
-    for (int i = 0; i < kProbes; ++i, h = (h + 1) & (kSlots - 1)) {
-      unsigned long long at = key[h];
-      if (at == kFree) at = atomicCAS(&key[h], kFree, k);
-      if (at == kFree || at == k) {
-        atomicAdd(&count[h], c);
-        if (SUMS) __hip_atomic_fetch_add(&sum[h], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        return true;
-      }
-    }
-    return false;
+  // before the first barrier
+  __device__ void enter(int e, int64_t nd) {
+    const int h = slot(nd);
+    node[e] = nd;
+    left[h] = (uint16_t)e;
+    count[h] = 0;
+    if (SUMS) sum[h] = 0.0f;
   }
-  __device__ void flush(int tid, int threads, int32_t* counts, float* sums) {
-    for (int i = tid; i < kSlots; i += threads) {
-      const unsigned long long k = key[i];
-      if (k == kFree) continue;
-      atomicAdd(&counts[k], count[i]);
-      if (SUMS) unsafeAtomicAdd(&sums[k], sum[i]);
-    }
+  // between the barriers; false: not taken, to be added to memory directly
+  __device__ bool add(int64_t nd, int c, float v) {
+    const int h = slot(nd);
+    if (node[left[h]] != nd) return false;
+    atomicAdd(&count[h], c);
+    if (SUMS) __hip_atomic_fetch_add(&sum[h], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return true;
+  }
+  // after the second barrier
+  __device__ void flush(int e, int64_t nd, int32_t* counts, float* sums) const {
+    const int h = slot(nd);
+    if (left[h] != e) return;
+    atomicAdd(&counts[nd], count[h]);
+    if (SUMS) unsafeAtomicAdd(&sums[nd], sum[h]);
   }
 };
 
 // reference-style backup over an explicit path matrix (vectorized_backup_kernel), one thread per
 // path.  The nodes of the first kSharedDepth levels go through the workgroup's table, the deeper
-// ones, which few paths share, straight to memory.  32768 paths of 32 trees (depth 6 on average):
-// 58.6 -> 14.1 us; 49152 paths of one tree, with the virtual loss on and off: 1945 -> 142 us.
-// Workgroups of 512 or 1024 threads add to a root less often (the one tree 92 and 66 us) but wait
-// longer at its LDS address: 4096 paths of 8 trees 16.8 us with 256, 22.8 and 35.1 us.  Adding a
-// wave's equal nodes up first changed neither.
+// ones, which few paths share, straight to memory.  A thread enters its deepest node first: where
+// two nodes of a workgroup meet in a slot, the shallower one, which more paths share, mostly keeps
+// it (49152 paths of one tree: 175 us the other way round, 26 us so).
+// Device time a call, against an atomic per path entry: 32768 paths of 32 trees (5.2 nodes on
+// average) 41.2 -> 10.4 us; 49152 paths of one tree (4.6) 939 -> 26.3; 64 paths of one tree 6.0 ->
+// 4.6, of 64 trees 3.5 -> 3.8; 32768 paths of 8 nodes that share none 24.8 -> 26.3.  4096 slots in
+// place of 2048 changed none of these by more than a tenth.
 constexpr int kPathThreads = 256;
 constexpr int kSharedDepth = 8;
 
 __global__ __launch_bounds__(kPathThreads) void paths_backup_kernel(
     omq_forest f, const int32_t* paths, const int32_t* plen, const int32_t* tree_of,
     const float* values, int batch, int max_depth, int sign_mode) {
-  __shared__ NodeTable<true> table;
+  __shared__ NodeTable<true, kPathThreads * kSharedDepth> table;
   const int tid = threadIdx.x;
-  table.clear(tid, kPathThreads);
-  __syncthreads();
   const int b = blockIdx.x * kPathThreads + tid;
   const int t = b < batch && tree_of ? tree_of[b] : 0;
-  if (b < batch && t >= 0 && t < f.num_trees) {  // entries naming no tree are skipped
-    const int64_t tb = (int64_t)t * f.capacity;
-    // entries d < min(length, max_depth); the leaf-positive sign counts the distance from the
-    // leaf by the length as given (vectorized_backup_kernel, mcts_kernels.cu:142-146), also for a
-    // length past the row
-    const int Lp = plen[b];
-    const int L = min(Lp, max_depth);
-    const float v = values[b];
-    const int32_t* row = paths + (int64_t)b * max_depth;
-    constexpr int kB = 4;  // entries whose loads are in flight together
-    for (int d0 = 0; d0 < L; d0 += kB) {
-      int xs[kB];
+  const bool on = b < batch && t >= 0 && t < f.num_trees;  // entries naming no tree are skipped
+  const int64_t tb = (int64_t)t * f.capacity;
+  // entries d < min(length, max_depth); the leaf-positive sign counts the distance from the
+  // leaf by the length as given (vectorized_backup_kernel, mcts_kernels.cu:142-146), also for a
+  // length past the row
+  const int Lp = on ? plen[b] : 0;
+  const int L = min(Lp, max_depth);
+  const float v = on ? values[b] : 0.0f;
+  const int32_t* row = paths + (int64_t)b * max_depth;
+  auto signed_value = [&](int d) {
+    const int e = sign_mode == OMQ_SIGN_LEAF_POSITIVE ? (Lp - 1 - d) : d;
+    return (e & 1) ? -v : v;
+  };
+  auto to_memory = [&](int64_t node, float sv) {
+    atomicAdd(&f.visit_counts[node], 1);
+    unsafeAtomicAdd(&f.value_sums[node], sv);
+  };
+  int xs[kSharedDepth];  // (-1 padding and out-of-range entries are skipped)
 #pragma unroll
-      for (int j = 0; j < kB; ++j) xs[j] = d0 + j < L ? row[d0 + j] : -1;
+  for (int d = 0; d < kSharedDepth; ++d) xs[d] = d < L ? row[d] : -1;
 #pragma unroll
-      for (int j = 0; j < kB; ++j) {
-        const int x = xs[j];
-        if (x < 0 || x >= f.capacity) continue;  // -1 padding and out-of-range entries
-        const int d = d0 + j;
-        const int e = sign_mode == OMQ_SIGN_LEAF_POSITIVE ? (Lp - 1 - d) : d;
-        const float sv = (e & 1) ? -v : v;
-        if (d >= kSharedDepth || !table.add(tb + x, 1, sv)) {
-          atomicAdd(&f.visit_counts[tb + x], 1);
-          unsafeAtomicAdd(&f.value_sums[tb + x], sv);
-        }
-      }
-    }
+  for (int d = kSharedDepth - 1; d >= 0; --d) {
+    if (xs[d] >= f.capacity) xs[d] = -1;
+    if (xs[d] >= 0) table.enter(d * kPathThreads + tid, tb + xs[d]);
   }
   __syncthreads();
-  table.flush(tid, kPathThreads, f.visit_counts, f.value_sums);
+#pragma unroll
+  for (int d = 0; d < kSharedDepth; ++d)
+    if (xs[d] >= 0 && !table.add(tb + xs[d], 1, signed_value(d)))
+      to_memory(tb + xs[d], signed_value(d));
+  constexpr int kB = 4;  // deeper entries whose loads are in flight together
+  for (int d0 = kSharedDepth; d0 < L; d0 += kB) {
+    int ys[kB];
+#pragma unroll
+    for (int j = 0; j < kB; ++j) ys[j] = d0 + j < L ? row[d0 + j] : -1;
+#pragma unroll
+    for (int j = 0; j < kB; ++j)
+      if (ys[j] >= 0 && ys[j] < f.capacity) to_memory(tb + ys[j], signed_value(d0 + j));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < kSharedDepth; ++d)
+    if (xs[d] >= 0)
+      table.flush(d * kPathThreads + tid, tb + xs[d], f.visit_counts, f.value_sums);
 }
 
-// delta per listed node; a workgroup takes kVlPer nodes per thread through its table (the path
-// nodes of the 32768 paths above: 25.0 -> 7.2 us)
-constexpr int kVlPer = 4;
+// delta per listed node; a workgroup takes kVlPer nodes per thread through its table, but for 64
+// consecutive nodes in order, whose add is coalesced already (4M nodes in order: 15.6 us through the
+// table, 11.7 so, 11.2 without a table at all).
+// Device time a call, against an atomic per entry: the path nodes of the 32768 paths above 27.6 ->
+// 6.6 us, of the 49152 588 -> 38; 1000 entries of one node 13.0 -> 2.2, of 1000 nodes 2.2 -> 2.4.
+// One node per thread up to kVlShort entries: at most 64 workgroups, so a node that all of them
+// share costs 1.5 us, and a workgroup of a quarter of the entries is done sooner (1000 to 16000
+// entries 2.2-2.7 us, 3.6-4.2 with four nodes per thread; 225k entries of one tree 59 us with one,
+// 38 with four).
+constexpr int kVlShort = 64 * kPathThreads;
+
+template <int kVlPer>
 __global__ __launch_bounds__(kPathThreads) void virtual_loss_kernel(omq_forest f,
                                                                     const int32_t* nodes,
                                                                     const int32_t* tree_of,
                                                                     int count, int delta) {
-  __shared__ NodeTable<false> table;
+  __shared__ NodeTable<false, kPathThreads * kVlPer> table;
   const int tid = threadIdx.x;
   const int64_t i0 = (int64_t)blockIdx.x * (kPathThreads * kVlPer) + tid;
-  int xs[kVlPer], ts[kVlPer];
+  int64_t nd[kVlPer];  // -1: none
 #pragma unroll
   for (int j = 0; j < kVlPer; ++j) {
     const int64_t i = i0 + j * kPathThreads;
-    xs[j] = i < count ? nodes[i] : -1;
-    ts[j] = i < count && tree_of ? tree_of[i] : 0;
+    const int x = i < count ? nodes[i] : -1;
+    const int t = i < count && tree_of ? tree_of[i] : 0;
+    const bool on = x >= 0 && x < f.capacity && t >= 0 && t < f.num_trees;
+    nd[j] = on ? (int64_t)t * f.capacity + x : -1;
+    const int64_t from = (int64_t)__shfl(nd[j], 0, kWave);
+    if (__all(on && nd[j] == from + lane_id())) {
+      atomicAdd(&f.visit_counts[nd[j]], delta);
+      nd[j] = -1;
+    }
   }
-  table.clear(tid, kPathThreads);
+#pragma unroll
+  for (int j = 0; j < kVlPer; ++j)
+    if (nd[j] >= 0) table.enter(j * kPathThreads + tid, nd[j]);
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kVlPer; ++j) {
-    const int x = xs[j], t = ts[j];
-    if (x < 0 || x >= f.capacity || t < 0 || t >= f.num_trees) continue;
-    const int64_t node = (int64_t)t * f.capacity + x;
-    if (!table.add(node, delta, 0.0f)) atomicAdd(&f.visit_counts[node], delta);
-  }
+  for (int j = 0; j < kVlPer; ++j)
+    if (nd[j] >= 0 && !table.add(nd[j], delta, 0.0f)) atomicAdd(&f.visit_counts[nd[j]], delta);
   __syncthreads();
-  table.flush(tid, kPathThreads, f.visit_counts, nullptr);
+#pragma unroll
+  for (int j = 0; j < kVlPer; ++j)
+    if (nd[j] >= 0) table.flush(j * kPathThreads + tid, nd[j], f.visit_counts, nullptr);
 }
 
 __global__ void reset_kernel(omq_forest f) {
@@ -224,9 +258,13 @@ hipError_t launch_paths_backup(const omq_forest& f, const int32_t* paths, const 
 
 hipError_t launch_virtual_loss(const omq_forest& f, const int32_t* nodes, const int32_t* tree_of,
                                int count, int delta, hipStream_t st) {
-  constexpr int kPer = kPathThreads * kVlPer;
-  hipLaunchKernelGGL(virtual_loss_kernel, dim3(count / kPer + (count % kPer != 0)),
-                     dim3(kPathThreads), 0, st, f, nodes, tree_of, count, delta);
+  auto blocks = [&](int per) { return dim3(count / per + (count % per != 0)); };
+  if (count <= kVlShort)
+    hipLaunchKernelGGL(virtual_loss_kernel<1>, blocks(kPathThreads), dim3(kPathThreads), 0, st, f,
+                       nodes, tree_of, count, delta);
+  else
+    hipLaunchKernelGGL(virtual_loss_kernel<4>, blocks(4 * kPathThreads), dim3(kPathThreads), 0, st,
+                       f, nodes, tree_of, count, delta);
   return hipGetLastError();
 }
 

@@ -198,6 +198,55 @@ def test_backup_and_virtual_loss_node_tables(device, B, D, nn):
     assert not _np(vl).any()
 
 
+@pytest.mark.parametrize("n", [1, 255, 257, 16384, 16385, 40_000])
+@pytest.mark.parametrize("kind", ["one node", "in order", "shuffled", "few", "runs"])
+def test_virtual_loss_lists(device, n, kind):
+    """Lists around the sizes where the work per thread changes: one node throughout, distinct
+    nodes in and out of order, a few nodes often, and runs of consecutive nodes that repeat, with
+    entries outside the array."""
+    rng = np.random.default_rng(n)
+    nn = 50_000
+    idx = {"one node": np.full(n, 77), "in order": 3 + np.arange(n),
+           "shuffled": rng.permutation(nn)[:n], "few": rng.integers(0, 9, n) ** 4,
+           "runs": (np.arange(n) % 640) + np.where(np.arange(n) % 1000 < 700, 0, nn - 300),
+           }[kind].astype(np.int32)
+    want = np.zeros(nn, np.int64)
+    np.add.at(want, idx[idx < nn], 1)
+    vl = torch.zeros(nn, dtype=torch.int32, device=device)
+    torch_ops.batch_apply_virtual_loss(_t(idx, device), vl)
+    assert np.array_equal(_np(vl), want)
+    torch_ops.batch_remove_virtual_loss(_t(idx, device), vl)
+    assert not _np(vl).any()
+
+
+@pytest.mark.parametrize("trees,paths", [(1, 2000), (64, 64), (300, 300)])
+def test_backup_of_tree_paths(device, trees, paths):
+    """Root-to-leaf paths of one and of many trees (one path each): workgroups whose nodes are
+    nearly all shared, and not at all."""
+    rng = np.random.default_rng(trees)
+    D, per, fan = 20, 3000, 3
+    P = np.full((paths, D), -1, np.int32)
+    plen = np.zeros(paths, np.int32)
+    for b in range(paths):
+        node, up = int(rng.integers(0, per)), []
+        while node > 0:
+            up.append(node)
+            node = (node - 1) // fan
+        up = [0] + up[::-1]
+        plen[b] = len(up)
+        P[b, :len(up)] = np.array(up) + (b % trees) * per
+    nn = per * trees
+    vals = (rng.integers(-4, 5, paths) / 4).astype(F)  # exact sums in any order
+    n_exp, w_exp = np.zeros(nn, np.int64), np.zeros(nn, np.float64)
+    for b in range(paths):
+        for d in range(plen[b]):
+            n_exp[P[b, d]] += 1
+            w_exp[P[b, d]] += vals[b] * (1.0 if (plen[b] - 1 - d) % 2 == 0 else -1.0)
+    n, w = torch.zeros(nn, dtype=torch.int32, device=device), torch.zeros(nn, device=device)
+    torch_ops.vectorized_backup(_t(P, device), _t(plen, device), _t(vals, device), n, w)
+    assert np.array_equal(_np(n), n_exp) and np.array_equal(_np(w), w_exp.astype(F))
+
+
 # ---- parallel_bfs_subtree / extract_subtree_edges --------------------------------------------
 def _check_subtree(device, rows, root, n, actions=True):
     ptr, col = _csr(rows)
