@@ -655,8 +655,9 @@ int omq_optimized_backup_scatter(const int32_t* paths, const int32_t* path_lengt
  * a FIFO breadth-first walk: levels in order, each node's children in row order, a child at
  * its first occurrence (the order of the reference's fallback, gpu_bfs.py:70-127); children
  * outside [0, max_nodes) are skipped.  *subtree_count = -1 when a level's rows add up past
- * 2^31 - 1 (overlapping rows).  One workgroup; workspace: OMQ_BFS_WORKSPACE_INTS(max_nodes)
- * int32 owned by the caller. */
+ * 2^31 - 1 (overlapping rows).  One workgroup searches, after a launch that clears the outputs
+ * (of more than 8192 nodes); workspace: OMQ_BFS_WORKSPACE_INTS(max_nodes) int32 owned by the
+ * caller. */
 int omq_parallel_bfs_subtree(const int32_t* row_ptr, const int32_t* col_indices,
                              int32_t num_edges, int32_t root_idx, int32_t max_nodes,
                              uint8_t* in_subtree, int32_t* node_remap, int32_t* subtree_count,

@@ -341,17 +341,35 @@ __device__ inline void bfs_row(const int32_t* row_ptr, int num_edges, int node, 
 }
 
 // ---- breadth-first subtree ------------------------------------------------------------------
-// Marks, ids and claims of every node before the search, by the whole chip (one workgroup took
-// about a fifth of the search for it).
-__global__ void bfs_clear_kernel(int root, int max_nodes, uint8_t* in_subtree, int32_t* remap,
-                                 int32_t* claim, int32_t* queue) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < max_nodes;
-       i += gridDim.x * blockDim.x) {
+// Marks, ids and claims of every node before the search: by the whole chip (one workgroup took
+// about a fifth of the search for it), or, up to kBfsClearHere nodes, by the search's workgroup
+// itself, which saves a launch (a graph of 10 nodes 14.5 -> 5.4 us with the narrow levels below; one
+// of 8000 43 us so, of 9000 48 us with the launch).
+__device__ inline void bfs_clear(int root, int max_nodes, uint8_t* in_subtree, int32_t* remap,
+                                 int32_t* claim, int32_t* queue, int64_t first, int64_t step) {
+  for (int64_t i = first; i < max_nodes; i += step) {
     in_subtree[i] = i == root ? 1 : 0;
     remap[i] = i == root ? 0 : -1;
     claim[i] = 0x7FFFFFFF;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) queue[0] = root;
+  if (first == 0) queue[0] = root;
+}
+__global__ void bfs_clear_kernel(int root, int max_nodes, uint8_t* in_subtree, int32_t* remap,
+                                 int32_t* claim, int32_t* queue) {
+  bfs_clear(root, max_nodes, in_subtree, remap, claim, queue,
+            (int64_t)blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+}
+
+// Exclusive scan of one int per thread over the workgroup in the vector registers (the total
+// within 31 bits); the waves' totals through LDS, scanned by every wave.
+__device__ inline int bfs_block_scan32(int v, int* s_wtot, int* tot) {
+  const int wave = (int)threadIdx.x / kWave, lane = lane_id();
+  const int upto = wave_incl_scan(v);
+  if (lane == kWave - 1) s_wtot[wave] = upto;
+  __syncthreads();
+  const int waves = wave_excl_scan(lane < kBfsWaves ? s_wtot[lane] : 0, tot);
+  __syncthreads();  // s_wtot is reused by the next scan
+  return readlane_i(waves, wave) + upto - v;
 }
 
 // Exclusive scans of an int64 and an int per thread over the workgroup, together.
@@ -365,6 +383,23 @@ __device__ inline int64_t bfs_block_scan2(int64_t v, int n, int64_t* s_wtot, int
   return ex >> 16;
 }
 
+// The same for values whose totals stay below 2^31 each, in 32 bits.
+__device__ inline int bfs_block_scan2_32(int v, int n, int64_t* s_wtot, int64_t* tot, int* n_ex,
+                                         int* n_tot) {
+  const int wave = (int)threadIdx.x / kWave, lane = lane_id();
+  const int upto = wave_incl_scan(v), n_upto = wave_incl_scan(n);
+  if (lane == kWave - 1) s_wtot[wave] = (int64_t)upto << 32 | n_upto;
+  __syncthreads();
+  const int64_t w = lane < kBfsWaves ? s_wtot[lane] : 0;
+  int t32;
+  const int waves = wave_excl_scan((int)(w >> 32), &t32);
+  const int n_waves = wave_excl_scan((int)w, n_tot);
+  __syncthreads();  // s_wtot is reused by the next scan
+  *tot = t32;
+  *n_ex = readlane_i(n_waves, wave) + n_upto - n;
+  return readlane_i(waves, wave) + upto - v;
+}
+
 // The search, by one workgroup; its time is its chains of dependent loads, so every round has
 // many of them in flight.  A level's rows are taken kBfsPer nodes per thread at a time: a scan of
 // their lengths gives each row its place in the level's list of candidate edges, the rows with
@@ -376,16 +411,30 @@ __device__ inline int64_t bfs_block_scan2(int64_t v, int n, int64_t* s_wtot, int
 // its row found by a binary search in memory, twice, and the clearing in this workgroup; 79 us
 // so.  A level of more candidates than the queue has room for (rows that overlap, repeated
 // children) finds its candidates again for the numbering.
+// A level costs the workgroup its barriers and scans whatever its size, so the levels that one wave
+// can take (at most 64 nodes, kNarrowTiles * 64 candidates) are taken by one wave, with the nodes in
+// registers and no barrier, one after the other until a wider level comes.  Device time of the
+// search, one candidate per thread / without the narrow levels / so: a chain of 2000 nodes 6391 /
+// 9010 / 2715 us, a binary tree of 4095 65.0 / 84.9 / 37.9, 40k nodes in levels of about 225 with
+// rows of one or two 1012 / 1543 / 822 (the row of a candidate by halving, and the scans in 32
+// bits); the 100k of 300k nodes above, with the edges, 136 -> 129.  (Four nodes per lane and 512
+// candidates in the narrow levels: the chain 3963 us, the 300k nodes 141.)
 // Workspace: queue [max_nodes], claim [max_nodes].
 constexpr int kBfsPer = 4;
 constexpr int kBfsChunk = kBfsThreads * kBfsPer;
 constexpr int kBfsTiles = 8;
 constexpr int kBfsNumber = 8;
+constexpr int kBfsShort = 8;  // rows shorter than this on average: a candidate's row by halving
+constexpr int kBfsEdges32 = 0x7FFFFFFF / kBfsChunk;  // a chunk's rows add up to 31 bits at most
+constexpr int kNarrowTiles = 4;
+constexpr int kBfsClearHere = 8192;
 
 __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
-    const int32_t* row_ptr, const int32_t* col, int num_edges, int max_nodes,
+    const int32_t* row_ptr, const int32_t* col, int num_edges, int root, int max_nodes,
     uint8_t* in_subtree, int32_t* remap, int32_t* count_out, int32_t* queue, int32_t* claim) {
   __shared__ int64_t s_wtot[kBfsWaves];
+  __shared__ int s_wtot32[kBfsWaves];
+  __shared__ int s_level[2];
   __shared__ int s_cex[kBfsChunk];  // rows with edges: place of the first edge in the chunk
   __shared__ int s_cof[kBfsChunk];  //   and its index in col
   const int tid = threadIdx.x;
@@ -419,7 +468,9 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
     }
     int64_t tot;
     int zx;
-    int64_t ex = bfs_block_scan2(mine, nzm, s_wtot, &tot, &zx, nz);
+    int64_t ex = num_edges <= kBfsEdges32
+                     ? bfs_block_scan2_32((int)mine, nzm, s_wtot, &tot, &zx, nz)
+                     : bfs_block_scan2(mine, nzm, s_wtot, &tot, &zx, nz);
 #pragma unroll
     for (int e = 0; e < kBfsPer; ++e) {
       if (len[e] > 0) {
@@ -442,15 +493,115 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
     int j = S * kWave + (kWave - 1 - __clzll(b2));
     const int q = q0 + lane;
     if (q >= tot) return -1;
-    while (j + 1 < nz && s_cex[j + 1] <= q) ++j;
+    // on to the last row that starts at or before q, at most 63 further (the rows have edges)
+    if (nz * kBfsShort > tot) {
+#pragma unroll
+      for (int h = kWave / 2; h >= 1; h >>= 1)
+        if (j + h < nz && s_cex[j + h] <= q) j += h;
+    } else {
+      while (j + 1 < nz && s_cex[j + 1] <= q) ++j;
+    }
     return col[s_cof[j] + (q - s_cex[j])];
   };
   auto outside = [&](int c) { return c >= 0 && c < max_nodes && !in_subtree[c]; };
   auto claimed_by = [&](int c) {  // (past this CU's L1: claims are made by atomics in L2)
     return __hip_atomic_load(&claim[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
+  // The narrow levels from [start, end) on, by one wave; returns at the first that is not.
+  auto narrow_levels = [&]() {
+    int node = lane < end - start ? queue[start + lane] : -1;
+    while (start < end && end - start <= kWave) {
+      int a = 0, len = 0;
+      if (node >= 0) {
+        int b;
+        bfs_row(row_ptr, num_edges, node, &a, &b);
+        len = b - a;
+      }
+      if (__any(len > kNarrowTiles * kWave)) return;
+      const int upto = wave_incl_scan(len);
+      const int tot = readlane_i(upto, kWave - 1);
+      if (tot > kNarrowTiles * kWave) return;
+      int c[kNarrowTiles];
+      bool win[kNarrowTiles];
+#pragma unroll
+      for (int u = 0; u < kNarrowTiles; ++u) {
+        c[u] = -1;
+        win[u] = false;
+        if (u * kWave >= tot) continue;
+        const int q = u * kWave + lane;
+        int lo = 0;  // the first lane whose rows end past q
+#pragma unroll
+        for (int h = kWave / 2; h >= 1; h >>= 1)
+          if (__shfl(upto, lo + h - 1, kWave) <= q) lo += h;
+        lo = min(lo, kWave - 1);
+        const int at = __shfl(a, lo, kWave) + (q - __shfl(upto - len, lo, kWave));
+        if (q < tot) c[u] = col[at];
+      }
+#pragma unroll
+      for (int u = 0; u < kNarrowTiles; ++u)
+        if (!outside(c[u])) c[u] = -1;
+      if (tot <= kWave) {
+        // a child's first candidate, from the lanes of the same child (a ballot per bit)
+        uint64_t same = __ballot(c[0] >= 0);
+        for (int b = 0; b < 32 - __clz(max_nodes); ++b) {
+          const bool one = (c[0] >> b) & 1;
+          const uint64_t bal = __ballot(one);
+          same &= one ? bal : ~bal;
+        }
+        win[0] = c[0] >= 0 && lowest_lane(same) == lane;
+      } else {
+        bool some = false;
+#pragma unroll
+        for (int u = 0; u < kNarrowTiles; ++u) {
+          if (c[u] >= 0) win[u] = atomicMin(&claim[c[u]], u * kWave + lane) > u * kWave + lane;
+          some = some || win[u];
+        }
+        if (__any(some)) {  // (on every claim's result: all are made before any is read)
+#pragma unroll
+          for (int u = 0; u < kNarrowTiles; ++u)
+            win[u] = win[u] && claimed_by(c[u]) == u * kWave + lane;
+        }
+      }
+      int added = 0;
+#pragma unroll
+      for (int u = 0; u < kNarrowTiles; ++u) {
+        const uint64_t m = __ballot(win[u]);
+        const int r = added + (int)__builtin_amdgcn_mbcnt_hi(
+                                  (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (win[u]) {
+          remap[c[u]] = end + r;
+          in_subtree[c[u]] = 1;
+          queue[end + r] = c[u];
+          s_cex[r] = c[u];
+        }
+        added += __popcll(m);
+      }
+      wave_sync();
+      node = lane < added ? s_cex[lane] : -1;
+      wave_sync();
+      start = end;
+      end += added;
+    }
+  };
+  if (max_nodes <= kBfsClearHere) {
+    bfs_clear(root, max_nodes, in_subtree, remap, claim, queue, tid, kBfsThreads);
+    __syncthreads();
+  }
   bool overflow = false;
   while (start < end) {
+    if (end - start <= kWave) {
+      if (wave == 0) {
+        narrow_levels();
+        if (lane == 0) {
+          s_level[0] = start;
+          s_level[1] = end;
+        }
+      }
+      __syncthreads();
+      start = s_level[0];
+      end = s_level[1];
+      if (start == end) break;
+    }
     const int L = end - start;
     int64_t run = 0;
     bool stash = true;  // the level's candidates so far are in queue[end, end + run)
@@ -495,8 +646,8 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
         for (int e = 0; e < kBfsNumber; ++e) by[e] = c[e] >= 0 ? claimed_by(c[e]) : -1;
 #pragma unroll
         for (int e = 0; e < kBfsNumber; ++e) won += c[e] >= 0 && by[e] == (int)(k + e) ? 1 : 0;
-        int64_t tot;
-        int at = end + added + (int)bfs_block_scan(won, s_wtot, &tot);
+        int tot;
+        int at = end + added + bfs_block_scan32(won, s_wtot32, &tot);
 #pragma unroll
         for (int e = 0; e < kBfsNumber; ++e) {
           if (c[e] >= 0 && by[e] == (int)(k + e)) {
@@ -506,7 +657,7 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
             ++at;
           }
         }
-        added += (int)tot;
+        added += tot;
       }
     } else {
       run = 0;
@@ -516,13 +667,13 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
         for (int64_t k0 = 0; k0 < tot; k0 += kBfsThreads) {
           const int c = k0 + wave * kWave < tot ? child_of((int)k0 + wave * kWave, nz, tot) : -1;
           const bool win = outside(c) && claimed_by(c) == (int)(run + k0 + tid);
-          int64_t wins;
-          const int at = end + added + (int)bfs_block_scan(win ? 1 : 0, s_wtot, &wins);
+          int wins;
+          const int at = end + added + bfs_block_scan32(win ? 1 : 0, s_wtot32, &wins);
           if (win) {
             remap[c] = at;
             queue[at] = c;
           }
-          added += (int)wins;
+          added += wins;
         }
         run += tot;
         __syncthreads();
@@ -659,13 +810,15 @@ hipError_t launch_bfs_subtree(const int32_t* row_ptr, const int32_t* col, int nu
                               int32_t* count, int32_t* ws, hipStream_t st) {
   int32_t* queue = ws;
   int32_t* claim = ws + max_nodes;
-  const int blocks = (int)std::min<int64_t>(1024, ((int64_t)max_nodes + 255) / 256);
-  hipLaunchKernelGGL(bfs_clear_kernel, dim3(blocks), dim3(256), 0, st, root, max_nodes,
-                     in_subtree, remap, claim, queue);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (max_nodes > kBfsClearHere) {
+    const int blocks = (int)std::min<int64_t>(1024, ((int64_t)max_nodes + 255) / 256);
+    hipLaunchKernelGGL(bfs_clear_kernel, dim3(blocks), dim3(256), 0, st, root, max_nodes,
+                       in_subtree, remap, claim, queue);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   hipLaunchKernelGGL(bfs_subtree_kernel, dim3(1), dim3(kBfsThreads), 0, st, row_ptr, col,
-                     num_edges, max_nodes, in_subtree, remap, count, queue, claim);
+                     num_edges, root, max_nodes, in_subtree, remap, count, queue, claim);
   return hipGetLastError();
 }
 

@@ -325,6 +325,43 @@ def test_subtree_wide_levels(device, repeat):
     _check_subtree(device, rows, int(np.argmax([len(r) for r in rows[1:41]])) + 1, n)
 
 
+@pytest.mark.parametrize("seed", range(10))
+def test_subtree_narrow_levels(device, seed):
+    """Levels of 1 to 300 nodes with short rows (among them 64 and 65 nodes, and about 64 and 256
+    candidates), children repeated within and across rows, edges back to earlier levels and out of
+    the graph, in graphs of node counts on both sides of 8192."""
+    rng = np.random.default_rng(500 + seed)
+    sizes = [1] + [int(rng.choice([1, 2, 16, 63, 64, 65, 128, 300])) for _ in range(25)]
+    base = np.concatenate([[0], np.cumsum(sizes)])
+    used = int(base[-1])
+    n = [used, 8192, 8193][seed % 3]
+    ids = rng.permutation(n)[:used]  # (levels are not runs of consecutive nodes)
+    rows = [[] for _ in range(n)]
+    for d in range(len(sizes) - 1):
+        most = int(rng.choice([2, 4, 9, 300 // sizes[d] + 2]))
+        for i in range(sizes[d]):
+            kids = [int(c) for c in ids[rng.integers(base[d + 1], base[d + 2],
+                                                     int(rng.integers(0, most)))]]
+            if rng.random() < 0.3:
+                kids += kids[:2] + [int(ids[rng.integers(0, base[d + 1])]), n + 3, -1]
+            rows[int(ids[base[d] + i])] += kids
+        rows[int(ids[base[d]])].append(int(ids[base[d + 1]]))  # (the next level is reached)
+    _check_subtree(device, rows, int(ids[0]), n)
+    _check_subtree(device, rows, int(ids[base[3]]), n)
+
+
+@pytest.mark.parametrize("width", [523, 525])
+def test_subtree_around_32_bit_scans(device, width):
+    """About 2^31 / 4096 edges, from where a chunk's scan takes 64 bits, in rows that repeat their
+    children."""
+    rng = np.random.default_rng(width)
+    n = 3001
+    rows = [list(range(1, 1001))] + [[int(c) for c in rng.integers(0, n, width)]
+                                     for _ in range(1000)] + [[] for _ in range(2000)]
+    assert (sum(map(len, rows)) > 0x7FFFFFFF // 4096) == (width == 525)
+    _check_subtree(device, rows, 0, n)
+
+
 def test_subtree_of_the_largest_node_count(device):
     """max_nodes = 2^31 - 1 (the most an int32 holds): the subtree of the last node, with children
     at both ends."""
