@@ -12,6 +12,8 @@
 // One wavefront per query: lanes stride the row, each keeping its first maximum; the wave then
 // takes the largest score (order-preserving keys) and, among the lanes that hold it, the lowest
 // row position.
+#include <type_traits>
+
 #include "omq_common.h"
 
 namespace omq {
@@ -206,7 +208,9 @@ expansion_compact_kernel(int32_t* nodes, int wave_size, int32_t* count) {
 // A row to a wave.  A row's time is its three dependent loads (bounds, edge, child's values), so
 // each lane has kUcbAhead positions in flight at a time: with 4, a row of up to 256 children is
 // one trip.  8192 rows of 112-225 children: the call 7.7 -> 6.7 us (the kernel 5.9; two ahead
-// 6.1, six 5.9).
+// 6.1, six 5.9).  Rows of at most 64 children are one trip anyway and take one position per lane:
+// 100000 rows of 2 children, kernel, 23.5 us with four, 18.2 with one; 65536 of 8 16.2 and 12.1; 8192
+// of 64 4.4 and 3.9.
 constexpr int kUcbAhead = 4;
 
 __global__ void batched_ucb_kernel(const float* q_values, const int32_t* visit_counts,
@@ -230,24 +234,25 @@ __global__ void batched_ucb_kernel(const float* q_values, const int32_t* visit_c
   float best = -1e10f;
   int best_pos = 0x7FFFFFFF;
   const int hi = min(end, num_children);
-  for (int64_t i0 = start + lane; i0 < hi; i0 += kUcbAhead * kWave) {
-    int c[kUcbAhead];
-    float pr[kUcbAhead], q[kUcbAhead];
-    int nv[kUcbAhead];
+  auto trip = [&](int64_t i0, auto ahead) {
+    constexpr int kN = decltype(ahead)::value;
+    int c[kN];
+    float pr[kN], q[kN];
+    int nv[kN];
 #pragma unroll
-    for (int j = 0; j < kUcbAhead; ++j) {
+    for (int j = 0; j < kN; ++j) {
       const int64_t i = i0 + j * kWave;
       c[j] = i < hi ? col_indices[i] : -1;
       pr[j] = i < hi ? priors[i] : 0.0f;
       if (c[j] >= num_children) c[j] = -1;
     }
 #pragma unroll
-    for (int j = 0; j < kUcbAhead; ++j) {
+    for (int j = 0; j < kN; ++j) {
       nv[j] = c[j] >= 0 ? visit_counts[c[j]] : 0;
       q[j] = c[j] >= 0 ? q_values[c[j]] : 0.0f;
     }
 #pragma unroll
-    for (int j = 0; j < kUcbAhead; ++j) {
+    for (int j = 0; j < kN; ++j) {
       if (c[j] < 0) continue;
       const float n = (float)nv[j];
       const float exploration = c_puct * pr[j] * sqrt_parent / (1.0f + n);
@@ -257,7 +262,12 @@ __global__ void batched_ucb_kernel(const float* q_values, const int32_t* visit_c
         best_pos = (int)(i0 + j * kWave - start);
       }
     }
-  }
+  };
+  if (hi - start <= kWave)
+    trip(start + lane, std::integral_constant<int, 1>());
+  else
+    for (int64_t i0 = start + lane; i0 < hi; i0 += kUcbAhead * kWave)
+      trip(i0, std::integral_constant<int, kUcbAhead>());
   const uint32_t key = best_pos != 0x7FFFFFFF ? fkey(best + 0.0f) : 0u;
   const int pos = wave_first_max_pos(key, best_pos);
   if (pos < 0) {

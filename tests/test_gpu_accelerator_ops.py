@@ -122,6 +122,12 @@ def test_batched_ucb_wide_rows(device, width):
     assert np.array_equal(got.cpu().numpy(), sel_np)
 
 
+@pytest.mark.parametrize("width", [1, 2, 63, 64, 65])
+def test_batched_ucb_short_rows(device, width):
+    """The same for rows of one position per lane, and the first wider one."""
+    test_batched_ucb_wide_rows(device, width)
+
+
 @pytest.mark.parametrize("mc", [4, 64, 150, 700])
 def test_fused_select_expand(device, mc):
     rng = np.random.default_rng(7 + mc)
