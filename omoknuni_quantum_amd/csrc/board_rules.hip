@@ -363,7 +363,7 @@ hipError_t launch_gomoku_terminal(const omq_forest& f, const omq_wave& w, const 
   return hipGetLastError();
 }
 
-// Feature planes of every wave slot (one 256-thread workgroup per slot u of tree t).  Slot
+// Feature planes of every wave slot (slot u of tree t; NW wavefronts each, below).  Slot
 // u < ucount[t] holds the position of unique leaf u; the other slots are written with zeros.
 // Planes follow CPUGameStates.get_nn_features, representation 'basic'
 // (python/mcts/cpu/cpu_game_states.py:430-494), with the leaf's player to move and move count
@@ -384,9 +384,15 @@ hipError_t launch_gomoku_terminal(const omq_forest& f, const omq_wave& w, const 
 // fill of the same buffers takes 42 us), bfloat16 NHWC 71.0 -> 36.2 us; 8192 slots 53.5 -> 35.2 and
 // 34.6 -> 16.6 us; 2048 slots (four waves) 16.0 -> 10.6 and 12.7 -> 10.4 us, where the launch bounds
 // both.  With one wave per slot each XCD writes one run of slots (the first of these 65.0 -> 63.3
-// us; all slots zero, without the chains, 51).  One wave per slot from 4096 slots (16 per CU): 512
-// slots took 18 us with it, 11 with four.
+// us; all slots zero, without the chains, 51).  One wave per slot from 4096 slots (16 per CU) on, and
+// from 2048 for channels-last planes, whose four waves each set up the words of their stores, and for
+// boards of at most 81 cells, whose slots are too short for four.  Device time, one wave / four:
+// 15x15 NCHW float32 512 slots 6.9 / 5.2 us, 2048 11.1 / 9.5, 4096 15.4 / 15.4, 8192 23.4 / 24.9; NHWC
+// bfloat16 512 slots 5.5 / 5.3, 2048 7.9 / 8.8, 4096 10.8 / 14.7; 7x7 NHWC bfloat16 2048 slots 5.1 /
+// 6.4, 3900 6.5 / 10.0 (NCHW 7.0 / 8.6).
 constexpr int kFeatOneWaveSlots = 4096;
+constexpr int kFeatOneWaveSlotsShort = 2048;
+constexpr int kFeatShortCells = 81;
 
 template <typename OutT>
 struct PlaneStore;
@@ -543,7 +549,8 @@ hipError_t launch_leaf_features_t(const omq_forest& f, const omq_wave& w, const 
                                   int planes, bool nhwc, OutT* out, hipStream_t st) {
   const size_t lds = (size_t)(((bs * bs) + 15) & ~15);
   dim3 grid(w.max_wave, f.num_trees);
-  const bool one_wave = (int64_t)w.max_wave * f.num_trees >= kFeatOneWaveSlots;
+  const int from = nhwc || bs * bs <= kFeatShortCells ? kFeatOneWaveSlotsShort : kFeatOneWaveSlots;
+  const bool one_wave = (int64_t)w.max_wave * f.num_trees >= from;
 #define OMQ_FEAT_LAUNCH(P, NH)                                                               \
   if (one_wave)                                                                              \
     hipLaunchKernelGGL((leaf_features_kernel<OutT, P, NH, 1>), grid, dim3(kWave), lds, st, f, \

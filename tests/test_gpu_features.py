@@ -148,3 +148,25 @@ def test_features_unaligned_buffers(device, bs, trees, wave):
                     eng.leaf_features(out, dev_boards, planes, nhwc=nhwc)
                     assert torch.equal(out.cpu(), want), (planes, dtype, nhwc, off)
                     assert (buf[:off] == 7).all() and (buf[off + want.numel():] == 7).all()
+
+
+@pytest.mark.parametrize("bs,trees,wave", [(7, 32, 64), (7, 23, 89), (9, 32, 64), (9, 1, 2049),
+                                           (10, 32, 64), (15, 23, 89), (15, 32, 64)])
+def test_features_of_middling_waves(device, bs, trees, wave):
+    """2047 to 2049 slots, from where channels-last planes and those of small boards take a wave per
+    slot, in every format, with slots past the leaves."""
+    model = games.gomoku(bs)
+    boards = games.random_boards(trees, bs, bs, 8)
+    eng = WaveEngine(model, trees, 1 + 60 * bs * bs, wave, 100, device, SearchParams(c_puct=1.4))
+    eng.set_roots(games.root_keys(8, trees), games.legal_masks(model, boards, trees))
+    eng.search(32, 16, SyntheticEvaluator())
+    eng.select(16)
+    dev_boards = torch.from_numpy(boards.reshape(-1).copy()).to(device)
+    for planes in (18, 19):
+        exp = torch.from_numpy(_expected(eng, boards, planes)[0])
+        for dtype in (torch.float32, torch.bfloat16):
+            for nhwc in (False, True):
+                want = (exp.permute(0, 2, 3, 1) if nhwc else exp).to(dtype).reshape(-1)
+                out = torch.full((want.numel(),), 7.0, dtype=dtype, device=device)
+                eng.leaf_features(out, dev_boards, planes, nhwc=nhwc)
+                assert torch.equal(out.cpu(), want), (planes, dtype, nhwc)
