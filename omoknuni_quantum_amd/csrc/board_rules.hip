@@ -16,11 +16,12 @@
 // The driver does not expand a terminal leaf (python/mcts/cpu/optimized_wave_search.py:374-376),
 // but it still backs up the evaluator's value for it.
 //
-// Here a leaf's position is never stored.  It is rebuilt in LDS from the root board and the
-// moves on the leaf's path: one wavefront per unique leaf, colours alternating from the
-// root's player to move.  The leaf is then scanned cell-parallel: lane l takes cells
-// l, l+64, ..., and a wave min over the winning cells reproduces the row-major first.  A
-// terminal leaf gets ulegal = 0, which keeps omq_expand from expanding it.
+// Here a leaf's position is never stored.  It is rebuilt from the root board and the moves on
+// the leaf's path, colours alternating from the root's player to move, by one wavefront per unique
+// leaf: as row masks in registers, one row of either player per lane, whose fives are shifts of
+// whole rows, or (small boards, other stones than 1 and 2) as a board in LDS that is scanned
+// cell-parallel, lane l taking cells l, l+64, ...  Either way the row-major first winning cell names
+// the winner.  A terminal leaf gets ulegal = 0, which keeps omq_expand from expanding it.
 #include "omq_common.h"
 
 namespace omq {
@@ -203,8 +204,14 @@ __device__ inline int scan_terminal(const int8_t* b, int cells, int bs, int rule
 // than 1 and 2, or another root player, is scanned cell by cell as the reference scans it.  64
 // trees of 256 leaves, 15x15: 13.0 us with the scan for every board, 10.3 us so; 16 trees of 32
 // leaves 5.8 and 4.2 us.
+// A board of one cell per lane is scanned too, and so is one of two cells per lane in large waves,
+// where the work counts and not its latency.  Device time, row masks / scan: 32 trees of 1024 leaves
+// 5x5 16.5 / 12.3 us, 8x8 16.4 / 13.0, 9x9 17.1 / 15.5, 11x11 16.4 / 16.6, 12x12 17.0 / 18.6; 32 of 256
+// 9x9 6.3 / 5.9; 16 of 64 9x9 4.1 / 4.4.
+constexpr int kRuleManySlots = 8192;
+
 __global__ void gomoku_terminal_kernel(omq_forest f, omq_wave w, const int8_t* root_boards,
-                                       const int32_t* root_player, int rule, int bs,
+                                       const int32_t* root_player, int rule, int bs, bool scan,
                                        int32_t* uterm) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int cells = bs * bs;
@@ -215,11 +222,25 @@ __global__ void gomoku_terminal_kernel(omq_forest f, omq_wave w, const int8_t* r
   const int lane = lane_id();
   const int64_t wb = (int64_t)t * w.max_wave;
   if (u >= w.ucount[t]) return;
+  auto scanned = [&]() {
+    int8_t* b = reinterpret_cast<int8_t*>(smem + (size_t)wave * stride);
+    int rp, stones;
+    rebuild_leaf_board<false>(f, w, root_boards, root_player, t, u, cells, b, &rp, &stones);
+    return scan_terminal(b, cells, bs, rule);
+  };
   const int s0 = w.ufirst[wb + u];
   int a_lo, a_hi;
   const int L = load_path_actions(f, w, t, s0, &a_lo, &a_hi);
   if (L <= 1) {  // the root position itself is not checked (the reference never flags it)
     if (uterm != nullptr && lane == 0) uterm[wb + u] = OMQ_TERM_NONE;
+    return;
+  }
+  if (scan) {
+    const int code = scanned();
+    if (lane == 0) {
+      if (code != OMQ_TERM_NONE) w.ulegal[wb + u] = 0;
+      if (uterm != nullptr) uterm[wb + u] = code;
+    }
     return;
   }
   const RowBits one{reinterpret_cast<uint32_t*>(smem + (size_t)wave * stride)};
@@ -257,11 +278,8 @@ __global__ void gomoku_terminal_kernel(omq_forest f, omq_wave w, const int8_t* r
       code = OMQ_TERM_DRAW;
     }
   } else {
-    int8_t* b = reinterpret_cast<int8_t*>(smem + (size_t)wave * stride);
     wave_sync();
-    int rp2, stones2;
-    rebuild_leaf_board<false>(f, w, root_boards, root_player, t, u, cells, b, &rp2, &stones2);
-    code = scan_terminal(b, cells, bs, rule);
+    code = scanned();
   }
   if (lane == 0) {
     if (code != OMQ_TERM_NONE) w.ulegal[wb + u] = 0;
@@ -358,8 +376,10 @@ hipError_t launch_gomoku_terminal(const omq_forest& f, const omq_wave& w, const 
   constexpr int wpb = 4;
   const size_t lds = (size_t)rule_lds_per_wave(bs * bs) * wpb;
   dim3 grid((w.max_wave + wpb - 1) / wpb, f.num_trees);
+  const bool scan = bs * bs <= kWave ||
+                    (bs * bs <= 2 * kWave && (int64_t)w.max_wave * f.num_trees >= kRuleManySlots);
   hipLaunchKernelGGL(gomoku_terminal_kernel, grid, dim3(wpb * kWave), lds, st, f, w, boards,
-                     root_player, rule, bs, uterm);
+                     root_player, rule, bs, scan, uterm);
   return hipGetLastError();
 }
 

@@ -130,3 +130,39 @@ def test_leaf_codes_of_dense_boards(device, bs, rule):
                     assert want == 0 or ulegal[t, u] == 0
                     codes.add(want)
         assert len(codes) >= 2
+
+
+@pytest.mark.parametrize("rule", [_lib.OMQ_RULE_FREESTYLE, _lib.OMQ_RULE_RENJU])
+@pytest.mark.parametrize("bs,slots", [(9, 8192), (9, 8160), (11, 8192), (12, 8192)])
+def test_leaf_codes_of_large_wave_buffers(device, bs, slots, rule):
+    """Boards of up to two cells per lane in wave buffers around the size from where they are
+    scanned, against the numpy scan."""
+    T, W = 32, 8
+    model = games.gomoku(bs)
+    rng = np.random.default_rng(bs + rule)
+    boards = (1 + (rng.random((T, bs, bs)) < 0.35)).astype(np.int8)
+    for t in range(T):
+        boards[t].reshape(-1)[rng.permutation(bs * bs)[:2 + t % 3 * bs]] = 0
+    eng = WaveEngine(model, T, 5_000, slots // T, 100, device, SearchParams(c_puct=1.4))
+    eng.set_roots(games.root_keys(5, T), games.legal_masks(model, boards, T))
+    eng.set_gomoku_rules(boards, rule)
+    eng.reset()
+    ev = SyntheticEvaluator(1.0)
+    codes = set()
+    for w in (1, W, W):
+        eng.run_wave(w, ev)
+        MW = eng.MW
+        uterm = eng.uterm.view(T, MW).cpu().numpy()
+        ufirst = eng.ufirst.view(T, MW).cpu().numpy()
+        plen = eng.path_len.view(T, MW).cpu().numpy()
+        paths = eng.paths.view(T, MW, eng.MD).cpu().numpy()
+        action = eng.action.view(T, eng.cap).cpu().numpy()
+        for t in range(T):
+            for u in range(int(eng.ucount[t])):
+                s = ufirst[t, u]
+                moves = [int(action[t, n]) for n in paths[t, s, 1:plen[t, s]]]
+                b, _, _ = leaf_position(boards[t], moves, None)
+                want = gomoku_terminal(b, rule == _lib.OMQ_RULE_RENJU) if moves else 0
+                assert uterm[t, u] == want, (t, u, moves)
+                codes.add(want)
+    assert len(codes) >= 2
