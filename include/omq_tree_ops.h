@@ -152,8 +152,9 @@ typedef struct omq_wave {
                                counts a tree's finished blocks in the first word of its row */
   int64_t* stats;           /* [T*OMQ_NSTATS] accumulated operation counters */
   int32_t* status;          /* [4] device-side error flags (bit set, never cleared by the library) */
-  int32_t* sel_scratch;     /* [OMQ_SEL_SCRATCH_INTS(T, max_wave)] omq_select's scratch: per-
-                               simulation leaf records (no contents to keep between calls) */
+  int32_t* sel_scratch;     /* [OMQ_SEL_SCRATCH_INTS(T, max_wave)] omq_select's scratch: the
+                               first simulation of each one's leaf (no contents to keep between
+                               calls) */
   uint32_t* umask;          /* NULL, or [T*max_wave*legal_words]: legal-action masks of the unique
                                leaves, written by omq_go_rules.  When it is not NULL,
                                omq_synthetic_evaluate and omq_expand take a board leaf's legal
@@ -166,7 +167,7 @@ typedef struct omq_wave {
 #define OMQ_SPIN_LIMIT_DEFAULT (1 << 22)
 
 /* int32 entries of omq_wave::sel_scratch for T trees of max_wave simulations */
-#define OMQ_SEL_SCRATCH_INTS(T, MW) (2 * (int64_t)(T) * (MW))
+#define OMQ_SEL_SCRATCH_INTS(T, MW) ((int64_t)(T) * (MW))
 
 /* stats counters (per tree, accumulated over waves) */
 #define OMQ_ST_INTERNAL 0     /* groups that selected a child (distinct internal nodes per wave) */
@@ -643,9 +644,9 @@ int omq_optimized_backup_scatter(const int32_t* paths, const int32_t* path_lengt
                                  void* stream);
 
 /* int32 workspace entries of omq_parallel_bfs_subtree and omq_extract_subtree_edges */
-#define OMQ_BFS_WORKSPACE_INTS(max_nodes) (3 * (int64_t)(max_nodes) + 1)
+#define OMQ_BFS_WORKSPACE_INTS(max_nodes) (2 * (int64_t)(max_nodes))
 #define OMQ_EDGES_WORKSPACE_INTS(num_nodes) \
-  ((int64_t)(num_nodes) + ((int64_t)(num_nodes) + 1023) / 1024 + 1)
+  (((int64_t)(num_nodes) + 15) / 16 + ((int64_t)(num_nodes) + 255) / 256 + 1)
 
 /* Breadth-first subtree of root_idx in a CSR graph (parallel_bfs_subtree_cuda,
  * python/mcts/gpu/mcts_kernels.cu:2246-2287, kernel :2095-2194; bound at :2396-2401; called

@@ -64,7 +64,7 @@ class OmqWave(ctypes.Structure):
 
 def sel_scratch_ints(T: int, MW: int) -> int:
     """OMQ_SEL_SCRATCH_INTS of include/omq_tree_ops.h."""
-    return 2 * T * MW
+    return T * MW
 
 
 OMQ_SPIN_LIMIT_DEFAULT = 1 << 22
@@ -131,12 +131,12 @@ SIGNATURES = {
 
 def bfs_workspace_ints(max_nodes: int) -> int:
     """OMQ_BFS_WORKSPACE_INTS of include/omq_tree_ops.h."""
-    return 3 * max_nodes + 1
+    return 2 * max_nodes
 
 
 def edges_workspace_ints(num_nodes: int) -> int:
     """OMQ_EDGES_WORKSPACE_INTS of include/omq_tree_ops.h."""
-    return num_nodes + (num_nodes + 1023) // 1024 + 1
+    return (num_nodes + 15) // 16 + (num_nodes + 255) // 256 + 1
 
 
 class LibraryNotBuilt(RuntimeError):

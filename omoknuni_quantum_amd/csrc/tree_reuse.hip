@@ -833,7 +833,8 @@ hipError_t launch_extract_edges(const int32_t* row_ptr, const int32_t* col, cons
                                 int32_t* ws, hipStream_t st) {
   const int blocks = edges_blocks(num_nodes);
   int32_t* local = ws;
-  // (together at most num_nodes / 16 + num_nodes / 256 + 2 of OMQ_EDGES_WORKSPACE_INTS)
+  // (OMQ_EDGES_WORKSPACE_INTS: the two together, and one so that it is never empty)
+  static_assert(kEdgeNodes == 16 && kEdgeBlockNodes == 256, "OMQ_EDGES_WORKSPACE_INTS");
   int32_t* block_tot = ws + ((int64_t)num_nodes + kEdgeNodes - 1) / kEdgeNodes;
   if (blocks == 0) {
     hipLaunchKernelGGL(edges_scan_kernel, dim3(1), dim3(kEdgeThreads), 0, st, block_tot, 0,

@@ -2599,7 +2599,6 @@ hipError_t launch_select(const omq_forest& f, const omq_wave& w, int W, float c_
   a.max_wave = w.max_wave;
   a.max_depth_buf = w.max_depth;
   a.num_trees = f.num_trees;
-  const int64_t TM = (int64_t)f.num_trees * w.max_wave;
   a.lfs = w.sel_scratch;
   RecordArgs ra;
   ra.actions = f.actions;

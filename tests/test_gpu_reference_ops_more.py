@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from omoknuni_quantum_amd import torch_ops
+from omoknuni_quantum_amd import _lib, torch_ops
 from omoknuni_quantum_amd.mcts_gpu_accelerator import get_mcts_gpu_accelerator
 from oracle import ref_np
 
@@ -378,3 +378,42 @@ def test_subtree_of_the_largest_node_count(device):
     assert bool(ins[n - 1]) and bool(ins[5]) and bool(ins[n - 2])
     del ptr, ins, remap
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 256, 257, 4097, 9000])
+def test_subtree_workspaces_hold_what_is_used(device, n):
+    """The search and the extraction on workspaces of just the declared sizes, whose neighbours
+    keep their contents, against the reference."""
+    rng = np.random.default_rng(n)
+    rows = [[] for _ in range(n)]
+    for i in range(1, n):
+        rows[int(rng.integers(max(0, i - 40), i))].append(i)
+    ptr, col = _csr(rows)
+    ins_e, remap_e, k_e = ref_np.parallel_bfs_subtree(ptr, col, 0, n)
+    pe, ce, _ = ref_np.extract_subtree_edges(ptr, col, None, ins_e, remap_e)
+    lib = _lib.load()
+    ne = len(col)
+    tp, tc = _t(ptr, device), _t(np.append(col, 0).astype(np.int32), device)
+    ins = torch.empty(n, dtype=torch.uint8, device=device)
+    remap, out = [torch.empty(n, dtype=torch.int32, device=device) for _ in range(2)]
+    child = torch.empty_like(out)
+    acts = torch.empty(n, dtype=torch.int16, device=device)
+    count = torch.empty(1, dtype=torch.int32, device=device)
+    stream = torch.cuda.current_stream(device).cuda_stream
+    pad, mark = 64, -77
+
+    def run(ints, call):
+        ws = torch.full((ints + 2 * pad,), mark, dtype=torch.int32, device=device)
+        assert call(ws.data_ptr() + 4 * pad, ints) == _lib.OMQ_OK
+        assert bool((ws[:pad] == mark).all()) and bool((ws[pad + ints:] == mark).all())
+        return int(count.item())
+
+    assert run(_lib.bfs_workspace_ints(n), lambda ws, k: lib.omq_parallel_bfs_subtree(
+        tp.data_ptr(), tc.data_ptr(), ne, 0, n, ins.data_ptr(), remap.data_ptr(),
+        count.data_ptr(), ws, k, stream)) == k_e
+    assert np.array_equal(_np(remap), remap_e)
+    k = run(_lib.edges_workspace_ints(n), lambda ws, k: lib.omq_extract_subtree_edges(
+        tp.data_ptr(), tc.data_ptr(), None, ne, ins.data_ptr(), remap.data_ptr(), n, n,
+        out.data_ptr(), child.data_ptr(), acts.data_ptr(), count.data_ptr(), ws, k, stream))
+    assert k == len(pe)
+    assert np.array_equal(_np(out[:k]), pe) and np.array_equal(_np(child[:k]), ce)

@@ -270,3 +270,29 @@ def test_registered_operators_are_recorded():
     names = {n.split(".")[0] for n in torch._C._dispatch_get_all_op_names()
              if n.startswith("omq::") and not n.startswith("omq::_")}
     assert names == {n for n in torch_ops.REGISTERED if n.startswith("omq::")}
+
+
+def test_workspace_sizes_mirror_the_header():
+    """The Python sizes of the callers' workspaces equal the header's macros, and a workspace of
+    one word less is refused."""
+    text = open(HEADER).read().replace("\\\n", " ")
+
+    def macro(name, **args):
+        params, body = re.search(rf"#define {name}\(([^)]*)\)(.*)", text).groups()
+        body = body.replace("(int64_t)", "").replace("/", "//")
+        return eval(body, dict(zip([x.strip() for x in params.split(",")], args.values())))
+
+    lib = _lib.load()
+    for n in (0, 1, 15, 16, 17, 255, 256, 257, 300_000, 2**31 - 1):
+        assert _lib.bfs_workspace_ints(n) == macro("OMQ_BFS_WORKSPACE_INTS", n=n)
+        assert _lib.edges_workspace_ints(n) == macro("OMQ_EDGES_WORKSPACE_INTS", n=n)
+        assert _lib.sel_scratch_ints(n, 2048) == macro("OMQ_SEL_SCRATCH_INTS", n=n, w=2048)
+        need = _lib.edges_workspace_ints(n)
+        assert lib.omq_extract_subtree_edges(8, 8, None, 1, 8, 8, n, 1, 8, 8, 8, 8, 8, need - 1,
+                                             None) == _lib.OMQ_E_ARG
+        assert str(need) in lib.omq_last_error().decode()
+        if n > 0:
+            need = _lib.bfs_workspace_ints(n)
+            assert lib.omq_parallel_bfs_subtree(8, 8, 1, 0, n, 8, 8, 8, 8, need - 1,
+                                                None) == _lib.OMQ_E_ARG
+            assert str(need) in lib.omq_last_error().decode()
