@@ -284,9 +284,14 @@ __global__ __launch_bounds__(kWave) void sample_actions_kernel(omq_forest f, con
 // cells, and the pass of a Go root) or its sparse-model count.  One workgroup per tree, one gamma
 // variate per thread (about 4 us each, a serial rejection loop in doubles: one wave per tree took
 // them six in a row on 362 actions, 24 us against 10 so), then the canonical wave sum by every wave
-// and the division.
+// and the division.  With many trees the chip is full, and the waves without a variate only take
+// places: from kNoiseManyTrees on a workgroup has no more of them than it needs (to a power of two).
+// Device time, 512 threads / so / one wave per tree: 1024 trees of 7x7 10.3 / 6.7 / 7.4 us, 4096
+// 27.1 / 14.1 / 14.9; 4096 of 20-45 actions 33.7 / 24.8 / 25.2.  With fewer trees they help to write
+// the row (64 trees of 20-45 of 4672 actions 6.7 us with 512 threads, 9.5 with 64).
 constexpr int kNoiseThreads = OMQ_MAX_ROW;
 constexpr int kNoiseMax = OMQ_MAX_ROW + 1;
+constexpr int kNoiseManyTrees = 512;
 __global__ __launch_bounds__(kNoiseThreads) void root_dirichlet_kernel(omq_forest f, double alpha,
                                                                        uint64_t seed,
                                                                        uint64_t counter,
@@ -306,7 +311,7 @@ __global__ __launch_bounds__(kNoiseThreads) void root_dirichlet_kernel(omq_fores
       c += __popc(f.root_legal[(int64_t)t * f.legal_words + i]);
     L = wave_sum_i(c);
   }
-  for (int i = tid; i < L && i < kNoiseMax; i += kNoiseThreads) {
+  for (int i = tid; i < L && i < kNoiseMax; i += (int)blockDim.x) {
     Stream st = make_stream(seed, counter, t, i);
     s_g[i] = gamma_mt(alpha, st);
   }
@@ -314,7 +319,7 @@ __global__ __launch_bounds__(kNoiseThreads) void root_dirichlet_kernel(omq_fores
   double part = 0.0;
   for (int i = lane; i < L && i < kNoiseMax; i += kWave) part = part + s_g[i];
   const double S = wave_sum_canonical_d(part);
-  for (int i = tid; i < A; i += kNoiseThreads) {
+  for (int i = tid; i < A; i += (int)blockDim.x) {
     if (i < L) row[i] = S > 0.0 ? s_g[i] / S : 1.0 / (double)L;
     else row[i] = 0.0;
   }
@@ -376,8 +381,12 @@ hipError_t launch_sample_actions(const omq_forest& f, const double* pol, double 
 
 hipError_t launch_root_dirichlet(const omq_forest& f, double alpha, uint64_t seed,
                                  uint64_t counter, double* noise, hipStream_t st) {
-  hipLaunchKernelGGL(root_dirichlet_kernel, dim3(f.num_trees), dim3(kNoiseThreads), 0, st, f,
-                     alpha, seed, counter, noise);
+  int threads = kNoiseThreads;
+  const int variates = f.game == OMQ_GAME_SPARSE ? f.max_legal : f.num_actions;
+  if (f.num_trees >= kNoiseManyTrees)
+    while (threads > kWave && threads / 2 >= variates) threads /= 2;
+  hipLaunchKernelGGL(root_dirichlet_kernel, dim3(f.num_trees), dim3(threads), 0, st, f, alpha,
+                     seed, counter, noise);
   return hipGetLastError();
 }
 

@@ -122,6 +122,20 @@ def test_device_dirichlet_of_the_widest_root(device):
         assert np.array_equal(got[t], orc.root_dirichlet(t, 0.3, 9, 1)), t
 
 
+@pytest.mark.parametrize("model", [games.gomoku(5), games.gomoku(9), games.gomoku(15), games.go(19),
+                                   games.chess_sparse()], ids=lambda m: f"{m.kind}{m.num_actions}")
+def test_device_dirichlet_of_many_trees(device, model):
+    """Forests of so many trees that a workgroup has as few threads as the row's entries need."""
+    T = 514
+    wl = get("C2" if model.is_board else "C4").scaled(
+        model=model, num_trees=T, capacity=600, wave_size=1, max_stones=model.cells)
+    eng, orc, _ = make_pair(wl, device=device)
+    eng.device_root_noise(0.3, 9, 1)
+    got = eng.noise.view(T, model.num_actions).cpu().numpy()
+    for t in range(T):
+        assert np.array_equal(got[t], orc.root_dirichlet(t, 0.3, 9, 1)), t
+
+
 @pytest.mark.parametrize("name", ["C1", "C3", "C4"])
 def test_root_children(device, name):
     """The root's child for an action and its visits: rows of 20-45, 225 and up to 362 children,
