@@ -687,55 +687,71 @@ __global__ __launch_bounds__(kBfsThreads) void bfs_subtree_kernel(
   if (tid == 0) count_out[0] = overflow ? -1 : end;
 }
 
-// Edge extraction: kept edges per wave and block scan (pass 1), scan of the block totals (pass 2),
-// writes (pass 3).  A wave takes kEdgeNodes consecutive nodes and their edges as one list, 64
-// edges at a time, kEdgeTiles such tiles in flight: consecutive lanes read consecutive edges and
-// write consecutive outputs.  100k edges of 300k nodes, of which a contiguous third is kept: one
-// node per thread with its row in a loop 20 us to count and 66 us to write, 64 nodes per wave 20
-// and 31 us (few waves hold all the edges), 16 nodes 12.5 and 14.3 us.  Workspace: the waves'
-// first edges [ceil(num_nodes / kEdgeNodes)], then the block totals.
+// Edge extraction: kept edges per group of nodes and scan in the chunk (pass 1), scan of the chunk
+// totals (pass 2), writes (pass 3).  A chunk is 256 nodes, 16 groups of 16.  A workgroup takes
+// kEdgeParts chunks, a grid's width apart, and each of its waves one group of each: 64 rows, whose
+// edges are one list, 64 edges at a time, kEdgeTiles such tiles in flight, so that consecutive lanes
+// read consecutive edges and write consecutive outputs.  The time is dependent loads, so it goes with
+// the number of waves where few nodes are kept (64 rows a wave), and where the nodes that have edges
+// lie together, as in a search tree, with the waves that these are spread over (16 of their rows a
+// wave).  Device time of the three launches, one node per thread with its row in a loop / 16 nodes a
+// wave with 64-bit scans / so:
+//   random tree of 300k nodes, none kept 8.7 / 19.7 / 8.3 us, 30 % 18.6 / 40.1 / 13.8, all 30.4 / 43.0 /
+//   17.8; of 2M 18.5 / 83.7 / 18.1, 47.9 / 198 / 47.4 and 99.4 / 215 / 75.1; of 20k, 30 % 14.5 / 15.5 / 11.3;
+//   64 children to a node, 300k nodes, 30 % 68.6 / 26.1 / 25.4, all 338 / 36.3 / 36.0; ten nodes 7.9 /
+//   9.9 / 9.0 (three short launches), a chain of 20k 9.0 / 15.5 / 11.5.
+// Workspace: the groups' first edges in the chunk, then the chunk totals.
 constexpr int kEdgeThreads = 1024;
+constexpr int kEdgeWaves = kEdgeThreads / kWave;
 constexpr int kEdgeTiles = 4;
-constexpr int kEdgeNodes = 16;
-constexpr int kEdgeBlockNodes = kEdgeThreads / kWave * kEdgeNodes;
+constexpr int kEdgeNodes = 16;  // of a group
+constexpr int kEdgeParts = kWave / kEdgeNodes;
+constexpr int kEdgeChunk = kEdgeWaves * kEdgeNodes;
 
-// Calls emit(keep mask, kept by this lane, edge, child, owner lane) for every tile of the kept
-// edges of the wave's nodes [n0, n0 + kEdgeNodes), in order.  Called by whole waves.
-template <class Emit>
-__device__ inline void walk_edges(const int32_t* row_ptr, const int32_t* col, int num_edges,
-                                  const uint8_t* in_subtree, int num_nodes, int64_t n0,
-                                  Emit emit) {
-  const int lane = lane_id();
-  const int64_t node = n0 + lane;
-  int a = 0, len = 0;
-  if (lane < kEdgeNodes && node < num_nodes && in_subtree[node]) {
-    int b;
-    bfs_row(row_ptr, num_edges, (int)node, &a, &b);
-    len = b - a;
-  }
-  // places of the rows in the wave's list (int64: rows may overlap)
+// The node of a lane (past the nodes where there is none); part p's group is that of lane 16 p.
+__device__ inline int64_t edge_node(int lane) {
+  const int64_t chunk = blockIdx.x + (int64_t)(lane / kEdgeNodes) * gridDim.x;
+  return chunk * kEdgeChunk + (int)threadIdx.x / kWave * kEdgeNodes + lane % kEdgeNodes;
+}
+
+// Inclusive prefix sums of the lanes' row lengths.
+__device__ inline int rows_upto(int len, int) { return wave_incl_scan(len); }
+__device__ inline int64_t rows_upto(int len, int64_t) {
   int64_t upto = len;
 #pragma unroll
   for (int off = 1; off < kWave; off <<= 1) {
     const int64_t y = __shfl_up(upto, off, kWave);
-    if (lane >= off) upto += y;
+    if (lane_id() >= off) upto += y;
   }
-  const int64_t total = __shfl(upto, kWave - 1, kWave);
-  for (int64_t q0 = 0; q0 < total; q0 += kEdgeTiles * kWave) {
+  return upto;
+}
+
+// Calls emit(kept by this lane, edge, child, owner lane) for every tile of the edges of the lanes'
+// rows [a, a + len), in order.  Called by whole waves; Int holds the rows' total and a round more.
+template <class Int, class Emit>
+__device__ inline void walk_rows(const int32_t* col, const uint8_t* in_subtree, int num_nodes,
+                                 int a, int len, Emit emit) {
+  const int lane = lane_id();
+  const Int upto = rows_upto(len, Int());
+  const Int total = __shfl(upto, kWave - 1, kWave);
+  for (Int q0 = 0; q0 < total; q0 += kEdgeTiles * kWave) {
     int edge[kEdgeTiles], own[kEdgeTiles], c[kEdgeTiles];
     bool keep[kEdgeTiles];
+    const int tiles = (int)min((total - q0 + kWave - 1) / kWave, (Int)kEdgeTiles);
 #pragma unroll
     for (int u = 0; u < kEdgeTiles; ++u) {
-      const int64_t q = q0 + u * kWave + lane;
+      edge[u] = -1;
+      own[u] = 0;
+      if (u >= tiles) continue;
+      const Int q = q0 + u * kWave + lane;
       int lo = 0;  // the first lane whose rows end past q
 #pragma unroll
       for (int h = kWave / 2; h >= 1; h >>= 1)
         if (__shfl(upto, lo + h - 1, kWave) <= q) lo += h;
-      lo = min(lo, kWave - 1);
-      const int64_t from = __shfl(upto - len, lo, kWave);
-      const int64_t base = __shfl(a, lo, kWave);
+      const Int from = __shfl(upto - len, lo, kWave);
+      const int base = __shfl(a, lo, kWave);
       own[u] = lo;
-      edge[u] = q < total ? (int)(base + (q - from)) : -1;
+      if (q < total) edge[u] = (int)(base + (q - from));
     }
 #pragma unroll
     for (int u = 0; u < kEdgeTiles; ++u) c[u] = edge[u] >= 0 ? col[edge[u]] : -1;
@@ -744,36 +760,80 @@ __device__ inline void walk_edges(const int32_t* row_ptr, const int32_t* col, in
       keep[u] = c[u] >= 0 && c[u] < num_nodes && in_subtree[c[u]];
 #pragma unroll
     for (int u = 0; u < kEdgeTiles; ++u)
-      emit(__ballot(keep[u]), keep[u], edge[u], c[u], own[u]);
+      if (u < tiles) emit(keep[u], edge[u], c[u], own[u]);
   }
+}
+template <class Emit>
+__device__ inline void walk_edges(const int32_t* col, int num_edges, const uint8_t* in_subtree,
+                                  int num_nodes, int a, int len, Emit emit) {
+  // (rows may overlap: a wave's add up to kWave * num_edges at most)
+  if (num_edges <= (0x7FFFFFFF - kEdgeTiles * kWave) / kWave)
+    walk_rows<int>(col, in_subtree, num_nodes, a, len, emit);
+  else
+    walk_rows<int64_t>(col, in_subtree, num_nodes, a, len, emit);
+}
+
+// The lane's row: its first edge and its length (0 outside the subtree).
+__device__ inline int edge_row(const int32_t* row_ptr, int num_edges, const uint8_t* in_subtree,
+                               int num_nodes, int64_t node, int* a) {
+  *a = 0;
+  if (node >= num_nodes || !in_subtree[node]) return 0;
+  int b;
+  bfs_row(row_ptr, num_edges, (int)node, a, &b);
+  return b - *a;
 }
 
 __global__ __launch_bounds__(kEdgeThreads) void edges_count_kernel(
     const int32_t* row_ptr, const int32_t* col, int num_edges, const uint8_t* in_subtree,
-    int num_nodes, int32_t* local, int32_t* block_tot) {
-  __shared__ int64_t s_wtot[kEdgeThreads / kWave];
+    int num_nodes, int32_t* local, int32_t* chunk_tot) {
+  __shared__ int64_t s_kept[kEdgeWaves][kEdgeParts];
   const int wave = (int)threadIdx.x / kWave;
-  const int64_t n0 = (int64_t)blockIdx.x * kEdgeBlockNodes + wave * kEdgeNodes;
-  int64_t n = 0;
-  walk_edges(row_ptr, col, num_edges, in_subtree, num_nodes, n0,
-             [&](uint64_t kept, bool, int, int, int) { n += __popcll(kept); });
-  int64_t tot;
-  const int64_t ex = bfs_block_scan(lane_id() == 0 ? n : 0, s_wtot, &tot);
-  if (lane_id() == 0 && n0 < num_nodes) local[n0 / kEdgeNodes] = (int32_t)ex;
-  if (threadIdx.x == 0) block_tot[blockIdx.x] = (int32_t)tot;
+  const int lane = lane_id();
+  int64_t n[kEdgeParts] = {};
+  int a;
+  const int len = edge_row(row_ptr, num_edges, in_subtree, num_nodes, edge_node(lane), &a);
+  if (__any(len > 0))
+    walk_edges(col, num_edges, in_subtree, num_nodes, a, len,
+               [&](bool mine, int, int, int owner) {
+#pragma unroll
+                 for (int p = 0; p < kEdgeParts; ++p)
+                   n[p] += __popcll(__ballot(mine && owner / kEdgeNodes == p));
+               });
+  if (lane == 0)
+#pragma unroll
+    for (int p = 0; p < kEdgeParts; ++p) s_kept[wave][p] = n[p];
+  __syncthreads();
+  if (lane >= kEdgeParts) return;
+  int64_t before = 0;
+  for (int i = 0; i < wave; ++i) before += s_kept[i][lane];
+  const int64_t first = edge_node(lane * kEdgeNodes);
+  if (first < num_nodes) local[first / kEdgeNodes] = (int32_t)before;
+  const int64_t chunk = first / kEdgeChunk;
+  if (wave == kEdgeWaves - 1 && chunk * kEdgeChunk < num_nodes)
+    chunk_tot[chunk] = (int32_t)(before + s_kept[wave][lane]);
 }
 
-__global__ __launch_bounds__(kEdgeThreads) void edges_scan_kernel(int32_t* block_tot, int blocks,
+// kScanPer chunks per thread and scan
+constexpr int kScanPer = 4;
+__global__ __launch_bounds__(kEdgeThreads) void edges_scan_kernel(int32_t* chunk_tot, int chunks,
                                                                   int32_t* edge_count) {
-  __shared__ int64_t s_wtot[kEdgeThreads / kWave];
+  __shared__ int64_t s_wtot[kEdgeWaves];
   int64_t run = 0;
-  for (int b0 = 0; b0 < blocks; b0 += kEdgeThreads) {
-    const int b = b0 + (int)threadIdx.x;
-    const int64_t v = b < blocks ? block_tot[b] : 0;
+  for (int b0 = 0; b0 < chunks; b0 += kEdgeThreads * kScanPer) {
+    const int b = b0 + (int)threadIdx.x * kScanPer;
+    int v[kScanPer];
+    int64_t mine = 0;
+#pragma unroll
+    for (int e = 0; e < kScanPer; ++e) v[e] = b + e < chunks ? chunk_tot[b + e] : 0;
+#pragma unroll
+    for (int e = 0; e < kScanPer; ++e) mine += v[e];
     int64_t tot;
-    const int64_t ex = bfs_block_scan(v, s_wtot, &tot);
-    __syncthreads();  // every block total of the chunk is read before any is overwritten
-    if (b < blocks) block_tot[b] = (int32_t)(run + ex);
+    int64_t at = run + bfs_block_scan(mine, s_wtot, &tot);
+#pragma unroll
+    for (int e = 0; e < kScanPer; ++e) {
+      if (b + e < chunks) chunk_tot[b + e] = (int32_t)at;
+      at += v[e];
+    }
     run += tot;
   }
   if (threadIdx.x == 0) edge_count[0] = (int32_t)min(run, (int64_t)0x7FFFFFFF);
@@ -782,26 +842,38 @@ __global__ __launch_bounds__(kEdgeThreads) void edges_scan_kernel(int32_t* block
 __global__ __launch_bounds__(kEdgeThreads) void edges_write_kernel(
     const int32_t* row_ptr, const int32_t* col, const int16_t* actions, int num_edges,
     const uint8_t* in_subtree, const int32_t* remap, int num_nodes, int max_edges,
-    const int32_t* local, const int32_t* block_off, int32_t* out_parent, int32_t* out_child,
+    const int32_t* local, const int32_t* chunk_off, int32_t* out_parent, int32_t* out_child,
     int16_t* out_action) {
   const int lane = lane_id();
-  const int64_t n0 =
-      (int64_t)blockIdx.x * kEdgeBlockNodes + (int)threadIdx.x / kWave * kEdgeNodes;
-  if (n0 >= num_nodes) return;  // (whole waves)
-  const int id = n0 + lane < num_nodes ? remap[n0 + lane] : -1;
-  int64_t pos = (int64_t)block_off[blockIdx.x] + local[n0 / kEdgeNodes];
-  walk_edges(row_ptr, col, num_edges, in_subtree, num_nodes, n0,
-             [&](uint64_t kept, bool mine, int edge, int child, int owner) {
+  const int64_t node = edge_node(lane);
+  int a;
+  const int len = edge_row(row_ptr, num_edges, in_subtree, num_nodes, node, &a);
+  if (!__any(len > 0)) return;
+  const int id = node < num_nodes ? remap[node] : -1;
+  const int64_t first = edge_node(lane % kEdgeParts * kEdgeNodes);
+  const int64_t off = first < num_nodes
+                          ? (int64_t)chunk_off[first / kEdgeChunk] + local[first / kEdgeNodes] : 0;
+  int64_t pos[kEdgeParts];  // the next output of each part's group
+#pragma unroll
+  for (int p = 0; p < kEdgeParts; ++p) pos[p] = __shfl(off, p, kWave);
+  walk_edges(col, num_edges, in_subtree, num_nodes, a, len,
+             [&](bool mine, int edge, int child, int owner) {
                const int parent = __shfl(id, owner, kWave);
-               const int64_t at = pos + (int)__builtin_amdgcn_mbcnt_hi(
-                                            (uint32_t)(kept >> 32),
-                                            __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0u));
+               int64_t at = 0;
+#pragma unroll
+               for (int p = 0; p < kEdgeParts; ++p) {
+                 const bool here = mine && owner / kEdgeNodes == p;
+                 const uint64_t kept = __ballot(here);
+                 const int before = (int)__builtin_amdgcn_mbcnt_hi(
+                     (uint32_t)(kept >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0u));
+                 if (here) at = pos[p] + before;
+                 pos[p] += __popcll(kept);
+               }
                if (mine && at < max_edges) {
                  out_parent[at] = parent;
                  out_child[at] = remap[child];
                  out_action[at] = actions != nullptr ? actions[edge] : (int16_t)0;
                }
-               pos += __popcll(kept);
              });
 }
 
@@ -822,36 +894,31 @@ hipError_t launch_bfs_subtree(const int32_t* row_ptr, const int32_t* col, int nu
   return hipGetLastError();
 }
 
-int edges_blocks(int num_nodes) {
-  return (int)(((int64_t)num_nodes + kEdgeBlockNodes - 1) / kEdgeBlockNodes);
-}
-
 hipError_t launch_extract_edges(const int32_t* row_ptr, const int32_t* col, const int16_t* actions,
                                 int num_edges, const uint8_t* in_subtree, const int32_t* remap,
                                 int num_nodes, int max_edges, int32_t* out_parent,
                                 int32_t* out_child, int16_t* out_action, int32_t* edge_count,
                                 int32_t* ws, hipStream_t st) {
-  const int blocks = edges_blocks(num_nodes);
+  // (OMQ_EDGES_WORKSPACE_INTS: local and chunk_tot, and one so that it is never empty)
+  static_assert(kEdgeNodes == 16 && kEdgeChunk == 256, "OMQ_EDGES_WORKSPACE_INTS");
+  const int chunks = (int)(((int64_t)num_nodes + kEdgeChunk - 1) / kEdgeChunk);
+  const int blocks = (chunks + kEdgeParts - 1) / kEdgeParts;
   int32_t* local = ws;
-  // (OMQ_EDGES_WORKSPACE_INTS: the two together, and one so that it is never empty)
-  static_assert(kEdgeNodes == 16 && kEdgeBlockNodes == 256, "OMQ_EDGES_WORKSPACE_INTS");
-  int32_t* block_tot = ws + ((int64_t)num_nodes + kEdgeNodes - 1) / kEdgeNodes;
-  if (blocks == 0) {
-    hipLaunchKernelGGL(edges_scan_kernel, dim3(1), dim3(kEdgeThreads), 0, st, block_tot, 0,
-                       edge_count);
-    return hipGetLastError();
+  int32_t* chunk_tot = ws + ((int64_t)num_nodes + kEdgeNodes - 1) / kEdgeNodes;
+  hipError_t e = hipSuccess;
+  if (blocks > 0) {
+    hipLaunchKernelGGL(edges_count_kernel, dim3(blocks), dim3(kEdgeThreads), 0, st, row_ptr, col,
+                       num_edges, in_subtree, num_nodes, local, chunk_tot);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(edges_count_kernel, dim3(blocks), dim3(kEdgeThreads), 0, st, row_ptr, col,
-                     num_edges, in_subtree, num_nodes, local, block_tot);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(edges_scan_kernel, dim3(1), dim3(kEdgeThreads), 0, st, block_tot, blocks,
+  hipLaunchKernelGGL(edges_scan_kernel, dim3(1), dim3(kEdgeThreads), 0, st, chunk_tot, chunks,
                      edge_count);
   e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || blocks == 0) return e;
   hipLaunchKernelGGL(edges_write_kernel, dim3(blocks), dim3(kEdgeThreads), 0, st, row_ptr, col,
-                     actions, num_edges, in_subtree, remap, num_nodes, max_edges, local,
-                     block_tot, out_parent, out_child, out_action);
+                     actions, num_edges, in_subtree, remap, num_nodes, max_edges, local, chunk_tot,
+                     out_parent, out_child, out_action);
   return hipGetLastError();
 }
 

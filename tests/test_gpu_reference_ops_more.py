@@ -380,6 +380,37 @@ def test_subtree_of_the_largest_node_count(device):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("n", [1, 17, 255, 256, 257, 1023, 1024, 1025, 1300, 70_000])
+@pytest.mark.parametrize("kind", ["tree", "front", "back", "overlap"])
+def test_edges_of_spread_groups(device, n, kind):
+    """The extraction at the edges of its chunks: rows all over the nodes, only in the first or the
+    last of them (long rows), and rows that overlap, of a random half of the nodes."""
+    rng = np.random.default_rng(n)
+    if kind == "tree":
+        lens = rng.integers(0, 3, n)
+    elif kind == "overlap":
+        lens = rng.integers(0, 10 if n < 2000 else 2, n)
+    else:
+        lens = np.zeros(n, np.int64)
+        few = max(1, min(n, 20))
+        lens[:few] = rng.integers(0, 700, few)
+        lens = lens if kind == "front" else lens[::-1]
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ne = int(ptr[-1])
+    if kind == "overlap":  # (rows that start anywhere and end past the next one's start)
+        ptr = np.sort(rng.integers(0, max(ne, 1), n + 1)).astype(np.int32)
+        ptr[::3] = 0
+        ptr[-1] = min(ne, 500)
+    col = rng.integers(-2, n + 3, ne).astype(np.int32)
+    act = rng.integers(-9, 9, ne).astype(np.int16)
+    ins = rng.random(n) < (0.5 if n < 2000 or kind != "overlap" else 0.002)
+    remap = rng.permutation(n).astype(np.int32)
+    pe, ce, ae = ref_np.extract_subtree_edges(ptr, col, act, ins, remap)
+    p, c, a = torch_ops.extract_subtree_edges(_t(ptr, device), _t(col, device), _t(act, device),
+                                              _t(ins, device), _t(remap, device), max(len(pe), 1))
+    assert np.array_equal(_np(p), pe) and np.array_equal(_np(c), ce) and np.array_equal(_np(a), ae)
+
+
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 256, 257, 4097, 9000])
 def test_subtree_workspaces_hold_what_is_used(device, n):
     """The search and the extraction on workspaces of just the declared sizes, whose neighbours
