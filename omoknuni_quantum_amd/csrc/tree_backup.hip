@@ -79,18 +79,17 @@ struct NodeTable {
     count[h] = 0;
     if (SUMS) sum[h] = 0.0f;
   }
-  // between the barriers; false: not taken, to be added to memory directly
-  __device__ bool add(int64_t nd, int c, float v) {
+  // between the barriers (an entry's owner stays what it is; the callers read all their owners
+  // before any of the owners' nodes, and those before any add, so that the reads overlap)
+  __device__ int owner(int64_t nd) const { return left[slot(nd)]; }
+  __device__ void add(int64_t nd, int c, float v) {
     const int h = slot(nd);
-    if (node[left[h]] != nd) return false;
     atomicAdd(&count[h], c);
     if (SUMS) __hip_atomic_fetch_add(&sum[h], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    return true;
   }
-  // after the second barrier
-  __device__ void flush(int e, int64_t nd, int32_t* counts, float* sums) const {
+  // after the second barrier, by the slot's owner
+  __device__ void flush(int64_t nd, int32_t* counts, float* sums) const {
     const int h = slot(nd);
-    if (left[h] != e) return;
     atomicAdd(&counts[nd], count[h]);
     if (SUMS) unsafeAtomicAdd(&sums[nd], sum[h]);
   }
@@ -98,22 +97,31 @@ struct NodeTable {
 
 // reference-style backup over an explicit path matrix (vectorized_backup_kernel), one thread per
 // path.  The nodes of the first kSharedDepth levels go through the workgroup's table, the deeper
-// ones, which few paths share, straight to memory.  A thread enters its deepest node first: where
-// two nodes of a workgroup meet in a slot, the shallower one, which more paths share, mostly keeps
-// it (49152 paths of one tree: 175 us the other way round, 26 us so).
-// Device time a call, against an atomic per path entry: 32768 paths of 32 trees (5.2 nodes on
-// average) 41.2 -> 10.4 us; 49152 paths of one tree (4.6) 939 -> 26.3; 64 paths of one tree 6.0 ->
-// 4.6, of 64 trees 3.5 -> 3.8; 32768 paths of 8 nodes that share none 24.8 -> 26.3.  4096 slots in
-// place of 2048 changed none of these by more than a tenth.
+// ones, which few paths share, straight to memory, in one add where all of a wave's paths are on the
+// same node (a line that every path follows: 64 paths of 64 such nodes 134 -> 22 us, 8192 of them
+// 4173 -> 74).  A thread enters its deepest node first: where two nodes of a workgroup meet in a slot,
+// the shallower one, which more paths share, mostly keeps it (49152 paths of one tree: 175 us the
+// other way round, 26 us so).
+// Up to kFewPaths paths, one wave, there is no table (8 nodes each: 3.5 us, 4.1 with it and one wave);
+// up to kSomePaths a workgroup is one wave, whose table's LDS accesses, which take most of a small
+// call, are a quarter of four waves'.  Device time a call, an atomic per entry / workgroups of 64 /
+// of 256, 8 nodes a path, in a tree whose nodes have two children and with no node shared: 512
+// paths 19.8 / 4.6 / 7.5 us and 5.3 / 4.4 / 7.4; 4096 132 / 7.6 / 10 and 5.5 / 5.2 / 8; 8192 260 / 11.7 /
+// 9.9 and 5.9 / 6.6 / 8.7; 16384 514 / 19.6 / 12.7 and 7.6 / 9.2 / 11.2; 32768 1040 / 36.6 / 18.5 and
+// 13.0 / 15.6 / 16.5.  With six children 8192 paths of 16 nodes 162 / 14.6 / 19.0.
 constexpr int kPathThreads = 256;
 constexpr int kSharedDepth = 8;
+constexpr int kFewPaths = kWave;
+constexpr int kSomePaths = 8192;
 
-__global__ __launch_bounds__(kPathThreads) void paths_backup_kernel(
+template <bool SHARED, int NT>
+__global__ __launch_bounds__(NT) void paths_backup_kernel(
     omq_forest f, const int32_t* paths, const int32_t* plen, const int32_t* tree_of,
     const float* values, int batch, int max_depth, int sign_mode) {
-  __shared__ NodeTable<true, kPathThreads * kSharedDepth> table;
+  constexpr int kTabled = SHARED ? kSharedDepth : 0;
+  __shared__ NodeTable<true, SHARED ? NT * kSharedDepth : 1> table;
   const int tid = threadIdx.x;
-  const int b = blockIdx.x * kPathThreads + tid;
+  const int b = blockIdx.x * NT + tid;
   const int t = b < batch && tree_of ? tree_of[b] : 0;
   const bool on = b < batch && t >= 0 && t < f.num_trees;  // entries naming no tree are skipped
   const int64_t tb = (int64_t)t * f.capacity;
@@ -133,32 +141,61 @@ __global__ __launch_bounds__(kPathThreads) void paths_backup_kernel(
     unsafeAtomicAdd(&f.value_sums[node], sv);
   };
   int xs[kSharedDepth];  // (-1 padding and out-of-range entries are skipped)
+  int own[kSharedDepth];  // their slots' owners
+  if constexpr (SHARED) {
 #pragma unroll
-  for (int d = 0; d < kSharedDepth; ++d) xs[d] = d < L ? row[d] : -1;
+    for (int d = 0; d < kSharedDepth; ++d) xs[d] = d < L ? row[d] : -1;
 #pragma unroll
-  for (int d = kSharedDepth - 1; d >= 0; --d) {
-    if (xs[d] >= f.capacity) xs[d] = -1;
-    if (xs[d] >= 0) table.enter(d * kPathThreads + tid, tb + xs[d]);
+    for (int d = kSharedDepth - 1; d >= 0; --d) {
+      if (xs[d] >= f.capacity) xs[d] = -1;
+      if (xs[d] >= 0) table.enter(d * NT + tid, tb + xs[d]);
+    }
+    __syncthreads();
+    bool taken[kSharedDepth];
+#pragma unroll
+    for (int d = 0; d < kSharedDepth; ++d) own[d] = xs[d] >= 0 ? table.owner(tb + xs[d]) : 0;
+#pragma unroll
+    for (int d = 0; d < kSharedDepth; ++d) taken[d] = table.node[own[d]] == tb + xs[d];
+#pragma unroll
+    for (int d = 0; d < kSharedDepth; ++d) {
+      if (xs[d] < 0) continue;
+      if (taken[d])
+        table.add(tb + xs[d], 1, signed_value(d));
+      else
+        to_memory(tb + xs[d], signed_value(d));
+    }
   }
-  __syncthreads();
-#pragma unroll
-  for (int d = 0; d < kSharedDepth; ++d)
-    if (xs[d] >= 0 && !table.add(tb + xs[d], 1, signed_value(d)))
-      to_memory(tb + xs[d], signed_value(d));
   constexpr int kB = 4;  // deeper entries whose loads are in flight together
-  for (int d0 = kSharedDepth; d0 < L; d0 += kB) {
+  for (int d0 = kTabled; __any(d0 < L); d0 += kB) {
     int ys[kB];
 #pragma unroll
     for (int j = 0; j < kB; ++j) ys[j] = d0 + j < L ? row[d0 + j] : -1;
 #pragma unroll
-    for (int j = 0; j < kB; ++j)
-      if (ys[j] >= 0 && ys[j] < f.capacity) to_memory(tb + ys[j], signed_value(d0 + j));
+    for (int j = 0; j < kB; ++j) {
+      const bool in = ys[j] >= 0 && ys[j] < f.capacity;
+      const uint64_t lanes = __ballot(in);
+      if (lanes == 0) continue;
+      const int64_t node = tb + ys[j];
+      const int64_t one = __shfl(node, lowest_lane(lanes), kWave);
+      const float sv = in ? signed_value(d0 + j) : 0.0f;
+      if (__all(!in || node == one) && __popcll(lanes) > 1) {
+        const float sum = wave_sum_canonical(sv);
+        if (lane_id() == 0) {
+          atomicAdd(&f.visit_counts[one], __popcll(lanes));
+          unsafeAtomicAdd(&f.value_sums[one], sum);
+        }
+      } else if (in) {
+        to_memory(node, sv);
+      }
+    }
   }
-  __syncthreads();
+  if constexpr (SHARED) {
+    __syncthreads();
 #pragma unroll
-  for (int d = 0; d < kSharedDepth; ++d)
-    if (xs[d] >= 0)
-      table.flush(d * kPathThreads + tid, tb + xs[d], f.visit_counts, f.value_sums);
+    for (int d = 0; d < kSharedDepth; ++d)
+      if (xs[d] >= 0 && own[d] == d * NT + tid)
+        table.flush(tb + xs[d], f.visit_counts, f.value_sums);
+  }
 }
 
 // delta per listed node; a workgroup takes kVlPer nodes per thread through its table, but for 64
@@ -198,13 +235,25 @@ __global__ __launch_bounds__(kPathThreads) void virtual_loss_kernel(omq_forest f
   for (int j = 0; j < kVlPer; ++j)
     if (nd[j] >= 0) table.enter(j * kPathThreads + tid, nd[j]);
   __syncthreads();
+  int own[kVlPer];
+  bool taken[kVlPer];
 #pragma unroll
-  for (int j = 0; j < kVlPer; ++j)
-    if (nd[j] >= 0 && !table.add(nd[j], delta, 0.0f)) atomicAdd(&f.visit_counts[nd[j]], delta);
+  for (int j = 0; j < kVlPer; ++j) own[j] = nd[j] >= 0 ? table.owner(nd[j]) : 0;
+#pragma unroll
+  for (int j = 0; j < kVlPer; ++j) taken[j] = table.node[own[j]] == nd[j];
+#pragma unroll
+  for (int j = 0; j < kVlPer; ++j) {
+    if (nd[j] < 0) continue;
+    if (taken[j])
+      table.add(nd[j], delta, 0.0f);
+    else
+      atomicAdd(&f.visit_counts[nd[j]], delta);
+  }
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < kVlPer; ++j)
-    if (nd[j] >= 0) table.flush(j * kPathThreads + tid, nd[j], f.visit_counts, nullptr);
+    if (nd[j] >= 0 && own[j] == j * kPathThreads + tid)
+      table.flush(nd[j], f.visit_counts, nullptr);
 }
 
 __global__ void reset_kernel(omq_forest f) {
@@ -250,9 +299,12 @@ hipError_t launch_backup(const omq_forest& f, const omq_wave& w, int W, float vi
 hipError_t launch_paths_backup(const omq_forest& f, const int32_t* paths, const int32_t* plen,
                                const int32_t* tree_of, const float* values, int batch,
                                int max_depth, int sign_mode, hipStream_t st) {
-  hipLaunchKernelGGL(paths_backup_kernel, dim3((batch + kPathThreads - 1) / kPathThreads),
-                     dim3(kPathThreads), 0, st, f, paths, plen, tree_of, values, batch, max_depth,
-                     sign_mode);
+  const int threads = batch <= kSomePaths ? kWave : kPathThreads;
+  const auto kernel = batch <= kFewPaths    ? paths_backup_kernel<false, kWave>
+                      : batch <= kSomePaths ? paths_backup_kernel<true, kWave>
+                                            : paths_backup_kernel<true, kPathThreads>;
+  hipLaunchKernelGGL(kernel, dim3(batch / threads + (batch % threads != 0)), dim3(threads), 0, st,
+                     f, paths, plen, tree_of, values, batch, max_depth, sign_mode);
   return hipGetLastError();
 }
 

@@ -247,6 +247,29 @@ def test_backup_of_tree_paths(device, trees, paths):
     assert np.array_equal(_np(n), n_exp) and np.array_equal(_np(w), w_exp.astype(F))
 
 
+@pytest.mark.parametrize("paths", [1, 63, 64, 65, 129, 8192, 8193])
+@pytest.mark.parametrize("shared", [3, 13, 30])
+def test_backup_of_batches_around_the_workgroup_sizes(device, paths, shared):
+    """Paths that follow one line for their first levels (past the levels that meet in LDS, and to
+    the end), of several lengths, with padding and entries outside the array on the way."""
+    rng = np.random.default_rng(paths + shared)
+    D, nn = 30, 30 * paths + 40
+    P = np.where(np.arange(D) < shared, np.arange(D), 40 + np.arange(paths * D).reshape(paths, D))
+    plen = np.where(rng.random(paths) < 0.7, D, rng.integers(0, D + 5, paths)).astype(np.int32)
+    odd = rng.random((paths, D)) < 0.02
+    P = np.where(odd, rng.choice([-1, nn, nn + 7], (paths, D)), P).astype(np.int32)
+    vals = (rng.integers(-4, 5, paths) / 4).astype(F)  # exact sums in any order
+    d = np.arange(D)
+    on = (d < plen[:, None]) & (P >= 0) & (P < nn)
+    sign = np.where((plen[:, None] - 1 - d) % 2 == 0, 1.0, -1.0)
+    n_exp, w_exp = np.zeros(nn, np.int64), np.zeros(nn, np.float64)
+    np.add.at(n_exp, P[on], 1)
+    np.add.at(w_exp, P[on], (vals[:, None] * sign)[on])
+    n, w = torch.zeros(nn, dtype=torch.int32, device=device), torch.zeros(nn, device=device)
+    torch_ops.vectorized_backup(_t(P, device), _t(plen, device), _t(vals, device), n, w)
+    assert np.array_equal(_np(n), n_exp) and np.array_equal(_np(w), w_exp.astype(F))
+
+
 # ---- parallel_bfs_subtree / extract_subtree_edges --------------------------------------------
 def _check_subtree(device, rows, root, n, actions=True):
     ptr, col = _csr(rows)
