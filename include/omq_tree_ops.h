@@ -41,7 +41,7 @@
 extern "C" {
 #endif
 
-#define OMQ_ABI_VERSION 4
+#define OMQ_ABI_VERSION 5
 
 /* error codes */
 #define OMQ_OK 0

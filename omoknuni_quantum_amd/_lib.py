@@ -13,7 +13,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_NAME = "libomq_tree_ops.so"
 LIB_PATH = os.path.join(_HERE, LIB_NAME)
 
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 # constants of include/omq_tree_ops.h
 OMQ_OK, OMQ_E_ARG, OMQ_E_LAUNCH, OMQ_E_LIMIT = 0, -1, -2, -3
@@ -182,12 +182,12 @@ def load(path: str | None = None) -> ctypes.CDLL:
                 f"{p} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`"
                 " (hipcc --offload-arch=gfx950); there is no fallback implementation")
         lib = ctypes.CDLL(p)
+        if lib.omq_abi_version() != ABI_VERSION:  # (first: another version lacks some names)
+            raise LibraryNotBuilt(f"{p} has ABI {lib.omq_abi_version()}, expected {ABI_VERSION}")
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        if lib.omq_abi_version() != ABI_VERSION:
-            raise LibraryNotBuilt(f"{p} has ABI {lib.omq_abi_version()}, expected {ABI_VERSION}")
         if path is None:
             _lib = lib
         return lib

@@ -135,6 +135,16 @@ def test_missing_library_fails_loudly(tmp_path):
         _lib.load(str(tmp_path / "absent.so"))
 
 
+def test_library_of_another_version_fails_loudly(tmp_path):
+    import subprocess
+
+    src, lib = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int omq_abi_version(void) { return 4; }\n")  # (and none of the other names)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True, timeout=60)
+    with pytest.raises(_lib.LibraryNotBuilt, match="ABI 4"):
+        _lib.load(str(lib))
+
+
 def test_torch_ops_registered_and_refuse_host_tensors():
     import torch
 
@@ -296,3 +306,18 @@ def test_workspace_sizes_mirror_the_header():
             assert lib.omq_parallel_bfs_subtree(8, 8, 1, 0, n, 8, 8, 8, 8, need - 1,
                                                 None) == _lib.OMQ_E_ARG
             assert str(need) in lib.omq_last_error().decode()
+
+
+def test_abi_version_names_one_interface():
+    """A change of the exported functions, of their arguments' number or of a caller's workspace
+    takes a new OMQ_ABI_VERSION, by which the loader refuses a library of another interface."""
+    import hashlib
+
+    text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S).replace("\\\n", " ")
+    version = int(re.search(r"#define OMQ_ABI_VERSION (\d+)", text).group(1))
+    calls = [f"{name}:{args.count(',') + 1}"
+             for name, args in re.findall(r"\b(omq_[a-z_]+)\s*\(([^)]*)\)\s*;", text)]
+    sizes = [" ".join(x.split()) for x in re.findall(r"#define OMQ_\w+_INTS.*", text)]
+    digest = hashlib.sha256("\n".join(sorted(calls) + sorted(sizes)).encode()).hexdigest()[:16]
+    assert _lib.ABI_VERSION == version
+    assert (version, digest) == (5, "bc994b71377cda2d")
